@@ -30,6 +30,24 @@ constexpr int kBwdThreads = 256;
 // 128; 3 at head_dim 64, whose registers then allow three workgroups per CU).
 constexpr int kDqPipe = 4;
 
+// Split dK/dV (bwd_dkdv_kernel, SPLIT): the workspace starts with two int32
+// counters per (batch, key block, KV head) item, then (256-byte aligned) the
+// fp32 partial sums.
+__host__ __device__ __forceinline__ int64_t dkdv_items(const fa_bwd_args &a) {
+    return int64_t((a.seqlen_k + 127) / 128) * a.batch * a.nheads_k;
+}
+__host__ __device__ __forceinline__ int64_t dkdv_count_bytes(int64_t items) { return (items * 8 + 255) & ~int64_t(255); }
+
+// Zeroes those counters: run by every workgroup of the kernel that fills dsum
+// (the dQ or the preprocess kernel), which precedes dK/dV on the stream.
+__device__ __forceinline__ void zero_dkdv_counts(const fa_bwd_args &a, int block, int n_blocks) {
+    if (!a.split_ws) return;
+    int32_t *count = reinterpret_cast<int32_t *>(a.split_ws);
+    const int64_t n = 2 * dkdv_items(a);
+    for (int64_t i = int64_t(block) * kBwdThreads + threadIdx.x; i < n; i += int64_t(n_blocks) * kBwdThreads)
+        count[i] = 0;
+}
+
 // ---------------------------------------------------------------------------
 // Preprocess: dsum[b][h][i] = -sum_d fp32(O) * fp32(dO) (stored negated, the
 // initial value of the dK/dV kernel's dP accumulators); padding rows get 0.
@@ -41,6 +59,7 @@ __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const fa_bwd_args a
     constexpr int KCH = HD / 8;
     constexpr int ROWS = kBwdThreads / KCH;  // rows per workgroup
     const int b = blockIdx.z, h = blockIdx.y;
+    zero_dkdv_counts(a, (b * gridDim.y + h) * gridDim.x + blockIdx.x, gridDim.x * gridDim.y * gridDim.z);
     const bool packed = a.cu_seqlens_q != nullptr;
     const SeqInfo si = seq_info(b, a.seqlen_q, a.seqlen_k, a.cu_seqlens_q, a.cu_seqlens_k, nullptr, 0);
     const int i = blockIdx.x * ROWS + threadIdx.x / KCH;
@@ -92,6 +111,7 @@ __global__ __launch_bounds__(256, HD == 64 ? 3 : 2) void bwd_dq_kernel(const fa_
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
     const int col = lane & 31, hh = lane >> 5;
+    zero_dkdv_counts(a, blockIdx.x, gridDim.x);
     const int packs = a.nheads >> lg;  // head packs per batch
     int b, h, mb;
     if (a.work_order && a.cu_seqlens_q) {
@@ -303,7 +323,8 @@ __global__ __launch_bounds__(256, HD == 64 ? 3 : 2) void bwd_dq_kernel(const fa_
 // dK^T += Q^T dS read them transposed.  The group's contributions accumulate
 // in fp32 registers (no per-q-head dK/dV buffers) and each wave stores its
 // keys' rows.  Needs D and LSE*log2(e) (the dsum workspace) from the dQ or
-// the preprocess kernel.
+// the preprocess kernel.  SPLIT: S workgroups share each (batch, key block, KV
+// head), each over a share of its steps, and sum their dK / dV (dkdv_reduce).
 constexpr int kDkvThreads = 256;
 
 template <int HD>
@@ -350,20 +371,88 @@ __global__ __launch_bounds__(kOrderThreads) void dq_order_kernel(const fa_bwd_ar
     }, a.work_order + int64_t(a.batch) * nnb, false);
 }
 
-template <int HD, bool CAUSAL>
-__global__ __launch_bounds__(kDkvThreads, 2) void bwd_dkdv_kernel(const fa_bwd_args a, const int nnb) {
+// Sums the S partial dK / dV tiles of an item.  The first S - 1 of its
+// workgroups to get here (count[0]) store theirs and count them stored
+// (count[1]); the last one waits for those stores, which are under way, and
+// adds the partials in the order of their shares, so the sum does not depend
+// on who came last.  Returns whether this workgroup holds the sum.  Partials
+// are stored and loaded at agent scope (past the XCD's L2, as in the split KV
+// kernel), 8 bytes a lane, 512 contiguous bytes a wave.
+template <int HD>
+__device__ __forceinline__ bool dkdv_reduce(const fa_bwd_args &a, int item, int part, int S, int *ticket,
+                                            f32x16 (&dk)[HD / 32], f32x16 (&dv)[HD / 32]) {
+    constexpr int N = HD / 2;  // pairs of floats a lane holds: dK, then dV
+    const int tid = threadIdx.x;
+    int32_t *count = reinterpret_cast<int32_t *>(a.split_ws) + 2 * int64_t(item);
+    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const bool last = *ticket == S - 1;
+    uint64_t *slots = reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(a.split_ws) + dkdv_count_bytes(dkdv_items(a))) +
+                      int64_t(item) * S * N * kDkvThreads + tid;
+    // The last workgroup adds to its own registers when its share is one of
+    // the first two (x0 + x1 = x1 + x0); otherwise it stores too and adds all
+    // shares from memory.
+    if (!last || part >= 2) {
+        uint64_t *slot = slots + int64_t(part) * N * kDkvThreads;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            f32x16 &t = i < N / 2 ? dk[i / 8] : dv[i / 8 - N / 16];
+            const f32x2 x = {t[2 * (i & 7)], t[2 * (i & 7) + 1]};
+            __hip_atomic_store(slot + i * kDkvThreads, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+        wait_vmem();
+        if (!last) {
+            __syncthreads();  // every wave's stores have completed
+            if (tid == 0) __hip_atomic_fetch_add(count + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
+        }
+#pragma unroll
+        for (int i = 0; i < HD / 32; ++i) dk[i] = dv[i] = zero16();
+    }
+    if (tid == 0) {
+        while (__hip_atomic_load(count + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < S - 1)
+            __builtin_amdgcn_s_sleep(1);
+        // Ready for another dK/dV call on the same workspace.
+        __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(count + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    for (int p = 0; p < S; ++p) {
+        if (p == part && part < 2) continue;
+        const uint64_t *slot = slots + int64_t(p) * N * kDkvThreads;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const f32x2 x = __builtin_bit_cast(
+                f32x2, __hip_atomic_load(slot + i * kDkvThreads, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            f32x16 &t = i < N / 2 ? dk[i / 8] : dv[i / 8 - N / 16];
+            t[2 * (i & 7)] += x[0];
+            t[2 * (i & 7) + 1] += x[1];
+        }
+    }
+    return true;
+}
+
+template <int HD, bool CAUSAL, bool SPLIT>
+__global__ __launch_bounds__(kDkvThreads, 2) void bwd_dkdv_kernel(const fa_bwd_args a, const int nnb, const int S) {
     using C = DkvCfg<HD>;
     constexpr int BN = C::BN, BM = C::BM, NT = C::NT, LROWS = C::LROWS;
     __shared__ __attribute__((aligned(16))) char smem[C::LDS];
+    __shared__ int ticket;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int kg = __builtin_amdgcn_readfirstlane(tid >> 6);  // the wave's key group (wave-uniform)
     const int wave = kg;
     const int col = lane & 31, hh = lane >> 5;
-    int b, hk, nb;
+    int b, hk, nb, part = 0;
     if (a.work_order && a.cu_seqlens_k) {
         // Item of the device-built order (kv head fastest); -1: no keys.
-        const int it = a.work_order[blockIdx.x / a.nheads_k];
+        int slot = blockIdx.x / a.nheads_k;
+        if constexpr (SPLIT) {
+            part = slot % S;
+            slot /= S;
+        }
+        const int it = a.work_order[slot];
         if (it < 0) return;
         b = __builtin_amdgcn_readfirstlane(it / nnb);
         nb = __builtin_amdgcn_readfirstlane(it - b * nnb);
@@ -372,6 +461,10 @@ __global__ __launch_bounds__(kDkvThreads, 2) void bwd_dkdv_kernel(const fa_bwd_a
         const int bh_count = a.batch * a.nheads_k;
         const int bhk = blockIdx.x % bh_count;
         nb = blockIdx.x / bh_count;  // smallest key blocks (most queries) first
+        if constexpr (SPLIT) {
+            part = nb % S;
+            nb /= S;
+        }
         b = bhk / a.nheads_k;
         hk = bhk - b * a.nheads_k;
     }
@@ -430,6 +523,15 @@ __global__ __launch_bounds__(kDkvThreads, 2) void bwd_dkdv_kernel(const fa_bwd_a
     // Query blocks that can see this key block, repeated for each q-head of the group.
     const int m_first = CAUSAL ? max(0, k0 - causal_off) / BM : 0;
     const int n_qb = max(0, (sq + BM - 1) / BM - m_first);
+    // SPLIT: this workgroup's share [t0, t1) of the G * n_qb steps (q-head
+    // slowest), starting at block i0 of q-head h0.
+    int t0 = 0, t1 = G * n_qb, h0 = 0, i0 = 0;
+    if constexpr (SPLIT) {
+        t0 = int(int64_t(G * n_qb) * part / S);
+        t1 = int(int64_t(G * n_qb) * (part + 1) / S);
+        h0 = n_qb > 0 ? t0 / n_qb : 0;
+        i0 = t0 - h0 * n_qb;
+    }
 
     TileCopier<HD, BM, NT> qcp, ocp;
     qcp.init(qrs, wave, lane);
@@ -444,10 +546,18 @@ __global__ __launch_bounds__(kDkvThreads, 2) void bwd_dkdv_kernel(const fa_bwd_a
     const f16 *ndo = (const f16 *)a.dout.ptr + base_off(a.dout, packed_q, b, si.q_start, hk * G);
     const float *nd = a.dsum + (int64_t(b) * a.nheads + hk * G) * a.lse_seqlen;
     int nh = 0, ni = 0;  // q-head (within the group) and block of the next copy
+    int left = t1 - t0;  // SPLIT: steps not yet copied
+    if constexpr (SPLIT) {
+        ni = i0;
+        nq += int64_t(h0) * a.q.head_stride;
+        ndo += int64_t(h0) * a.dout.head_stride;
+        nd += int64_t(h0) * a.lse_seqlen;
+    }
     const uint32_t smem_l = lds_addr(smem);
     const int64_t q_step = int64_t(BM) * qrs, do_step = int64_t(BM) * dors;
-    const f16 *nq_row = nq + int64_t(m_first) * q_step, *ndo_row = ndo + int64_t(m_first) * do_step;
+    const f16 *nq_row = nq + int64_t(m_first + ni) * q_step, *ndo_row = ndo + int64_t(m_first + ni) * do_step;
     auto issue_next = [&](int st) {
+        if constexpr (SPLIT) --left;
         const int q0 = (m_first + ni) * BM;
         const uint32_t qt_l = smem_l + st * C::STAGE, ot_l = qt_l + C::QTILE, lf_l = ot_l + C::QTILE;
         if (q0 + BM <= sq) {
@@ -594,7 +704,7 @@ __global__ __launch_bounds__(kDkvThreads, 2) void bwd_dkdv_kernel(const fa_bwd_a
     auto step = [&](int i, auto mask_tag, bool compute) {
         wait_vmem();
         __syncthreads();  // block j is in LDS; every wave is done with stage (j & 1) ^ 1
-        if (nh < G) issue_next((j & 1) ^ 1);
+        if (SPLIT ? left > 0 : nh < G) issue_next((j & 1) ^ 1);
         if (compute) block(j, (m_first + i) * BM, mask_tag);
         ++j;
     };
@@ -608,15 +718,27 @@ __global__ __launch_bounds__(kDkvThreads, 2) void bwd_dkdv_kernel(const fa_bwd_a
     // The first block's copies go out with the V rows and the K loads; the
     // first step's wait and barrier cover all of them.  With no block to walk,
     // the V copies still land before the wave ends.
-    if (n_qb > 0)
+    if (t1 > t0)
         issue_next(0);
     else
         wait_vmem();
-    for (int hidx = 0; hidx < G && n_qb > 0; ++hidx) {
-        for (int i = 0; i < i1; ++i) step(i, std::true_type{}, false);
-        for (int i = i1; i < i2; ++i) step(i, std::true_type{}, true);
-        for (int i = i2; i < i3; ++i) step(i, std::false_type{}, true);
-        for (int i = i3; i < n_qb; ++i) step(i, std::true_type{}, true);
+    if constexpr (SPLIT) {
+        for (int t = t0, i = i0; t < t1; i = 0) {
+            const int end = min(n_qb, i + t1 - t);
+            t += end - i;
+            for (const int e = min(i1, end); i < e; ++i) step(i, std::true_type{}, false);
+            for (const int e = min(i2, end); i < e; ++i) step(i, std::true_type{}, true);
+            for (const int e = min(i3, end); i < e; ++i) step(i, std::false_type{}, true);
+            for (; i < end; ++i) step(i, std::true_type{}, true);
+        }
+        if (S > 1 && !dkdv_reduce<HD>(a, (b * nnb + nb) * a.nheads_k + hk, part, S, &ticket, dk, dv)) return;
+    } else {
+        for (int hidx = 0; hidx < G && n_qb > 0; ++hidx) {
+            for (int i = 0; i < i1; ++i) step(i, std::true_type{}, false);
+            for (int i = i1; i < i2; ++i) step(i, std::true_type{}, true);
+            for (int i = i2; i < i3; ++i) step(i, std::false_type{}, true);
+            for (int i = i3; i < n_qb; ++i) step(i, std::true_type{}, true);
+        }
     }
 
     // Lane (col, hh) holds d = 32 dt + 8 a4 + 4 hh + t (accumulator 4 a4 + t)
@@ -687,12 +809,65 @@ static int launch_dq(const fa_bwd_args &a, hipStream_t s) {
     return int(hipGetLastError());
 }
 
+// Workgroups S that share a (batch, key block, KV head) item of the dK/dV
+// grid.  One each when the grid fills the chip; with few items, or causal ones
+// of very different lengths, the longest item decides the kernel's time and S
+// workgroups each take a share of its steps.  The estimate below (in steps of
+// 32 queries, about 1 us at head_dim 128 and 0.54 at 64 with two workgroups on
+// a CU) is the busiest CU's steps (equal items: whole rounds over the CUs;
+// causal ones are dealt longest first, about half an item of imbalance; a CU
+// with one workgroup is about 10 % slower per step), plus the partials'
+// traffic and the last workgroup's reads.  Measured on MI355X, causal
+// unless noted, us of the dK/dV kernel at S = 1 -> the S taken (best of 1..16):
+//   b1 s8192 32/8 d128: 1285 -> 1027 (S 4, 1027)   b1 s4096 32/8: 484 -> 288 (4, 280)
+//   b1 s2048 32/8: 248 -> 102 (4, 102)             b1 s512 32/8: 70 -> 36 (4, 36)
+//   b1 s4096 16/16: 170 -> 153 (2, 153)            b1 s2048 32/2: 960 -> 129 (12, 129)
+//   b1 s8192 32/8 d64: 789 -> 564 (4, 564)         b1 s4096 32/2 no mask: 1952 -> 520 (8, 520)
+//   b4 s1024 16/16: 52 (1; 70 at S 2)              b2 s4096 16/16 no mask: 501 (1; 534 at S 2)
+static int dkdv_splits(const fa_bwd_args &a) {
+    constexpr int kMaxSplits = 16;
+    constexpr int64_t kMaxBytes = int64_t(256) << 20;  // of partials
+    const int64_t items = dkdv_items(a), cus = device_cus();
+    const int64_t cap = std::min<int64_t>(kMaxSplits, kMaxBytes / std::max<int64_t>(1, items * 1024 * a.head_dim));
+    if (cap < 2 || a.seqlen_q <= 0) return 1;
+    const int nnb = (a.seqlen_k + 127) / 128, n_qb = (a.seqlen_q + 31) / 32, G = a.nheads / a.nheads_k;
+    const int64_t off = int64_t(a.seqlen_k) - a.seqlen_q;
+    // Steps of the longest item and of all items (varlen: as if every sequence were the longest).
+    const double longest = double(G) * n_qb;
+    double total = longest * nnb;
+    if (a.causal) {
+        total = 0;
+        for (int nb = 0; nb < nnb; ++nb)
+            total += double(G) * std::max<int64_t>(0, n_qb - std::max<int64_t>(0, int64_t(nb) * 128 - off) / 32);
+    }
+    total *= double(a.batch) * a.nheads_k / cus;
+    int best = 1;
+    double best_t = 0;
+    for (int S = 1; S <= cap; ++S) {
+        const int64_t wgs = items * S;
+        double t = a.causal ? std::max(longest / S, total * (1 + 0.5 * cus / wgs))
+                            : double((wgs + cus - 1) / cus) * longest / S;
+        if (wgs <= cus) t *= 1.1;
+        t += (S - 1) * (0.025 * items + 3);
+        if (S == 1 || t < best_t) {
+            best = S;
+            best_t = t;
+        }
+    }
+    return best;
+}
+static size_t dkdv_ws_bytes(const fa_bwd_args &a, int S) {
+    const int64_t items = dkdv_items(a);
+    return S > 1 ? size_t(dkdv_count_bytes(items) + items * S * 2 * 128 * a.head_dim * int64_t(sizeof(float))) : 0;
+}
+
 template <int HD, bool CAUSAL>
 static int launch_dkdv(const fa_bwd_args &a, hipStream_t s) {
     // seqlen_k bounds every sequence's key count (max_seqlen_k for varlen).
     static_assert(DkvCfg<HD>::BN == 128, "bwd_order_kernel and fa_bwd_order_len assume 128-key blocks");
     const int nnb = (a.seqlen_k + DkvCfg<HD>::BN - 1) / DkvCfg<HD>::BN;
-    const int64_t grid = int64_t(nnb) * a.batch * a.nheads_k;
+    const int S = a.split_ws && a.split_ws_bytes >= int64_t(dkdv_ws_bytes(a, dkdv_splits(a))) ? dkdv_splits(a) : 1;
+    const int64_t grid = int64_t(nnb) * a.batch * a.nheads_k * S;
     if (grid == 0) return FA_OK;
     if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
     if (a.work_order && a.cu_seqlens_k) {
@@ -700,7 +875,12 @@ static int launch_dkdv(const fa_bwd_args &a, hipStream_t s) {
         const int rc = int(hipGetLastError());
         if (rc) return rc;
     }
-    hipLaunchKernelGGL((bwd_dkdv_kernel<HD, CAUSAL>), dim3(unsigned(grid)), dim3(kDkvThreads), 0, s, a, nnb);
+    if (S > 1)
+        hipLaunchKernelGGL((bwd_dkdv_kernel<HD, CAUSAL, true>), dim3(unsigned(grid)), dim3(kDkvThreads), 0, s, a, nnb,
+                           S);
+    else
+        hipLaunchKernelGGL((bwd_dkdv_kernel<HD, CAUSAL, false>), dim3(unsigned(grid)), dim3(kDkvThreads), 0, s, a, nnb,
+                           1);
     return int(hipGetLastError());
 }
 
@@ -746,6 +926,13 @@ extern "C" size_t fa_bwd_order_len(const fa_bwd_args *a) {
     const size_t nnb = size_t((std::max(a->seqlen_k, 0) + 127) / 128);
     const size_t nmb = size_t((std::max(a->lse_seqlen, 0) + 31) / 32);  // dQ blocks of 32 positions at the least
     return size_t(a->batch) * (nnb + nmb);
+}
+
+extern "C" size_t fa_bwd_split_bytes(const fa_bwd_args *a) {
+    if (!a || a->batch <= 0 || a->seqlen_q <= 0 || a->seqlen_k <= 0 || a->nheads <= 0 || a->nheads_k <= 0 ||
+        (a->head_dim != 64 && a->head_dim != 128))
+        return 0;
+    return fa::dkdv_ws_bytes(*a, fa::dkdv_splits(*a));
 }
 
 extern "C" int fa_bwd(const fa_bwd_args *args, void *stream) {

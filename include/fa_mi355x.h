@@ -108,12 +108,24 @@ typedef struct fa_bwd_args {
      * first only when every sequence has the same length.  Results are the same
      * either way (each item is computed independently). */
     int32_t *work_order;
+    /* Optional workspace of split_ws_bytes >= fa_bwd_split_bytes(args) bytes,
+     * 256-byte aligned, when that is not 0: the grid of dK/dV key blocks is too
+     * small for the chip, and several workgroups then share each key block's
+     * queries and sum their fp32 partial dK / dV in it.  fa_bwd_dq or
+     * fa_bwd_preprocess clears its counters, fa_bwd_dkdv leaves them cleared.
+     * NULL (or a smaller one) gives each key block to one workgroup. */
+    void *split_ws;
+    int64_t split_ws_bytes;
 } fa_bwd_args;
 
 /* Length in int32s of the work_order workspace: batch * (ceil(seqlen_k / 128) +
  * ceil(lse_seqlen / 32)).  No counterpart in the reference (its grids are in
  * natural order). */
 size_t fa_bwd_order_len(const fa_bwd_args *args);
+/* Bytes of the split_ws workspace, 0 when the dK/dV grid fills the chip by
+ * itself.  It depends on the sizes, head counts, head_dim and causal alone.  No
+ * counterpart in the reference. */
+size_t fa_bwd_split_bytes(const fa_bwd_args *args);
 /* D = rowsum(dO * O) (flash_bwd_preprocess_kernel.h:23-96), stored negated in dsum plane 0. */
 int fa_bwd_preprocess(const fa_bwd_args *args, void *stream);
 /* dQ kernel (flash_bwd_kernel.h:25-609); computes and stores the dsum workspace itself. */
@@ -239,14 +251,14 @@ const char *fa_error_string(int code);
 
 /*
  * Version of the argument-struct layouts above.  It changes whenever a struct
- * gains, loses or moves a field (3: fa_fwd_args.work_order, fa_bwd_args.work_order
- * and fa_kvcache_args.split_count appended).  A caller compiled against this
+ * gains, loses or moves a field (4: fa_bwd_args.split_ws and split_ws_bytes
+ * appended).  A caller compiled against this
  * header checks fa_abi_version() == FA_ABI_VERSION once after loading the
  * library and refuses a mismatch: the entry points themselves cannot tell a
  * shorter struct from an older caller.  No counterpart in the reference (its
  * bindings are compiled together with its kernels).
  */
-#define FA_ABI_VERSION 3
+#define FA_ABI_VERSION 4
 int fa_abi_version(void);
 
 #ifdef __cplusplus
