@@ -706,6 +706,334 @@ __global__ __launch_bounds__(256, 2) void kv_splitkv_kernel(const fa_kvcache_arg
 }
 
 // ---------------------------------------------------------------------------
+// Many query rows per KV head (prompt chunks).  kv_splitkv_kernel reads a
+// split's K / V once per 32 rows, each wave its own tiles: at 512 tokens x 4
+// heads it reads them 64 times and runs at the L2's rate.  Here a workgroup
+// holds 128 rows, 32 per wave, and its waves share every 64-key block through
+// LDS (two stages, one barrier a block, two workgroups per CU), as in the
+// forward kernel; P still goes through PV as hi + lo fp16 halves, so each V
+// operand read from LDS feeds two MFMAs, and the matrix cores bound it (48
+// MFMAs a 32 x 64 block and wave against 326 VALU instructions).  Two sequences
+// of 512 tokens on 4k - 12k keys, 32 / 8 heads, head_dim 128: 452 -> 205 us a
+// call (288 -> 635 TFLOP/s with PV counted once, about 950 as executed).
+// Items, their order and the options are kv_splitkv_kernel's; a split takes a
+// share of the keys that some row of its tile sees (with a window those are
+// few of the sequence's).  With num_splits > 1 the last split of a row tile to
+// finish adds the others' partials to its own.
+constexpr int kChunkRows = 128, kChunkKeys = 64, kChunkPages = 1024;
+constexpr int kChunkMinRows = 64, kChunkMaxSplits = 32;
+
+// Merges the partial rows (O normalised, LSE) of a row tile's splits.  The
+// first S - 1 items to get here (count[0]) store theirs, lane by lane, and
+// count them stored (count[1]); the last one waits for those stores, which are
+// under way, and sums all in split order, its own from registers.  row0:
+// the tile's first row of a split's accumulators, rows_here x HD values from there.
+// Returns whether this item holds the sum.
+template <int HD>
+__device__ __forceinline__ bool chunk_merge(const fa_kvcache_args &a, int32_t *count, int split, int64_t row0,
+                                            int rows_here, int row, int hh, int *ticket, f32x16 (&o)[HD / 32],
+                                            float &lse) {
+    constexpr int N = HD / 4;  // pairs of floats a lane holds
+    const int S = a.num_splits, tid = threadIdx.x;
+    const int64_t nrow = int64_t(a.batch) * a.nheads * a.seqlen_q;
+    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const bool live = row < rows_here;
+    // Pair i of a lane: element (2 i + hh) * rows_here + row, 256 contiguous bytes a half wave.
+    uint64_t *pairs = reinterpret_cast<uint64_t *>(a.out_accum + row0 * HD) + hh * rows_here + row;
+    const int step = 2 * rows_here;
+    float *lses = a.lse_accum + row0 + row;
+    if (*ticket < S - 1) {
+        if (live) {
+            uint64_t *slot = pairs + int64_t(split) * nrow * (HD / 2);
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const f32x2 x = {o[i / 8][2 * (i & 7)], o[i / 8][2 * (i & 7) + 1]};
+                __hip_atomic_store(slot + i * step, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (hh == 0)
+                __hip_atomic_store(lses + int64_t(split) * nrow, lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        wait_vmem();
+        __syncthreads();  // every wave's stores have completed
+        if (tid == 0) __hip_atomic_fetch_add(count + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+    }
+    if (tid == 0)
+        while (__hip_atomic_load(count + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < S - 1)
+            __builtin_amdgcn_s_sleep(1);
+    __syncthreads();
+    if (!live) return true;
+    auto lse_of = [&](int s) {
+        return s == split ? lse
+                          : __hip_atomic_load(lses + int64_t(s) * nrow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    float mx = -INFINITY, sum = 0.f;
+    for (int s = 0; s < S; ++s) mx = fmaxf(mx, lse_of(s));
+    for (int s = 0; s < S; ++s) sum += mx == -INFINITY ? 0.f : expf(lse_of(s) - mx);
+    const float total = mx == -INFINITY ? -INFINITY : mx + logf(sum);
+    f32x16 acc[HD / 32];
+#pragma unroll
+    for (int i = 0; i < HD / 32; ++i) acc[i] = zero16();
+    for (int s = 0; s < S; ++s) {
+        const float w = total == -INFINITY ? 0.f : expf(lse_of(s) - total);
+        const uint64_t *slot = pairs + int64_t(s) * nrow * (HD / 2);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            // (The own slot is read as well, and not used.)
+            const f32x2 x = __builtin_bit_cast(
+                f32x2, __hip_atomic_load(slot + i * step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            f32x16 &t = acc[i / 8];
+            t[2 * (i & 7)] = fmaf(w, s == split ? o[i / 8][2 * (i & 7)] : x[0], t[2 * (i & 7)]);
+            t[2 * (i & 7) + 1] = fmaf(w, s == split ? o[i / 8][2 * (i & 7) + 1] : x[1], t[2 * (i & 7) + 1]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < HD / 32; ++i) o[i] = acc[i];
+    lse = total;
+    return true;
+}
+
+template <int HD, bool EXT>
+__global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcache_args a, const int row_tiles,
+                                                                 int32_t *const count) {
+    constexpr int BN = kChunkKeys, TILE = BN * HD * 2, STAGE = 2 * TILE;
+    __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+    __shared__ int pages[kChunkPages];
+    __shared__ int ticket;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31, hh = lane >> 5;
+    const int G = a.nheads / a.nheads_k, R = G * a.seqlen_q, S = a.num_splits;
+    TileReader<HD> rd;
+    rd.init(lane);
+    const int64_t krs = a.k_cache.row_stride, vrs = a.v_cache.row_stride;
+    TileCopier<HD, BN, kKvThreads> kcp, vcp;
+    kcp.init(krs, wave, lane);
+    vcp.init(vrs, wave, lane);
+    int rest = blockIdx.x;
+    const int rt = rest % row_tiles;
+    rest /= row_tiles;
+    const int hk = rest % a.nheads_k;
+    rest /= a.nheads_k;
+    const int split = rest % S;
+    const int b = a.batch_order[rest / S];
+
+    const KvSeq sq = kv_seq(a, b);
+    if (sq.err && a.status && tid == 0) atomicOr(a.status, sq.err);
+    const int L = sq.err ? 0 : sq.L0 + a.seqlen_new;
+    const int kstart = EXT && a.cache_leftpad ? min(max(a.cache_leftpad[b], 0), L) : 0;
+
+    // This lane's query row (row qpos * G + g of the KV head).
+    const int first = rt * kChunkRows, rows_here = min(kChunkRows, R - first);
+    const int row = 32 * wave + col;
+    const bool row_ok = row < rows_here;
+    const int qpos = row_ok ? (first + row) / G : 0;
+    const int hq = hk * G + (row_ok ? (first + row) % G : 0);
+    const int off = L - a.seqlen_q;  // key position of query 0
+    const int qkey = qpos + off;
+    // Keys [key_lo, key_hi) a query at key position p sees.  The splits divide
+    // the keys that some row of the tile sees, [t_lo, t_hi).
+    const int wl = EXT && a.local_window ? a.window_left : -1, wr = EXT && a.local_window ? a.window_right : -1;
+    auto key_lo = [&](int p) { return wl >= 0 ? max(kstart, p - wl) : kstart; };
+    auto key_hi = [&](int p) {
+        int hi = a.causal ? min(L, p + 1) : L;
+        if (wr >= 0) hi = min(hi, p + wr + 1);
+        return hi;
+    };
+    const int t_lo = key_lo(first / G + off), t_n = max(0, key_hi((first + rows_here - 1) / G + off) - t_lo);
+    const int s0 = t_lo + int(int64_t(t_n) * split / S), s1 = t_lo + int(int64_t(t_n) * (split + 1) / S);
+    const int nb0 = s0 / BN, nb1 = s1 > s0 ? (s1 - 1) / BN + 1 : nb0;
+    // Of the split's keys: those the lane's row sees, [lo, hi), those some row
+    // of the wave sees and those every row of it sees.
+    const int lo = max(s0, key_lo(qkey)), hi = min(s1, key_hi(qkey));
+    const int p0w = (first + 32 * wave) / G + off, p1w = (first + min(rows_here, 32 * wave + 32) - 1) / G + off;
+    const int any_lo = max(s0, key_lo(p0w)), any_hi = 32 * wave < rows_here ? min(s1, key_hi(p1w)) : s0;
+    const int all_lo = max(s0, key_lo(p1w)), all_hi = min(s1, key_hi(p0w));
+
+    const bool neg = a.softmax_scale < 0.f;
+    const bool capped = EXT && a.softcap > 0.f, alibi = EXT && a.alibi_slopes != nullptr;
+    const bool natural = capped || alibi;  // scores formed in natural units
+    const float cscale = natural ? kLog2e : fabsf(a.softmax_scale) * kLog2e;
+    const float cap_in = capped ? fabsf(a.softmax_scale) / a.softcap : 0.f;
+    const float slope = alibi ? a.alibi_slopes[int64_t(b) * a.alibi_batch_stride + hq] : 0.f;
+    const int rpos = sq.L0 + (a.causal || a.local_window ? qpos : 0);  // rotary position
+    f16x8 qB[HD / 16];
+    {
+        const f16 *qp = (const f16 *)a.q.ptr + int64_t(b) * a.q.batch_stride + int64_t(qpos) * a.q.row_stride +
+                        int64_t(hq) * a.q.head_stride;
+#pragma unroll
+        for (int g = 0; g < HD / 16; ++g) {
+            u32x4 v = row_ok ? ldg16(qp + 16 * g + 8 * hh) : zero_u4();
+            if (EXT && row_ok && 16 * g + 8 * hh < a.rotary_dim) v = rotary8(a, v, qp, 16 * g + 8 * hh, rpos);
+            if (neg) v = neg_h8(v);
+            qB[g] = as_h8(v);
+        }
+    }
+    // Page ids of the walked keys (the launcher takes this kernel only when they fit).
+    const int page = a.page_block_size;
+    const int pg0 = a.block_table ? nb0 * BN / page : 0;
+    if (a.block_table && nb1 > nb0) {
+        const int32_t *bt = a.block_table + int64_t(b) * a.block_table_stride + pg0;
+        const int n_pages = (nb1 * BN - 1) / page - pg0 + 1;
+        for (int i = tid; i < n_pages; i += kKvThreads) pages[i] = bt[i];
+    }
+    wait_vmem();  // only the tile copies are in flight in the loop
+    __syncthreads();
+
+    const f16 *kc = (const f16 *)a.k_cache.ptr + int64_t(hk) * a.k_cache.head_stride;
+    const f16 *vc = (const f16 *)a.v_cache.ptr + int64_t(hk) * a.v_cache.head_stride;
+    auto issue = [&](int nb) FA_INLINE {
+        int64_t blk = sq.row;
+        int at = nb * BN;  // token within the cache row or page
+        if (a.block_table) {
+            const int pi = at / page;
+            blk = __builtin_amdgcn_readfirstlane(pages[pi - pg0]);
+            at -= pi * page;
+        }
+        const f16 *kb = kc + blk * a.k_cache.batch_stride + int64_t(at) * krs;
+        const f16 *vb = vc + blk * a.v_cache.batch_stride + int64_t(at) * vrs;
+        const int soff = (nb & 1) * STAGE;
+        if (nb * BN + BN <= L) {
+            kcp.template copy_to<true>(lds_addr(smem) + soff, kb, krs);
+            vcp.template copy_to<true>(lds_addr(smem) + soff + TILE, vb, vrs);
+        } else {  // keys past L re-read key L - 1 (masked)
+            dma_tile<HD, BN, kKvThreads>(smem + soff, kb, krs, 0, L - 1 - nb * BN, wave, lane);
+            dma_tile<HD, BN, kKvThreads>(smem + soff + TILE, vb, vrs, 0, L - 1 - nb * BN, wave, lane);
+        }
+    };
+
+    f32x16 o[HD / 32];
+#pragma unroll
+    for (int i = 0; i < HD / 32; ++i) o[i] = zero16();
+    float m_t = -INFINITY, l_p = 0.f;
+    if (nb1 > nb0) issue(nb0);
+    for (int nb = nb0; nb < nb1; ++nb) {
+        wait_vmem();
+        __syncthreads();  // block nb is in LDS; every wave is done with the other stage
+        if (nb + 1 < nb1) issue(nb + 1);
+        const int p0 = nb * BN;
+        if (p0 >= any_hi || p0 + BN <= any_lo) continue;  // no key for this wave
+        // The lane's read bases with this block's stage added (opaque, so the
+        // per-read addresses are not hoisted to hold registers; see TileReader).
+        const int soff = (nb & 1) * STAGE;
+        int ab = rd.a_base + soff, tb0 = rd.tr_base[0] + soff, tb1 = rd.tr_base[1] + soff;
+        asm volatile("" : "+v"(ab), "+v"(tb0), "+v"(tb1));
+        f32x16 s[2];
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+            s[kt] = zero16();
+#pragma unroll
+            for (int g = 0; g < HD / 16; ++g)
+                s[kt] = mfma32(rd.a_operand_at(smem + 32 * kt * (HD * 2), ab, g), qB[g], s[kt]);
+        }
+        if constexpr (EXT) {
+            if (natural) {
+                const float sc = fabsf(a.softmax_scale);
+                const float dist0 = float(qkey - p0 - 8 * hh);
+#pragma unroll
+                for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        float x = capped ? a.softcap * tanh_fast(s[kt][r] * cap_in) : s[kt][r] * sc;
+                        if (alibi) x -= slope * fabsf(dist0 - float(kt * 32 + acc_lrow(r, 0)));
+                        s[kt][r] = x;
+                    }
+            }
+        }
+        if (p0 < all_lo || p0 + BN > all_hi) {
+            const int lo_c = lo - p0 - 8 * hh, hi_c = hi - p0 - 8 * hh;
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int c = kt * 32 + acc_lrow(r, 0);
+                    if (c < lo_c || c >= hi_c) s[kt][r] = -INFINITY;
+                }
+        }
+        float mx = s[0][0];
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kt][r]);
+        mx = max_xor32(mx);
+        const float mx_t = mx == -INFINITY ? -INFINITY : mx * cscale;
+        if (__builtin_amdgcn_ballot_w64(mx_t > m_t + kKvRescaleSlack) != 0) {
+            const float m_new = fmaxf(m_t, mx_t);
+            const float alpha = m_new == -INFINITY ? 1.f : exp2_fast(m_t - m_new);
+            l_p *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < HD / 32; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+            m_t = m_new;
+        }
+        const float m_use = m_t == -INFINITY ? 0.f : m_t;
+        float rs = 0.f;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float p = exp2_fast(fmaf(s[kt][r], cscale, -m_use));
+                s[kt][r] = p;
+                rs += p;
+            }
+        l_p += rs;
+        float minus1 = -1.f;
+        asm("" : "+v"(minus1));
+#pragma unroll
+        for (int gg = 0; gg < 4; ++gg) {
+            f16x8 pl;
+            u32x4 hi4 = __builtin_bit_cast(u32x4, pack8(s[gg >> 1], 8 * (gg & 1)));
+            asm("" : "+v"(hi4));  // opaque: the halves below come from the packed words, not from conversions of their own
+            const f16x8 ph = as_h8(hi4);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) pl[u] = (f16)fmaf(float(ph[u]), minus1, s[gg >> 1][8 * (gg & 1) + u]);
+#pragma unroll
+            for (int dt = 0; dt < HD / 32; ++dt) {
+                const f16x8 va = rd.tr_operand_at(smem + TILE + 16 * gg * (HD * 2), tb0, tb1, dt);
+                o[dt] = mfma32(va, ph, o[dt]);
+                o[dt] = mfma32(va, pl, o[dt]);
+            }
+        }
+    }
+
+    const float l_tot = sum_xor32(l_p);
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    float lse = l_tot > 0.f ? (m_t + log2_fast(l_tot)) * kLn2 : -INFINITY;
+#pragma unroll
+    for (int dt = 0; dt < HD / 32; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[dt][r] *= inv;
+    const int64_t tile = (int64_t(b) * a.nheads_k + hk) * row_tiles + rt;
+    const int64_t row0 = (int64_t(b) * a.nheads_k + hk) * R + first;
+    // Opaque to the optimiser: the row's output addresses are formed here, not
+    // before the block loop and held through it.
+    int orow = row;
+    asm volatile("" : "+v"(orow));
+    if (S == 1 || chunk_merge<HD>(a, count + 2 * tile, split, row0, rows_here, orow, hh, &ticket, o, lse)) {
+        if (orow < rows_here) {
+            const int oq = (first + orow) / G, oh = hk * G + (first + orow) % G;
+            f16 *op = (f16 *)a.o.ptr + int64_t(b) * a.o.batch_stride + int64_t(oq) * a.o.row_stride +
+                      int64_t(oh) * a.o.head_stride;
+#pragma unroll
+            for (int dt = 0; dt < HD / 32; ++dt)
+#pragma unroll
+                for (int a4 = 0; a4 < 4; ++a4) {
+                    f16x4 v;
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) v[t] = (f16)o[dt][4 * a4 + t];
+                    *reinterpret_cast<f16x4 *>(op + dt * 32 + 8 * a4 + 4 * hh) = v;
+                }
+            if (hh == 0)
+                a.lse[(int64_t(b) * a.nheads + oh) * a.seqlen_q + oq] = lse == -INFINITY ? 0.f : lse;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Combine kernel: one wave per (batch, head, qpos) row.
 template <int HD>
 __global__ __launch_bounds__(256) void kv_combine_kernel(const fa_kvcache_args a) {
@@ -732,6 +1060,30 @@ static int check_kv(const fa_kvcache_args *p) {
     return FA_OK;
 }
 
+// Splits of the many-row kernel: the fewest key blocks on the busiest CU (a CU
+// with one workgroup is about 10 % slower per block) and 1.3 blocks' time for
+// every split to merge.  Measured on MI355X with 32 / 8 heads, head_dim 128, us
+// per call at 1 split -> the splits taken: 512 rows x 1 sequence of 8k keys
+// 226 -> 128 (4 splits), 128 x 1 x 8k 214 -> 59 (8), 32 x 8 x 8k 215 -> 82 (4),
+// 1024 x 1 x 15k 444 -> 410 (2).
+static int chunk_num_splits(int64_t heads, int rows, int capacity, int num_cus) {
+    const int64_t tiles = heads * ((rows + kChunkRows - 1) / kChunkRows), cus = std::max(num_cus, 1);
+    const double blocks = (double(capacity) + kChunkKeys - 1) / kChunkKeys;
+    int best = 1;
+    double best_t = 0;
+    for (int S = 1; S <= 16 && (S == 1 || blocks >= 4 * S); ++S) {
+        const int64_t wgs = tiles * S;
+        double t = double((wgs + cus - 1) / cus) * blocks / S;
+        if (wgs <= cus) t *= 1.1;
+        t += 1.3 * (S - 1);
+        if (S == 1 || t < best_t) {
+            best = S;
+            best_t = t;
+        }
+    }
+    return best;
+}
+
 }  // namespace fa
 
 extern "C" int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_dim, int seqlen_q, int batch,
@@ -750,6 +1102,7 @@ extern "C" int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_d
     if (requested > 0) return requested;
     if (batch <= 0 || nheads_k <= 0 || nheads <= 0 || seqlen_k_capacity <= 0) return 1;
     const int rows = (nheads / nheads_k) * seqlen_q;
+    if (rows >= fa::kChunkMinRows) return fa::chunk_num_splits(int64_t(batch) * nheads_k, rows, seqlen_k_capacity, num_cus);
     const int64_t wgs = int64_t(batch) * nheads_k * ((rows + 31) / 32);
     const int64_t by_len = (int64_t(seqlen_k_capacity) + 4096) / 8192;
     const int64_t by_fill = (int64_t(std::max(num_cus, 1)) + wgs - 1) / std::max<int64_t>(wgs, 1);
@@ -843,10 +1196,42 @@ int kv_heads_per_item(const fa_kvcache_args &a) {
     return hpi;
 }
 
+// Whether the split kernel of a call is kv_chunk_kernel: at least 64 query rows
+// per KV head (with 64 rows, 8 sequences of 8k keys, 32 / 8 heads: 71 us against
+// 114 at the best split counts; one sequence 50 against 49; with 32 rows the
+// other kernel reads K and V once as well and its waves share the keys), few
+// enough splits for one workgroup to merge, and the split counts to do it with.
+// Its 64-key blocks must not straddle pages, and its page ids fit in LDS.
+bool use_chunk(const fa_kvcache_args &a) {
+    const int R = (a.nheads / a.nheads_k) * a.seqlen_q;
+    if (R < kChunkMinRows || a.num_splits > kChunkMaxSplits || !a.batch_order || (a.num_splits > 1 && !a.split_count))
+        return false;
+    return !a.block_table || (a.page_block_size % kChunkKeys == 0 && a.cache_capacity > 0 &&
+                              a.cache_capacity / a.page_block_size <= kChunkPages);
+}
+int launch_chunk(const fa_kvcache_args &a, hipStream_t s) {
+    const int row_tiles = ((a.nheads / a.nheads_k) * a.seqlen_q + kChunkRows - 1) / kChunkRows;
+    const int64_t n = int64_t(a.batch) * a.nheads_k * row_tiles * a.num_splits;
+    if (n == 0) return FA_OK;
+    const bool ext = a.local_window || a.softcap > 0.f || a.cache_leftpad || a.alibi_slopes || a.rotary_dim > 0;
+    auto go = [&](auto hd_tag, auto ext_tag) {
+        hipLaunchKernelGGL((kv_chunk_kernel<decltype(hd_tag)::value, decltype(ext_tag)::value>), dim3(unsigned(n)),
+                           dim3(kKvThreads), 0, s, a, row_tiles, a.split_count);
+    };
+    using H128 = std::integral_constant<int, 128>;
+    using H64 = std::integral_constant<int, 64>;
+    if (a.head_dim == 128)
+        ext ? go(H128{}, std::true_type{}) : go(H128{}, std::false_type{});
+    else
+        ext ? go(H64{}, std::true_type{}) : go(H64{}, std::false_type{});
+    return int(hipGetLastError());
+}
+
 // The split kernel.  With batch_order (ranked and its counter reset by
 // launch_prep on the same stream): a resident grid of two workgroups per CU
 // that deals the items out in that order.  Without it: one workgroup per item.
 int launch_split(const fa_kvcache_args &a, hipStream_t s) {
+    if (use_chunk(a)) return launch_chunk(a, s);
     const int hpi = kv_heads_per_item(a);
     const int64_t gx = split_items(a) / hpi;
     if (gx == 0) return FA_OK;

@@ -201,7 +201,7 @@ typedef struct fa_kvcache_args {
     int32_t rotary_interleaved;
     /* Workspace of fa_kv_split_count_len(args) int32s, or NULL.  With it, batch_order
      * and num_splits > 1, the split kernel combines the partials itself: the last of
-     * the num_splits items of each (batch, kv head, 32-row tile) to finish reads them
+     * the num_splits items of each (batch, kv head, row tile) to finish reads them
      * and writes o and lse, so fa_kv_combine has nothing left to do (it returns at
      * once) and fa_fwd_kvcache runs two kernels (append with ordering, split) instead
      * of four.  The ordering kernel zeroes these counts on every call. */

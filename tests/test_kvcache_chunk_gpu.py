@@ -1,0 +1,90 @@
+"""KV-cache calls with many query rows per KV head (kv_chunk_kernel: 128-row
+tiles over shared 64-key blocks) against the oracle, at the sizes where its
+tiles, blocks, splits and masks end; the same logical cache contiguous, remapped
+and paged must give the same bits."""
+
+import pytest
+import torch
+
+import flash_attention_interface as fai
+from helpers import assert_2x, assert_lse, kv_oracle, randn16
+from oracle import kvcache as okv
+from test_kvcache_gpu import _paged_from_contiguous
+
+# batch, queries, heads, kv heads, head_dim, capacity, appended, lengths before the append, splits, causal, options.
+# 64 rows (the least), 65, 127 - 129, a group of 3; keys at block and page edges, an empty cache, fewer keys than
+# splits; windows smaller than a tile's positions, keys before a leftpad, every option at once.
+CASES = [
+    (2, 16, 8, 2, 128, 512, 16, (0, 496), 1, True, {}),
+    (2, 13, 10, 2, 64, 768, 5, (64, 700), 3, True, {}),
+    (1, 43, 3, 1, 128, 1024, 43, (213,), 4, True, {}),
+    (3, 32, 8, 2, 64, 512, 0, (512, 1, 0), 5, False, {}),
+    (2, 127, 2, 2, 128, 768, 127, (1, 641), 0, True, {}),
+    (1, 300, 4, 4, 64, 1280, 300, (900,), 0, True, {}),
+    (1, 100, 6, 2, 128, 2048, 100, (1500,), 2, False, {}),
+    (2, 33, 8, 2, 128, 1024, 33, (900, 40), 3, True, {"window": (70, -1)}),
+    (2, 64, 4, 2, 64, 1024, 64, (950, 100), 2, False, {"window": (5, 200)}),
+    (2, 40, 4, 1, 128, 768, 40, (300, 700), 2, True, {"softcap": 15.0, "alibi": True}),
+    (2, 40, 4, 1, 64, 768, 40, (300, 700), 0, False, {"leftpad": (33, 650), "alibi": True}),
+    (2, 50, 6, 2, 128, 768, 50, (130, 700), 3, True, {"rotary": 64, "window": (200, 0), "softcap": 20.0,
+                                                      "leftpad": (100, 0)}),
+]
+
+
+def _call(device, q, kc, vc, k, v, lens, idx, table, splits, causal, kw):
+    dev = lambda t: None if t is None else t.to(device)  # noqa: E731
+    kcd, vcd = kc.clone().to(device), vc.clone().to(device)
+    out, lse = fai.flash_attn_with_kvcache(
+        q.to(device), kcd, vcd, k=dev(k), v=dev(v), cache_seqlens=lens.to(device), cache_batch_idx=dev(idx),
+        block_table=dev(table), causal=causal, num_splits=splits, return_softmax_lse=True,
+        **{n: dev(x) if isinstance(x, torch.Tensor) else x for n, x in kw.items()})
+    torch.cuda.synchronize()
+    return out.cpu(), lse.cpu(), kcd.cpu(), vcd.cpu()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_kvcache_chunk(device, case):
+    b, sq, h, hk, hd, cap, new, lens, splits, causal, opt = CASES[case]
+    g = torch.Generator().manual_seed(8300 + case)
+    print(f"case chunk {CASES[case]}", flush=True)
+    q, kc, vc = randn16((b, sq, h, hd), g), randn16((b, cap, hk, hd), g), randn16((b, cap, hk, hd), g)
+    k = randn16((b, new, hk, hd), g) if new else None
+    v = randn16((b, new, hk, hd), g) if new else None
+    seqlens = torch.tensor(lens, dtype=torch.int32)
+    ends = seqlens + new
+    window, softcap = opt.get("window", (-1, -1)), opt.get("softcap", 0.0)
+    slopes = 2.0 ** -torch.arange(1, h + 1, dtype=torch.float32) if opt.get("alibi") else None
+    leftpad = torch.tensor(opt["leftpad"], dtype=torch.int32) if "leftpad" in opt else None
+    kw = dict(window_size=window, softcap=softcap, alibi_slopes=slopes, cache_leftpad=leftpad)
+    q_ref, k_ref = q, k
+    if "rotary" in opt:
+        angle = torch.rand((cap, opt["rotary"] // 2), generator=g) * 6.0
+        kw.update(rotary_cos=angle.cos().half(), rotary_sin=angle.sin().half(), rotary_interleaved=False)
+        pos = seqlens.long()[:, None]
+        step = torch.arange(sq)[None, :]
+        q_ref = okv.rotary_embed(q, kw["rotary_cos"], kw["rotary_sin"], pos + step, False)
+        k_ref = okv.rotary_embed(k, kw["rotary_cos"], kw["rotary_sin"], pos + step[:, :new], False)
+    _, _, kc_ref, vc_ref = kv_oracle(q, kc, vc, k_ref, v, seqlens, None, None, causal, 1, None)
+    ku, vu = okv.materialize(kc_ref, vc_ref, ends, None, None)
+    o_ref, l_ref = okv.splitkv_attention(q_ref, ku, vu, ends, hd ** -0.5, causal, 1, window=window, softcap=softcap,
+                                         alibi_slopes=slopes, leftpad=leftpad)
+    kp, vp, table = _paged_from_contiguous(kc, vc, torch.full_like(seqlens, cap - new), 256, g)
+    perm = torch.randperm(b + 2, generator=g)[:b].to(torch.int32)
+    kr, vr = randn16((b + 2, cap, hk, hd), g), randn16((b + 2, cap, hk, hd), g)
+    kr[perm.long()], vr[perm.long()] = kc, vc
+    got = _call(device, q, kp, vp, k, v, seqlens, None, table, splits, causal, kw)
+    assert_2x("out", got[0], o_ref, o_ref.to(torch.float16))
+    assert_lse(got[1], l_ref)
+    again = _call(device, q, kp, vp, k, v, seqlens, None, table, splits, causal, kw)
+    assert torch.equal(got[0], again[0]) and torch.equal(got[1], again[1]), "whichever split finishes last"
+    if splits > 1 or opt:  # contiguous caches take this kernel too
+        plain = _call(device, q, kc, vc, k, v, seqlens, None, None, splits, causal, kw)
+        remap = _call(device, q, kr, vr, k, v, seqlens, perm, None, splits, causal, kw)
+        assert torch.equal(plain[2], kc_ref) and torch.equal(plain[3], vc_ref)
+        if splits > 1:
+            for x in (plain, remap):
+                assert torch.equal(x[0], got[0]) and torch.equal(x[1], got[1])
+        else:  # the heuristic may cut another capacity into another number of splits
+            assert_2x("out", plain[0], o_ref, o_ref.to(torch.float16))
+            assert_2x("out", remap[0], o_ref, o_ref.to(torch.float16))
