@@ -26,7 +26,9 @@
 //     separated by workgroup barriers, so one group's softmax runs on the
 //     VALU while the other group's MFMAs run on the matrix cores;
 //   * fwd_kernel (head_dim 64 and small grids): 4 waves, two (head_dim 128)
-//     or three (head_dim 64) independent workgroups per CU.
+//     or three (head_dim 64) independent workgroups per CU; on grids too small
+//     for that, two groups of 4 waves per workgroup and several workgroups per
+//     query block share the key blocks (fwd_plan).
 #include <type_traits>
 
 #include "fa_common.h"
@@ -67,23 +69,23 @@ struct FwdWork {
     bool neg;
 };
 
-// Fills w for workgroup blockIdx.x; false when the block has no query rows
+// Fills w for workgroup bid (of the unsplit grid); false when the block has no query rows
 // (its LSE padding is then written here).
 template <int BM, bool CAUSAL>
-__device__ __forceinline__ bool fwd_work(const fa_fwd_args &a, int num_m_blocks, int lg, FwdWork &w) {
+__device__ __forceinline__ bool fwd_work(const fa_fwd_args &a, int num_m_blocks, int lg, int bid, FwdWork &w) {
     int mb;
     const int gp = 1 << lg;
     const int packs = a.nheads >> lg;  // head packs per batch
     if (a.work_order && a.cu_seqlens_q) {
         // Item of the device-built order (head packs fastest), longest first.
-        const int it = a.work_order[blockIdx.x / packs];
+        const int it = a.work_order[bid / packs];
         w.b = __builtin_amdgcn_readfirstlane(it / num_m_blocks);
         mb = __builtin_amdgcn_readfirstlane(it - w.b * num_m_blocks);
-        w.h = (blockIdx.x % packs) * gp;
+        w.h = (bid % packs) * gp;
     } else {
         const int bp_count = a.batch * packs;
-        const int bp = blockIdx.x % bp_count;
-        mb = blockIdx.x / bp_count;
+        const int bp = bid % bp_count;
+        mb = bid / bp_count;
         if (CAUSAL) mb = num_m_blocks - 1 - mb;  // causal blocks are issued heaviest first
         w.b = bp / packs;
         w.h = (bp - w.b * packs) * gp;
@@ -213,15 +215,15 @@ __device__ __forceinline__ void softmax_block(f32x16 (&s)[2], f16x8 (&pB)[4], f3
 }
 
 // Epilogue: O / l in fp16, LSE = ln(sum exp(scale*S)); empty rows give 0 / 0.
-template <int HD>
+// Dimension tiles [D0, D1); the LSE goes with the first one.
+template <int HD, int D0, int D1>
 __device__ __forceinline__ void store_row(const fa_fwd_args &a, const FwdWork &w, int qi, int hh,
-                                          const f32x16 (&o)[HD / 32], const SoftmaxRow &r) {
-    const float l_tot = sum_xor32(r.l_p);
+                                          const f32x16 (&o)[HD / 32], float m_t, float l_tot) {
     if (qi < w.sq) {
         const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
         f16 *orow = w.op + int64_t(qi) * a.o.row_stride;
 #pragma unroll
-        for (int dt = 0; dt < HD / 32; ++dt)
+        for (int dt = D0; dt < D1; ++dt)
 #pragma unroll
             for (int a4 = 0; a4 < 4; ++a4) {
                 f16x4 v;
@@ -229,10 +231,86 @@ __device__ __forceinline__ void store_row(const fa_fwd_args &a, const FwdWork &w
                 for (int t = 0; t < 4; ++t) v[t] = (f16)(o[dt][4 * a4 + t] * inv);
                 *reinterpret_cast<f16x4 *>(orow + dt * 32 + 8 * a4 + 4 * hh) = v;
             }
-        if (hh == 0) w.lse_row[qi] = l_tot > 0.f ? (r.m_t + log2_fast(l_tot)) * kLn2 : 0.f;
-    } else if (hh == 0 && qi < a.lse_seqlen) {
+        if (D0 == 0 && hh == 0) w.lse_row[qi] = l_tot > 0.f ? (m_t + log2_fast(l_tot)) * kLn2 : 0.f;
+    } else if (D0 == 0 && hh == 0 && qi < a.lse_seqlen) {
         w.lse_row[qi] = 0.f;
     }
+}
+
+// Splits (fwd_kernel, SPLIT): the workspace starts with two int32 counters per
+// workgroup of the unsplit grid (an item: 128 rows), then, 256-byte aligned, the
+// items' S x 128 rows' (maximum, sum) and their S x 128 x HD partial O in fp32.
+__host__ __device__ __forceinline__ int64_t fwd_count_bytes(int64_t items) { return (items * 8 + 255) & ~int64_t(255); }
+
+// Sums the S partial results of an item over dimension tiles [D0, D1) of O.
+// The first S - 1 workgroups to get here (count[0]) store theirs and count them
+// stored (count[1]); the last one waits for those stores, which are under way,
+// and sums all in split order, its own from registers.  Returns whether this
+// workgroup holds the sum.
+template <int HD, int D0, int D1>
+__device__ __forceinline__ bool fwd_merge(const fa_fwd_args &a, int64_t items, int item, int part, int S, int r,
+                                          int *ticket, f32x16 (&o)[HD / 32], float &m, float &l) {
+    constexpr int N = 8 * (D1 - D0), NT = 512;  // pairs of floats a lane holds, threads
+    const int tid = threadIdx.x, hh = (tid >> 5) & 1;
+    int32_t *count = reinterpret_cast<int32_t *>(a.split_ws) + 2 * int64_t(item);
+    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int got = *ticket;
+    uint64_t *rows = reinterpret_cast<uint64_t *>(static_cast<char *>(a.split_ws) + fwd_count_bytes(items));
+    uint64_t *pairs = rows + items * S * 128 + int64_t(item) * S * N * NT + tid;
+    rows += int64_t(item) * S * 128 + r;
+    if (got < S - 1) {
+        uint64_t *slot = pairs + int64_t(part) * N * NT;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const f32x16 &t = o[D0 + i / 8];
+            const f32x2 x = {t[2 * (i & 7)], t[2 * (i & 7) + 1]};
+            __hip_atomic_store(slot + i * NT, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (D0 == 0 && hh == 0)
+            __hip_atomic_store(rows + part * 128, __builtin_bit_cast(uint64_t, f32x2{m, l}), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        wait_vmem();
+        __syncthreads();  // every wave's stores have completed
+        if (tid == 0) __hip_atomic_fetch_add(count + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+    }
+    if (tid == 0)
+        while (__hip_atomic_load(count + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < S - 1)
+            __builtin_amdgcn_s_sleep(1);
+    __syncthreads();
+    auto row_of = [&](int p) {
+        return p == part ? f32x2{m, l}
+                         : __builtin_bit_cast(f32x2, __hip_atomic_load(rows + p * 128, __ATOMIC_RELAXED,
+                                                                       __HIP_MEMORY_SCOPE_AGENT));
+    };
+    float mx = -INFINITY, sum = 0.f;
+    for (int p = 0; p < S; ++p) mx = fmaxf(mx, row_of(p)[0]);
+    f32x16 acc[D1 - D0];
+#pragma unroll
+    for (int i = 0; i < D1 - D0; ++i) acc[i] = zero16();
+    for (int p = 0; p < S; ++p) {
+        const f32x2 ml = row_of(p);
+        const float wt = ml[0] == -INFINITY ? 0.f : exp2_fast(ml[0] - mx);
+        sum = fmaf(ml[1], wt, sum);
+        const uint64_t *slot = pairs + int64_t(p) * N * NT;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            // (The own slot is read as well, and not used.)
+            const f32x2 x = __builtin_bit_cast(
+                f32x2, __hip_atomic_load(slot + i * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            const f32x16 &t = o[D0 + i / 8];
+            f32x16 &c = acc[i / 8];
+            c[2 * (i & 7)] = fmaf(wt, p == part ? t[2 * (i & 7)] : x[0], c[2 * (i & 7)]);
+            c[2 * (i & 7) + 1] = fmaf(wt, p == part ? t[2 * (i & 7) + 1] : x[1], c[2 * (i & 7) + 1]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < D1 - D0; ++i) o[D0 + i] = acc[i];
+    m = mx;
+    l = sum;
+    return true;
 }
 
 // Copies of K / V block nb into an LDS tile by all NT threads.  A block that
@@ -272,19 +350,32 @@ struct KvLoader {
 // a score costs half the MFMA work of head_dim 128 for the same reads of V;
 // measured 3-6 % faster at seqlen 8192); two workgroups of 256 queries per
 // CU.  The per-tile arithmetic is the same, so the results are the same bits.
-template <int HD, bool CAUSAL, int QT>
-__global__ __launch_bounds__(256, QT == 2 || HD == 128 ? 2 : 3) void fwd_kernel(const fa_fwd_args a,
-                                                                                const int num_m_blocks, const int lg) {
-    constexpr int NT = 256;
+// NG = 2: two groups of 4 waves over the same rows take the key blocks in turn,
+// each through its own LDS stages, and merge their results through LDS at the
+// end.  SPLIT: S workgroups per query block do the same and merge through
+// split_ws.  A block's place in that order depends on its key position alone.
+template <int HD, bool CAUSAL, int QT, int NG, bool SPLIT>
+__global__ __launch_bounds__(256 * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 2 : 3) void fwd_kernel(
+    const fa_fwd_args a, const int num_m_blocks, const int lg, const int S) {
+    constexpr int NT = 256;  // threads of a wave group
+    static_assert(QT == 1 || NG == 1, "two groups: one tile per wave");
+    static_assert(NG == 2 || !SPLIT, "splits: two groups");
     using C = FwdCfg<HD, NT>;
     constexpr int BM = C::BM * QT, BN = C::BN;
-    __shared__ __attribute__((aligned(16))) char smem[2 * C::STAGE];
+    __shared__ __attribute__((aligned(16))) char smem[NG * 2 * C::STAGE];
+    __shared__ int ticket;
 
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
+    const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
+    const int wave = NG == 1 ? wave8 : wave8 & 3, grp = NG == 1 ? 0 : wave8 >> 2;
+    const int g0 = grp * 2 * C::STAGE;  // the group's LDS stages
     const int hh = lane >> 5;
     FwdWork w;
-    if (!fwd_work<BM, CAUSAL>(a, num_m_blocks, lg, w)) return;
+    const int bp_count = a.batch * (a.nheads >> lg);
+    const int unit = SPLIT ? blockIdx.x / bp_count : 0;  // SPLIT: the S shares of a block of positions in turn
+    const int part = SPLIT ? unit % S : 0;
+    const int bid = SPLIT ? unit / S * bp_count + (blockIdx.x - unit * bp_count) : blockIdx.x;
+    if (!fwd_work<BM, CAUSAL>(a, num_m_blocks, lg, bid, w)) return;
 
     // The wave's tiles QT * wave + t: one head (the launcher packs at most BM / 64 heads when QT = 2,
     // so a head spans at least 64 positions).
@@ -309,26 +400,30 @@ __global__ __launch_bounds__(256, QT == 2 || HD == 128 ? 2 : 3) void fwd_kernel(
     rd.init(lane);
     KvLoader<HD, NT> ld;
     ld.init(a, wave, lane);
+    const int part_step = SPLIT ? S : 1, step = NG * part_step;  // of the workgroup's blocks and of the group's
+    const int nb0 = part + part_step * grp;                      // the group's first block
     auto issue = [&](int nb, int st) FA_INLINE {
-        ld.k(a, w, smem, st * C::STAGE, nb, wave, lane);
-        ld.v(a, w, smem, st * C::STAGE + C::TILE, nb, wave, lane);
+        ld.k(a, w, smem, g0 + st * C::STAGE, nb, wave, lane);
+        ld.v(a, w, smem, g0 + st * C::STAGE + C::TILE, nb, wave, lane);
     };
 
     // One key block: S^T = K Q^T, online softmax, O^T += V^T P^T.  MASK is a
     // compile-time switch so the blocks away from the causal diagonal and
     // the sequence end carry no masking work at all.  A tile with no visible
     // key in a block it shares with the wave's other tile gets P = 0 there
-    // (its O, sums and maximum unchanged).
-    auto block = [&](int nb, auto mask_tag) FA_INLINE {
+    // (its O, sums and maximum unchanged).  The workgroup takes key blocks
+    // part, part + S, ... and each of its groups every NG-th of them.
+    auto block = [&](int it, auto mask_tag) FA_INLINE {
         constexpr bool MASK = decltype(mask_tag)::value;
-        const int buf = nb & 1;
+        const int buf = it & 1, nb = it * step + nb0;
         wait_vmem();
         __syncthreads();  // block nb is in LDS; every wave is done with stage buf ^ 1
-        if (nb + 1 < w.n_blocks) issue(nb + 1, buf ^ 1);
+        if (nb + step < w.n_blocks) issue(nb + step, buf ^ 1);
+        if (NG > 1 && nb >= w.n_blocks) return;
         const int n0 = nb * BN;
         if (CAUSAL && MASK && n0 > q_lo + 32 * QT - 1 + w.causal_off) return;  // no visible key for this wave
         if (q_lo >= w.sq) return;                                               // no query row of the sequence
-        const char *ks = smem + buf * C::STAGE;
+        const char *ks = smem + g0 + buf * C::STAGE;
         const char *vs = ks + C::TILE;
         f32x16 s[QT][2];
         f16x8 pB[QT][4];
@@ -400,11 +495,60 @@ __global__ __launch_bounds__(256, QT == 2 || HD == 128 ? 2 : 3) void fwd_kernel(
     // is below the sequence end and at or below the diagonal of the first query.
     int n_full = min(w.n_blocks, w.sk / BN);
     if (CAUSAL) n_full = min(n_full, max(0, (w.m0 + w.causal_off + 1) / BN));
-    if (w.n_blocks > 0) issue(0, 0);
-    for (int nb = 0; nb < n_full; ++nb) block(nb, std::false_type{});
-    for (int nb = n_full; nb < w.n_blocks; ++nb) block(nb, std::true_type{});
+    // Iterations in which every group has a block, and one without a mask.
+    const int last0 = nb0 - part_step * grp + part_step * (NG - 1);  // the last group's first block
+    if (nb0 < w.n_blocks) issue(nb0, 0);
+    const int it_full = n_full > last0 ? (n_full - 1 - last0) / step + 1 : 0;
+    const int n_it = w.n_blocks > part ? (w.n_blocks - 1 - part) / step + 1 : 0;
+    for (int it = 0; it < it_full; ++it) block(it, std::false_type{});
+    for (int it = it_full; it < n_it; ++it) block(it, std::true_type{});
+    if constexpr (NG == 1) {
 #pragma unroll
-    for (int t = 0; t < QT; ++t) store_row<HD>(a, w, qi[t], hh, o[t], row[t]);
+        for (int t = 0; t < QT; ++t) store_row<HD, 0, HD / 32>(a, w, qi[t], hh, o[t], row[t].m_t, sum_xor32(row[t].l_p));
+    } else {
+        // Each group finishes half of the head's dimensions: it hands the other
+        // half of its O, and its maxima and sums, to the other group.
+        constexpr int H = HD / 64;  // 32-wide dimension tiles of a half
+        const int t4 = tid & 255, r = 32 * wave + (lane & 31);
+        const float l_own = sum_xor32(row[0].l_p), m_own = row[0].m_t;
+        f32x4 *xo = reinterpret_cast<f32x4 *>(smem);                          // [group][4 H][256 threads]
+        f32x2 *xr = reinterpret_cast<f32x2 *>(smem + 2 * 4 * H * 256 * 16);   // [group][128 rows]
+        __syncthreads();  // every wave is done with the tiles
+        if (hh == 0) xr[grp * 128 + r] = f32x2{m_own, l_own};
+        auto finish = [&](auto grp_tag) FA_INLINE {
+            constexpr int GRP = decltype(grp_tag)::value;
+#pragma unroll
+            for (int i = 0; i < 4 * H; ++i) {
+                const f32x16 &t = o[0][(1 - GRP) * H + i / 4];
+                xo[(GRP * 4 * H + i) * 256 + t4] = f32x4{t[4 * (i & 3)], t[4 * (i & 3) + 1], t[4 * (i & 3) + 2],
+                                                         t[4 * (i & 3) + 3]};
+            }
+            __syncthreads();
+            const f32x2 other = xr[(1 - GRP) * 128 + r];
+            float m = fmaxf(m_own, other[0]);
+            const float a_own = m_own == -INFINITY ? 0.f : exp2_fast(m_own - m);
+            const float a_other = other[0] == -INFINITY ? 0.f : exp2_fast(other[0] - m);
+#pragma unroll
+            for (int i = 0; i < 4 * H; ++i) {
+                const f32x4 x = xo[((1 - GRP) * 4 * H + i) * 256 + t4];
+                f32x16 &t = o[0][GRP * H + i / 4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) t[4 * (i & 3) + e] = fmaf(x[e], a_other, t[4 * (i & 3) + e] * a_own);
+            }
+            // In group order, so that both groups have the same bits.
+            float l = GRP == 0 ? fmaf(other[1], a_other, l_own * a_own) : fmaf(l_own, a_own, other[1] * a_other);
+            if constexpr (SPLIT) {
+                const int item = (w.b * (a.nheads >> lg) + (w.h >> lg)) * num_m_blocks + w.m0 / w.P;
+                if (!fwd_merge<HD, GRP * H, GRP * H + H>(a, num_m_blocks * bp_count, item, part, S, r, &ticket, o[0], m, l))
+                    return;
+            }
+            store_row<HD, GRP * H, GRP * H + H>(a, w, qi[0], hh, o[0], m, l);
+        };
+        if (grp == 0)
+            finish(std::integral_constant<int, 0>{});
+        else
+            finish(std::integral_constant<int, 1>{});
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -431,7 +575,7 @@ __global__ __launch_bounds__(512, 1) void fwd_pp_kernel(const fa_fwd_args a, con
     const int grp = wave >> 2;                                  // 0: matrix phase first
     const int hh = lane >> 5;
     FwdWork w;
-    if (!fwd_work<BM, CAUSAL>(a, num_m_blocks, lg, w)) return;
+    if (!fwd_work<BM, CAUSAL>(a, num_m_blocks, lg, blockIdx.x, w)) return;
 
     const int q_lo = fwd_wave(a, w, 2 * (wave & 3) + grp);
     const int qi = q_lo + (lane & 31);
@@ -575,7 +719,7 @@ __global__ __launch_bounds__(512, 1) void fwd_pp_kernel(const fa_fwd_args a, con
         top(j);
         mid();
     }
-    store_row<HD>(a, w, qi, hh, o, row);
+    store_row<HD, 0, HD / 32>(a, w, qi, hh, o, row.m_t, sum_xor32(row.l_p));
 }
 
 // Varlen work order (order_items in fa_common.h): item it = b * nmb + mb is
@@ -613,6 +757,59 @@ static int fwd_pack_log2(const fa_fwd_args &a, int BM) {
     return lg;
 }
 
+// How the 128-row kernel runs: wave groups per workgroup and workgroups (splits)
+// per query block.  W: 128-row blocks (counted in 32-row tiles, so that a GQA
+// group packed into workgroups and its expanded heads get the same plan and
+// bits), NB: key blocks of the longest row.  Measured on MI355X, us at one group
+// and split -> as planned (groups x splits), head_dim 128 unless noted:
+//   one workgroup per CU leaves each SIMD one wave; a second group halves the
+//   chain of key blocks (1.82 us for a pair of blocks against 2 x 1.22):
+//     b1 s1024 32/8 causal (W 256): 26.9 -> 23.5 (2 x 1)   s509: 16.7 -> 15.7 (2 x 1)
+//     b1 s4096 16/16 causal (W 512): 104 -> 89 (2 x 1)     s2048 16/16: 45.7 -> 38.3 (2 x 1)
+//     1024 rows x 16384 keys 32/8 (W 256): 328 -> 294 (2 x 1)
+//   it loses when two workgroups per CU fill the chip without a mask (W 512,
+//   s4096: 153 -> 159), on short chains (W 256, s256: 11.8 -> 12.7) and past W 512
+//   (W 768, s2048: 74.5 -> 82);
+//   with idle CUs, splits take the rest (one launch to clear the counters and a
+//   merge: about 8 us, 2 more per split; a block pair takes 1.84 us, 1.31 at 64):
+//     512 rows x 16384 keys 32/8: 311 -> 160 (2 x 2)       128 rows: 309 -> 60 (2 x 8)
+//     b1 s2048 8/8 causal: 45.3 -> 30.2 (2 x 2)            512 x 8192 16/4 d64: 127 -> 38 (2 x 4)
+struct FwdPlan {
+    int groups, splits;
+};
+static FwdPlan fwd_plan(const fa_fwd_args &a) {
+    const int64_t W = (int64_t(a.batch) * a.nheads * ((int64_t(a.lse_seqlen) + 31) / 32) + 3) / 4, cus = device_cus();
+    const int NB = (a.seqlen_k + kFwdBN - 1) / kFwdBN;
+    FwdPlan plan = {1, 1};
+    if (2 * W <= cus ? NB >= 8 : W <= cus ? NB >= 12 : W <= 2 * cus && a.causal && NB >= 32) plan.groups = 2;
+    if (plan.groups == 1 || 2 * W > cus || a.cu_seqlens_q) return plan;
+    const double pairs = 0.5 * NB, unit = a.head_dim == 128 ? 1.84 : 1.31;
+    double best = pairs * unit;
+    for (int S = 2; S <= 16 && W * S <= cus; ++S) {
+        const double t = pairs / S * unit + 6 + 2 * S;
+        if (t < best) {
+            best = t;
+            plan.splits = S;
+        }
+    }
+    return plan;
+}
+// Workgroups of the unsplit 128-row grid.
+static int64_t fwd_items(const fa_fwd_args &a) {
+    const int lg = fwd_pack_log2(a, 128), P = 128 >> lg;
+    return int64_t((a.lse_seqlen + P - 1) / P) * a.batch * (a.nheads >> lg);
+}
+static size_t fwd_split_bytes(const fa_fwd_args &a, int S) {
+    const int64_t items = fwd_items(a);
+    return S > 1 ? size_t(fwd_count_bytes(items) + items * S * 128 * (8 + 4 * int64_t(a.head_dim))) : 0;
+}
+
+// Clears the splits' counters before fwd_kernel.
+__global__ void zero_counts_kernel(int32_t *count, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) count[i] = 0;
+}
+
 template <int HD, bool CAUSAL>
 static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
     // The ping-pong kernel when its grid fills the chip at least twice over
@@ -648,8 +845,8 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
             if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
             const int rc = launch_order(a, int(m_blocks), P, stream);
             if (rc) return rc;
-            hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 2>), dim3(unsigned(grid)), dim3(256), 0, stream, a,
-                               int(m_blocks), lg);
+            hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 2, 1, false>), dim3(unsigned(grid)), dim3(256), 0, stream, a,
+                               int(m_blocks), lg, 1);
             return int(hipGetLastError());
         }
     }
@@ -661,7 +858,25 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
     if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
     const int rc = launch_order(a, num_m_blocks, P, stream);
     if (rc) return rc;
-    hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 1>), dim3(unsigned(grid)), dim3(256), 0, stream, a, num_m_blocks, lg);
+    const FwdPlan plan = fwd_plan(a);
+    const int S = a.split_ws && a.split_ws_bytes >= int64_t(fwd_split_bytes(a, plan.splits)) ? plan.splits : 1;
+    if (S > 1) {
+        hipLaunchKernelGGL(zero_counts_kernel, dim3(unsigned((2 * grid + 255) / 256)), dim3(256), 0, stream,
+                           reinterpret_cast<int32_t *>(a.split_ws), int(2 * grid));
+        const int rc2 = int(hipGetLastError());
+        if (rc2) return rc2;
+    }
+    auto go = [&](auto ng_tag, auto split_tag) {
+        constexpr int NG = decltype(ng_tag)::value;
+        hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 1, NG, decltype(split_tag)::value>), dim3(unsigned(grid * S)),
+                           dim3(256 * NG), 0, stream, a, num_m_blocks, lg, S);
+    };
+    using G1 = std::integral_constant<int, 1>;
+    using G2 = std::integral_constant<int, 2>;
+    if (S > 1)
+        go(G2{}, std::true_type{});
+    else
+        plan.groups == 2 ? go(G2{}, std::false_type{}) : go(G1{}, std::false_type{});
     return int(hipGetLastError());
 }
 
@@ -681,6 +896,13 @@ extern "C" int fa_fwd(const fa_fwd_args *args, void *stream) {
     if (a.head_dim == 128)
         return a.causal ? fa::launch_fwd<128, true>(a, s) : fa::launch_fwd<128, false>(a, s);
     return a.causal ? fa::launch_fwd<64, true>(a, s) : fa::launch_fwd<64, false>(a, s);
+}
+
+extern "C" size_t fa_fwd_split_bytes(const fa_fwd_args *a) {
+    if (!a || a->batch <= 0 || a->seqlen_q <= 0 || a->seqlen_k <= 0 || a->nheads <= 0 || a->nheads_k <= 0 ||
+        (a->head_dim != 64 && a->head_dim != 128))
+        return 0;
+    return fa::fwd_split_bytes(*a, fa::fwd_plan(*a).splits);
 }
 
 extern "C" size_t fa_fwd_order_len(const fa_fwd_args *a) {

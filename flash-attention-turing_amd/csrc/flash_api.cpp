@@ -101,10 +101,10 @@ int num_cus(int device) {
     return n;
 }
 
-// The workspace in which workgroups that share a key block sum their dK / dV
-// (undefined when the grid needs no sharing).
-at::Tensor split_workspace(fa_bwd_args &a, const at::Tensor &like) {
-    const size_t bytes = fa_bwd_split_bytes(&a);
+// The workspace in which workgroups that share a query or key block sum their
+// results (undefined when the grid needs no sharing).
+template <class Args>
+at::Tensor split_workspace(Args &a, size_t bytes, const at::Tensor &like) {
     if (bytes == 0) return at::Tensor();
     at::Tensor ws = at::empty({int64_t(bytes)}, like.options().dtype(at::kByte));
     a.split_ws = ws.data_ptr();
@@ -150,6 +150,7 @@ std::vector<at::Tensor> mha_fwd(at::Tensor q, at::Tensor k, at::Tensor v, const 
     a.lse_seqlen = i32(seqlen_q, "seqlen_q");
     a.softmax_scale = softmax_scale;
     a.causal = is_causal ? 1 : 0;
+    at::Tensor split_ws = split_workspace(a, fa_fwd_split_bytes(&a), q);
     check_rc(fa_fwd(&a, current_stream()), "fa_fwd");
     return {o, l};
 }
@@ -203,7 +204,7 @@ std::vector<at::Tensor> mha_bwd(at::Tensor q, at::Tensor k, at::Tensor v, at::Te
     a.lse_seqlen = i32(seqlen_q, "seqlen_q");
     a.softmax_scale = softmax_scale;
     a.causal = is_causal ? 1 : 0;
-    at::Tensor split_ws = split_workspace(a, q);
+    at::Tensor split_ws = split_workspace(a, fa_bwd_split_bytes(&a), q);
     check_rc(fa_bwd(&a, current_stream()), "fa_bwd");
     for (auto *g : {&dq, &dk, &dv}) g->finish();
     return {dq.dst, dk.dst, dv.dst};
@@ -332,7 +333,7 @@ std::vector<at::Tensor> mha_varlen_bwd(at::Tensor q, at::Tensor k, at::Tensor v,
     // dQ and dK/dV work items ordered longest first on the device (sequences of mixed lengths).
     at::Tensor work_order = at::empty({int64_t(std::max<size_t>(fa_bwd_order_len(&a), 1))}, cu_seqlens_k.options());
     a.work_order = work_order.data_ptr<int32_t>();
-    at::Tensor split_ws = split_workspace(a, q);
+    at::Tensor split_ws = split_workspace(a, fa_bwd_split_bytes(&a), q);
     check_rc(fa_bwd(&a, current_stream()), "fa_bwd (varlen)");
     for (auto *g : {&dq, &dk, &dv}) g->finish();
     return {dq.dst, dk.dst, dv.dst};
@@ -610,6 +611,7 @@ std::vector<at::Tensor> mha_fwd_kvcache(at::Tensor q, at::Tensor k_cache, at::Te
     f.causal = is_causal ? 1 : 0;
     f.k_batch = i32(batch_size_cache, "cache batch size");
     f.status = status;
+    at::Tensor split_ws = split_workspace(f, fa_fwd_split_bytes(&f), q);
     check_rc(fa_fwd(&f, stream), "fa_fwd (kv-cache chunk)");
     return {out, lse};
 }

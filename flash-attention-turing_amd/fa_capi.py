@@ -44,7 +44,7 @@ class FaFwdArgs(ctypes.Structure):
         ("seqused_k_add", _i32),
         ("batch", _i32), ("seqlen_q", _i32), ("seqlen_k", _i32), ("nheads", _i32), ("nheads_k", _i32),
         ("head_dim", _i32), ("lse_seqlen", _i32), ("softmax_scale", _f32), ("causal", _i32),
-        ("k_batch", _i32), ("status", _p), ("work_order", _p),
+        ("k_batch", _i32), ("status", _p), ("work_order", _p), ("split_ws", _p), ("split_ws_bytes", _i64),
     ]
 
 
@@ -89,7 +89,7 @@ _ARGP = {
 }
 
 # FA_ABI_VERSION of include/fa_mi355x.h whose struct layouts the classes above mirror.
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 _lib = None
 
@@ -120,6 +120,8 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
     lib.fa_fwd_order_len.restype = ctypes.c_size_t
     lib.fa_bwd_order_len.argtypes = [ctypes.POINTER(FaBwdArgs)]
     lib.fa_bwd_order_len.restype = ctypes.c_size_t
+    lib.fa_fwd_split_bytes.argtypes = [ctypes.POINTER(FaFwdArgs)]
+    lib.fa_fwd_split_bytes.restype = ctypes.c_size_t
     lib.fa_bwd_split_bytes.argtypes = [ctypes.POINTER(FaBwdArgs)]
     lib.fa_bwd_split_bytes.restype = ctypes.c_size_t
     lib.fa_error_string.argtypes = [ctypes.c_int]

@@ -74,11 +74,21 @@ typedef struct fa_fwd_args {
      * the device, most work first, and launches the workgroups in that order;
      * NULL keeps the natural order.  Results are the same either way. */
     int32_t *work_order;
+    /* Optional workspace of split_ws_bytes >= fa_fwd_split_bytes(args) bytes,
+     * 256-byte aligned, when that is not 0: the grid of query blocks is too small
+     * for the chip, and several workgroups then share each block's keys and sum
+     * their fp32 partial results in it.  NULL (or a smaller one): one each. */
+    void *split_ws;
+    int64_t split_ws_bytes;
 } fa_fwd_args;
 
 /* Length in int32s of fa_fwd's work_order workspace: batch * ceil(lse_seqlen / 32).
  * No counterpart in the reference (its grid is in natural order). */
 size_t fa_fwd_order_len(const fa_fwd_args *args);
+/* Bytes of fa_fwd's split_ws workspace, 0 when the grid fills the chip by itself.
+ * It depends on the sizes, head counts, head_dim and causal alone.  No counterpart
+ * in the reference. */
+size_t fa_fwd_split_bytes(const fa_fwd_args *args);
 int fa_fwd(const fa_fwd_args *args, void *stream);
 
 /*
@@ -252,13 +262,13 @@ const char *fa_error_string(int code);
 /*
  * Version of the argument-struct layouts above.  It changes whenever a struct
  * gains, loses or moves a field (4: fa_bwd_args.split_ws and split_ws_bytes
- * appended).  A caller compiled against this
+ * appended; 5: the same for fa_fwd_args).  A caller compiled against this
  * header checks fa_abi_version() == FA_ABI_VERSION once after loading the
  * library and refuses a mismatch: the entry points themselves cannot tell a
  * shorter struct from an older caller.  No counterpart in the reference (its
  * bindings are compiled together with its kernels).
  */
-#define FA_ABI_VERSION 4
+#define FA_ABI_VERSION 5
 int fa_abi_version(void);
 
 #ifdef __cplusplus
