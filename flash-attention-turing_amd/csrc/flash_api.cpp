@@ -349,12 +349,15 @@ std::vector<at::Tensor> mha_fwd_kvcache(at::Tensor q, at::Tensor k_cache, at::Te
                                         std::optional<at::Tensor> alibi_slopes, std::optional<at::Tensor> out_opt,
                                         const float softmax_scale, bool is_causal, int window_size_left,
                                         int window_size_right, const float softcap, bool rotary_interleaved,
-                                        int num_splits, std::optional<at::Tensor> status_opt) {
+                                        int num_splits, std::optional<at::Tensor> status_opt,
+                                        bool lengths_checked) {
     // Order and texts follow flash_api.cpp:530-628.  status (optional, after
     // the reference's arguments): an int32 device word; when given, the cache
     // capacity and cache_batch_idx bounds are checked on the device instead of
     // by host reads (no synchronisation, so the call can be graph-captured):
     // 1 (capacity) / 2 (cache row) are ORed into it for the caller to report.
+    // lengths_checked (likewise): the caller has read cache_seqlens and checked
+    // the capacity, so it is not read (and waited for) a second time.
     TORCH_CHECK(!out_opt.has_value(), "Turing KV-cache does not support a preallocated output tensor yet");
     // Rotary embeddings, local windows, softcap, ALiBi and cache_leftpad
     // (rejected by the reference, flash_api.cpp:530-539) take upstream
@@ -443,9 +446,9 @@ std::vector<at::Tensor> mha_fwd_kvcache(at::Tensor q, at::Tensor k_cache, at::Te
                     "status must be a contiguous int32 tensor on the device of q");
         status = st.data_ptr<int32_t>();
     }
-    // Without a status word, the reference's host-visible checks (two
-    // device-to-host reads); the kernels bound every access either way.
-    if (!status && batch_size > 0) {
+    // Without a status word, the reference's host-visible checks (device-to-host
+    // reads); the kernels bound every access either way.
+    if (!status && !lengths_checked && batch_size > 0) {
         const int64_t max_end = cache_seqlens.max().item<int>() + seqlen_new;
         TORCH_CHECK(max_end <= seqlen_cache, "cache capacity is insufficient for the requested append length");
     }
@@ -638,5 +641,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("rotary_sin"), py::arg("cache_batch_idx"), py::arg("cache_leftpad"), py::arg("block_table"),
           py::arg("alibi_slopes"), py::arg("out"), py::arg("softmax_scale"), py::arg("is_causal"),
           py::arg("window_size_left"), py::arg("window_size_right"), py::arg("softcap"),
-          py::arg("rotary_interleaved"), py::arg("num_splits"), py::arg("status") = py::none());
+          py::arg("rotary_interleaved"), py::arg("num_splits"), py::arg("status") = py::none(),
+          py::arg("lengths_checked") = false);
 }
