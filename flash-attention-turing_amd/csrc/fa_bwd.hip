@@ -346,7 +346,16 @@ struct DkvCfg {
 // keys the block's last position sees (causal: min(sk, P (mb + 1) + sk - sq),
 // else sk), in 64-key buckets.  The list of the dK/dV items comes first in
 // work_order, that of the dQ items after it (fa_bwd_order_len).
-__global__ __launch_bounds__(kOrderThreads) void bwd_order_kernel(const fa_bwd_args a, const int nnb) {
+// Workgroups past the first zero the gradient rows of no sequence (order_wgs is
+// 0 without a work_order).
+__global__ __launch_bounds__(kOrderThreads) void bwd_order_kernel(const fa_bwd_args a, const int nnb,
+                                                                  const int order_wgs) {
+    if (int(blockIdx.x) >= order_wgs) {
+        for (const fa_tensor *t : {&a.dk, &a.dv})
+            zero_gaps(*t, a.cu_seqlens_k, a.batch, a.seqlen_k, a.dkv_rows, a.nheads_k, a.head_dim,
+                      blockIdx.x - order_wgs, gridDim.x - order_wgs);
+        return;
+    }
     order_items(a.batch * nnb, [&](int it) {
         const int b = it / nnb, nb = it - b * nnb;
         const int sk = a.cu_seqlens_k[b + 1] - a.cu_seqlens_k[b];
@@ -359,7 +368,12 @@ __global__ __launch_bounds__(kOrderThreads) void bwd_order_kernel(const fa_bwd_a
 }
 
 __global__ __launch_bounds__(kOrderThreads) void dq_order_kernel(const fa_bwd_args a, const int nnb, const int nmb,
-                                                                 const int P) {
+                                                                 const int P, const int order_wgs) {
+    if (int(blockIdx.x) >= order_wgs) {
+        zero_gaps(a.dq, a.cu_seqlens_q, a.batch, a.lse_seqlen, a.dq_rows, a.nheads, a.head_dim, blockIdx.x - order_wgs,
+                  gridDim.x - order_wgs);
+        return;
+    }
     order_items(a.batch * nmb, [&](int it) {
         const int b = it / nmb, mb = it - b * nmb;
         const int sq = a.cu_seqlens_q[b + 1] - a.cu_seqlens_q[b];
@@ -797,14 +811,15 @@ static int launch_dq(const fa_bwd_args &a, hipStream_t s) {
     const int P = DqCfg<HD>::BM >> lg;
     const int nmb = (a.lse_seqlen + P - 1) / P;
     const int64_t grid = int64_t(nmb) * a.batch * (a.nheads >> lg);
-    if (grid == 0) return FA_OK;
     if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
-    if (a.work_order && a.cu_seqlens_q) {
-        const int nnb = (a.seqlen_k + 127) / 128;
-        hipLaunchKernelGGL(dq_order_kernel, dim3(1), dim3(kOrderThreads), 0, s, a, nnb, nmb, P);
+    if (a.cu_seqlens_q && (a.work_order || a.dq_rows > 0)) {
+        const int nnb = (a.seqlen_k + 127) / 128, order_wgs = a.work_order ? 1 : 0;
+        hipLaunchKernelGGL(dq_order_kernel, dim3(order_wgs + (a.dq_rows > 0 ? kZeroBlocks : 0)), dim3(kOrderThreads), 0,
+                           s, a, nnb, nmb, P, order_wgs);
         const int rc = int(hipGetLastError());
         if (rc) return rc;
     }
+    if (grid == 0) return FA_OK;
     hipLaunchKernelGGL((bwd_dq_kernel<HD, CAUSAL>), dim3(unsigned(grid)), dim3(kBwdThreads), 0, s, a, nmb, lg);
     return int(hipGetLastError());
 }
@@ -868,13 +883,15 @@ static int launch_dkdv(const fa_bwd_args &a, hipStream_t s) {
     const int nnb = (a.seqlen_k + DkvCfg<HD>::BN - 1) / DkvCfg<HD>::BN;
     const int S = a.split_ws && a.split_ws_bytes >= int64_t(dkdv_ws_bytes(a, dkdv_splits(a))) ? dkdv_splits(a) : 1;
     const int64_t grid = int64_t(nnb) * a.batch * a.nheads_k * S;
-    if (grid == 0) return FA_OK;
     if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
-    if (a.work_order && a.cu_seqlens_k) {
-        hipLaunchKernelGGL(bwd_order_kernel, dim3(1), dim3(kOrderThreads), 0, s, a, nnb);
+    if (a.cu_seqlens_k && (a.work_order || a.dkv_rows > 0)) {
+        const int order_wgs = a.work_order ? 1 : 0;
+        hipLaunchKernelGGL(bwd_order_kernel, dim3(order_wgs + (a.dkv_rows > 0 ? kZeroBlocks : 0)), dim3(kOrderThreads),
+                           0, s, a, nnb, order_wgs);
         const int rc = int(hipGetLastError());
         if (rc) return rc;
     }
+    if (grid == 0) return FA_OK;
     if (S > 1)
         hipLaunchKernelGGL((bwd_dkdv_kernel<HD, CAUSAL, true>), dim3(unsigned(grid)), dim3(kDkvThreads), 0, s, a, nnb,
                            S);

@@ -726,7 +726,15 @@ __global__ __launch_bounds__(512, 1) void fwd_pp_kernel(const fa_fwd_args a, con
 // block mb of P query positions of sequence b, its work about positions x
 // keys seen by the block's last position, in buckets of P x 64; blocks past a
 // sequence's end come last (they still write LSE padding).
-__global__ __launch_bounds__(kOrderThreads) void fwd_order_kernel(const fa_fwd_args a, const int nmb, const int P) {
+// Workgroups past the first zero the output rows of no sequence (order_wgs is 0
+// without a work_order).
+__global__ __launch_bounds__(kOrderThreads) void fwd_order_kernel(const fa_fwd_args a, const int nmb, const int P,
+                                                                  const int order_wgs) {
+    if (int(blockIdx.x) >= order_wgs) {
+        zero_gaps(a.o, a.cu_seqlens_q, a.batch, a.lse_seqlen, a.o_rows, a.nheads, a.head_dim, blockIdx.x - order_wgs,
+                  gridDim.x - order_wgs);
+        return;
+    }
     order_items(a.batch * nmb, [&](int it) {
         const int b = it / nmb, mb = it - b * nmb;
         const int sq = a.cu_seqlens_q[b + 1] - a.cu_seqlens_q[b];
@@ -740,8 +748,10 @@ __global__ __launch_bounds__(kOrderThreads) void fwd_order_kernel(const fa_fwd_a
 }
 
 static int launch_order(const fa_fwd_args &a, int nmb, int P, hipStream_t stream) {
-    if (!a.work_order || !a.cu_seqlens_q) return FA_OK;
-    hipLaunchKernelGGL(fwd_order_kernel, dim3(1), dim3(kOrderThreads), 0, stream, a, nmb, P);
+    if (!a.cu_seqlens_q || (!a.work_order && a.o_rows <= 0)) return FA_OK;
+    const int order_wgs = a.work_order ? 1 : 0;
+    hipLaunchKernelGGL(fwd_order_kernel, dim3(order_wgs + (a.o_rows > 0 ? kZeroBlocks : 0)), dim3(kOrderThreads), 0,
+                       stream, a, nmb, P, order_wgs);
     return int(hipGetLastError());
 }
 
@@ -854,10 +864,9 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
     const int lg = fwd_pack_log2(a, BM), P = BM >> lg;
     const int num_m_blocks = (a.lse_seqlen + P - 1) / P;
     const int64_t grid = int64_t(num_m_blocks) * a.batch * (a.nheads >> lg);
-    if (grid == 0) return FA_OK;
     if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
     const int rc = launch_order(a, num_m_blocks, P, stream);
-    if (rc) return rc;
+    if (rc || grid == 0) return rc;
     const FwdPlan plan = fwd_plan(a);
     const int S = a.split_ws && a.split_ws_bytes >= int64_t(fwd_split_bytes(a, plan.splits)) ? plan.splits : 1;
     if (S > 1) {

@@ -52,25 +52,28 @@ inline at::Tensor aligned(const at::Tensor &t) { return is_aligned(t) ? t : t.cl
 // A gradient output: the caller's tensor (for instance one slice of a packed
 // dqkv) when it is given, written in place if its layout suits the kernels and
 // through a temporary copied into it otherwise; a new tensor when absent.
-// zero: rows no sequence covers (varlen padding) read 0 in a new tensor.
+// zero (varlen): rows no sequence covers read 0.  The kernels zero them (rest)
+// in a tensor that they write directly; a temporary starts as zeros.
 struct GradOut {
     at::Tensor dst, buf;
+    bool rest;
     void finish() {
         if (!buf.is_same(dst)) dst.copy_(buf);
     }
 };
-inline GradOut grad_out(const std::optional<at::Tensor> &given, const at::Tensor &like, bool zero,
+// varlen: in a caller's tensor they read 0 only with zero_given.
+inline GradOut grad_out(const std::optional<at::Tensor> &given, const at::Tensor &like, bool varlen, bool zero_given,
                         const char *name) {
-    auto fresh = [&] { return zero ? at::zeros(like.sizes(), like.options()) : at::empty(like.sizes(), like.options()); };
     if (!given.has_value()) {
-        at::Tensor t = fresh();
-        return {t, t};
+        at::Tensor t = at::empty(like.sizes(), like.options());
+        return {t, t, varlen};
     }
     const at::Tensor &g = *given;
     check_fp16_cuda(g, name);
     TORCH_CHECK(g.device() == like.device(), name, " must be on the device of its input");
     TORCH_CHECK(g.sizes() == like.sizes(), name, " must have the shape of its input");
-    return {g, is_aligned(g) ? g : fresh()};
+    if (is_aligned(g)) return {g, g, varlen && zero_given};
+    return {g, varlen ? at::zeros(like.sizes(), like.options()) : at::empty(like.sizes(), like.options()), false};
 }
 
 inline fa_tensor desc4(const at::Tensor &t) {  // [batch][row][head][d]
@@ -181,7 +184,8 @@ std::vector<at::Tensor> mha_bwd(at::Tensor q, at::Tensor k, at::Tensor v, at::Te
     out = aligned(out);
     dout = aligned(dout);
 
-    GradOut dq = grad_out(dq_, q, false, "dq"), dk = grad_out(dk_, k, false, "dk"), dv = grad_out(dv_, v, false, "dv");
+    GradOut dq = grad_out(dq_, q, false, false, "dq"), dk = grad_out(dk_, k, false, false, "dk"),
+            dv = grad_out(dv_, v, false, false, "dv");
     at::Tensor dsum = at::empty({2, l.numel()}, l.options());  // -D, then LSE*log2(e)
 
     fa_bwd_args a{};
@@ -249,8 +253,8 @@ std::vector<at::Tensor> mha_varlen_fwd(at::Tensor q, at::Tensor k, at::Tensor v,
     k = aligned(k);
     v = aligned(v);
 
-    // Packed rows past cu_seqlens_q[-1] belong to no sequence and stay 0.
-    at::Tensor out = at::zeros(q.sizes(), q.options());
+    // Packed rows past cu_seqlens_q[-1] belong to no sequence and read 0 (o_rows).
+    at::Tensor out = at::empty(q.sizes(), q.options());
     at::Tensor l = at::empty({batch_size, num_heads, max_seqlen_q}, q.options().dtype(at::kFloat));
 
     fa_fwd_args a{};
@@ -270,6 +274,7 @@ std::vector<at::Tensor> mha_varlen_fwd(at::Tensor q, at::Tensor k, at::Tensor v,
     a.lse_seqlen = max_seqlen_q;
     a.softmax_scale = softmax_scale;
     a.causal = is_causal ? 1 : 0;
+    a.o_rows = i32(q.size(0), "total_q");
     // Query blocks ordered most work first on the device (sequences of mixed lengths).
     at::Tensor work_order = at::empty({int64_t(std::max<size_t>(fa_fwd_order_len(&a), 1))}, cu_seqlens_q.options());
     a.work_order = work_order.data_ptr<int32_t>();
@@ -281,7 +286,7 @@ std::vector<at::Tensor> mha_varlen_bwd(at::Tensor q, at::Tensor k, at::Tensor v,
                                        at::Tensor dout, at::Tensor cu_seqlens_q, at::Tensor cu_seqlens_k,
                                        const int max_seqlen_q, const int max_seqlen_k, const float softmax_scale,
                                        bool is_causal, std::optional<at::Tensor> dq_, std::optional<at::Tensor> dk_,
-                                       std::optional<at::Tensor> dv_) {
+                                       std::optional<at::Tensor> dv_, bool zero_rest) {
     TORCH_CHECK(q.dim() == 3 && k.dim() == 3 && v.dim() == 3, "q, k, v must be rank-3 packed tensors");
     check_cu_seqlens(cu_seqlens_q, cu_seqlens_k);
     const int64_t batch_size = cu_seqlens_q.numel() - 1;
@@ -304,8 +309,14 @@ std::vector<at::Tensor> mha_varlen_bwd(at::Tensor q, at::Tensor k, at::Tensor v,
     dout = aligned(dout);
 
     // Packed rows past the last sequence belong to no sequence: 0 in a new
-    // gradient tensor, left as they are in a caller's.
-    GradOut dq = grad_out(dq_, q, true, "dq"), dk = grad_out(dk_, k, true, "dk"), dv = grad_out(dv_, v, true, "dv");
+    // gradient tensor, left as they are in a caller's (0 too with zero_rest).
+    GradOut dq = grad_out(dq_, q, true, zero_rest, "dq"), dk = grad_out(dk_, k, true, zero_rest, "dk"),
+            dv = grad_out(dv_, v, true, zero_rest, "dv");
+    if (dk.rest != dv.rest) {  // one flag for both in the kernels' arguments
+        if (dk.rest) dk.buf.zero_();
+        if (dv.rest) dv.buf.zero_();
+        dk.rest = dv.rest = false;
+    }
     at::Tensor dsum = at::empty({2, l.numel()}, l.options());  // -D, then LSE*log2(e)
 
     fa_bwd_args a{};
@@ -330,6 +341,8 @@ std::vector<at::Tensor> mha_varlen_bwd(at::Tensor q, at::Tensor k, at::Tensor v,
     a.lse_seqlen = max_seqlen_q;
     a.softmax_scale = softmax_scale;
     a.causal = is_causal ? 1 : 0;
+    a.dq_rows = dq.rest ? i32(q.size(0), "total_q") : 0;
+    a.dkv_rows = dk.rest ? i32(k.size(0), "total_k") : 0;
     // dQ and dK/dV work items ordered longest first on the device (sequences of mixed lengths).
     at::Tensor work_order = at::empty({int64_t(std::max<size_t>(fa_bwd_order_len(&a), 1))}, cu_seqlens_k.options());
     a.work_order = work_order.data_ptr<int32_t>();
@@ -635,7 +648,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("varlen_bwd", &mha_varlen_bwd, "Varlen backward pass", py::arg("q"), py::arg("k"), py::arg("v"),
           py::arg("out"), py::arg("l"), py::arg("dout"), py::arg("cu_seqlens_q"), py::arg("cu_seqlens_k"),
           py::arg("max_seqlen_q"), py::arg("max_seqlen_k"), py::arg("softmax_scale"), py::arg("is_causal"),
-          py::arg("dq") = py::none(), py::arg("dk") = py::none(), py::arg("dv") = py::none());
+          py::arg("dq") = py::none(), py::arg("dk") = py::none(), py::arg("dv") = py::none(),
+          py::arg("zero_rest") = false);
     m.def("fwd_kvcache", &mha_fwd_kvcache, "KV-cache forward pass", py::arg("q"), py::arg("k_cache"),
           py::arg("v_cache"), py::arg("k"), py::arg("v"), py::arg("cache_seqlens"), py::arg("rotary_cos"),
           py::arg("rotary_sin"), py::arg("cache_batch_idx"), py::arg("cache_leftpad"), py::arg("block_table"),

@@ -45,6 +45,7 @@ class FaFwdArgs(ctypes.Structure):
         ("batch", _i32), ("seqlen_q", _i32), ("seqlen_k", _i32), ("nheads", _i32), ("nheads_k", _i32),
         ("head_dim", _i32), ("lse_seqlen", _i32), ("softmax_scale", _f32), ("causal", _i32),
         ("k_batch", _i32), ("status", _p), ("work_order", _p), ("split_ws", _p), ("split_ws_bytes", _i64),
+        ("o_rows", _i32),
     ]
 
 
@@ -55,7 +56,7 @@ class FaBwdArgs(ctypes.Structure):
         ("lse", _p), ("dsum", _p), ("cu_seqlens_q", _p), ("cu_seqlens_k", _p),
         ("batch", _i32), ("seqlen_q", _i32), ("seqlen_k", _i32), ("nheads", _i32), ("nheads_k", _i32),
         ("head_dim", _i32), ("lse_seqlen", _i32), ("softmax_scale", _f32), ("causal", _i32),
-        ("work_order", _p), ("split_ws", _p), ("split_ws_bytes", _i64),
+        ("work_order", _p), ("split_ws", _p), ("split_ws_bytes", _i64), ("dq_rows", _i32), ("dkv_rows", _i32),
     ]
 
 
@@ -89,7 +90,7 @@ _ARGP = {
 }
 
 # FA_ABI_VERSION of include/fa_mi355x.h whose struct layouts the classes above mirror.
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 _lib = None
 

@@ -78,12 +78,14 @@ def _flash_attn_varlen_backward(
     dq=None,
     dk=None,
     dv=None,
+    zero_rest: bool = False,
 ):
-    """dq / dk / dv, when given, are written in place (rows no sequence covers are left as they are)."""
+    """dq / dk / dv, when given, are written in place (rows no sequence covers are left as they are, or
+    zeroed with zero_rest)."""
     dout, q, k, v, out, lse = (maybe_contiguous(t) for t in (dout, q, k, v, out, lse))
     dq, dk, dv = flash_attn_gpu.varlen_bwd(
         q, k, v, out, lse, dout, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal,
-        dq, dk, dv,
+        dq, dk, dv, zero_rest,
     )
     return dq, dk, dv
 
@@ -240,10 +242,10 @@ class FlashAttnVarlenQKVPackedFunc(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         q, k, v, out, lse, cu_seqlens = ctx.saved_tensors
-        dqkv, (dq, dk, dv) = _packed_grad(ctx.packed, 1, True)
+        dqkv, (dq, dk, dv) = _packed_grad(ctx.packed, 1, False)
         _flash_attn_varlen_backward(
             dout, q, k, v, out, lse, cu_seqlens, cu_seqlens, ctx.max_seqlen, ctx.max_seqlen,
-            ctx.softmax_scale, ctx.causal, dq, dk, dv,
+            ctx.softmax_scale, ctx.causal, dq, dk, dv, zero_rest=True,
         )
         return dqkv, None, None, None, None, None
 
@@ -267,10 +269,10 @@ class FlashAttnVarlenKVPackedFunc(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k = ctx.saved_tensors
-        dkv, (dk, dv) = _packed_grad(ctx.packed, 1, True)
+        dkv, (dk, dv) = _packed_grad(ctx.packed, 1, False)
         dq, _, _ = _flash_attn_varlen_backward(
             dout, q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k, ctx.max_seqlen_q, ctx.max_seqlen_k,
-            ctx.softmax_scale, ctx.causal, None, dk, dv,
+            ctx.softmax_scale, ctx.causal, None, dk, dv, zero_rest=True,
         )
         return dq, dkv, None, None, None, None, None, None, None
 

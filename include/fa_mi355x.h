@@ -80,6 +80,10 @@ typedef struct fa_fwd_args {
      * their fp32 partial results in it.  NULL (or a smaller one): one each. */
     void *split_ws;
     int64_t split_ws_bytes;
+    /* Rows of the packed o tensor (varlen calls), or 0.  When set, o's rows that no
+     * sequence covers (before cu_seqlens_q[0], from cu_seqlens_q[batch] on) are
+     * zeroed on the device; 0 leaves them as they are. */
+    int32_t o_rows;
 } fa_fwd_args;
 
 /* Length in int32s of fa_fwd's work_order workspace: batch * ceil(lse_seqlen / 32).
@@ -126,6 +130,9 @@ typedef struct fa_bwd_args {
      * NULL (or a smaller one) gives each key block to one workgroup. */
     void *split_ws;
     int64_t split_ws_bytes;
+    /* Rows of the packed dq and of the packed dk / dv, or 0, as fa_fwd_args.o_rows:
+     * fa_bwd_dq zeroes dq's rows of no sequence, fa_bwd_dkdv those of dk and dv. */
+    int32_t dq_rows, dkv_rows;
 } fa_bwd_args;
 
 /* Length in int32s of the work_order workspace: batch * (ceil(seqlen_k / 128) +
@@ -262,13 +269,14 @@ const char *fa_error_string(int code);
 /*
  * Version of the argument-struct layouts above.  It changes whenever a struct
  * gains, loses or moves a field (4: fa_bwd_args.split_ws and split_ws_bytes
- * appended; 5: the same for fa_fwd_args).  A caller compiled against this
+ * appended; 5: the same for fa_fwd_args; 6:
+ * fa_fwd_args.o_rows, fa_bwd_args.dq_rows and dkv_rows).  A caller compiled against this
  * header checks fa_abi_version() == FA_ABI_VERSION once after loading the
  * library and refuses a mismatch: the entry points themselves cannot tell a
  * shorter struct from an older caller.  No counterpart in the reference (its
  * bindings are compiled together with its kernels).
  */
-#define FA_ABI_VERSION 5
+#define FA_ABI_VERSION 6
 int fa_abi_version(void);
 
 #ifdef __cplusplus
