@@ -176,7 +176,8 @@ __device__ __forceinline__ void append_chunk(const fa_kvcache_args &a, const int
 // sequence with the r-th most keys, by a counting sort over key-count buckets
 // (exact below 32 keys, then 32 buckets per power of two: about 3 % apart;
 // order within a bucket is arbitrary, which changes no result), and zero the
-// split kernel's work counter batch_order[batch] and its n_count split counts.
+// split kernel's work counter batch_order[batch] and its n_count split counts
+// (the counts alone without rank).
 // The other workgroups append one 16-byte chunk per thread.  The two parts
 // touch disjoint memory (the ranking reads cache_seqlens only).
 __device__ __forceinline__ int kv_len_bucket(int n) {
@@ -186,10 +187,12 @@ __device__ __forceinline__ int kv_len_bucket(int n) {
 }
 template <int HD>
 __global__ __launch_bounds__(kOrderThreads) void kv_prep_kernel(const fa_kvcache_args a, const int order_wgs,
-                                                                int32_t *const count, const int n_count) {
+                                                                const bool rank, int32_t *const count,
+                                                                const int n_count) {
     if (int(blockIdx.x) < order_wgs) {
-        if (threadIdx.x == 0) a.batch_order[a.batch] = 0;
         for (int i = threadIdx.x; i < n_count; i += kOrderThreads) count[i] = 0;
+        if (!rank) return;
+        if (threadIdx.x == 0) a.batch_order[a.batch] = 0;
         order_items(
             a.batch,
             [&](int b) {
@@ -361,7 +364,12 @@ __device__ __forceinline__ float tanh_fast(float x) {
 // CU) and each workgroup, after its first item blockIdx.x, takes the next
 // unclaimed item from a device counter, so no workgroup is relaunched and
 // the items are dealt out greedily in that order.  The counter
-// (batch_order[batch]) is zeroed by kv_prep_kernel on the same stream.
+// (batch_order[batch]) is zeroed by kv_prep_kernel on the same stream; an item
+// that finds the whole list under way claims nothing.  With at most one item
+// per CU the sequences are taken as they come (ranked is false) and not ranked:
+// one sequence of 1500 tokens, 32 / 8 heads, 17.8 -> 15.7 us a call.  With two
+// per CU the order still pairs long items with short ones (64 sequences of 1.5k
+// - 3k tokens, 512 items: 117 us ranked, 122 not).
 // With count (num_splits > 1, DYN) the split kernel also combines: count[(b *
 // nheads_k + hk) * row_tiles + rt] (zeroed by kv_prep_kernel) counts the
 // finished splits of that row tile, and the item that finishes last combines
@@ -374,7 +382,8 @@ __device__ __forceinline__ float tanh_fast(float x) {
 // of a head-interleaved cache row, where one head alone reads 128 or 256.
 template <int HD, bool DYN, bool EXT, int HPI>
 __global__ __launch_bounds__(256, 2) void kv_splitkv_kernel(const fa_kvcache_args a, const int row_tiles,
-                                                            const int n_items, int32_t *const count) {
+                                                            const int n_items, int32_t *const count,
+                                                            const bool ranked) {
     using C = KvCfg<HD>;
     static_assert(HPI == 1 || HPI == 2 || HPI == 4, "heads per item");
     constexpr int WPH = kKvWaves / HPI;  // waves per head
@@ -395,7 +404,7 @@ __global__ __launch_bounds__(256, 2) void kv_splitkv_kernel(const fa_kvcache_arg
         rest /= n_groups;
         const int split = rest % a.num_splits;
         const int rank = rest / a.num_splits;
-        const int b = a.batch_order ? a.batch_order[rank] : rank;
+        const int b = DYN && ranked ? a.batch_order[rank] : rank;
         const int G = a.nheads / a.nheads_k;
         const int R = G * a.seqlen_q;  // rows of this (batch, kv head): row = qpos * G + g
 
@@ -738,7 +747,7 @@ __global__ __launch_bounds__(256, 2) void kv_splitkv_kernel(const fa_kvcache_arg
                     rows(I4{}, Pre{});
             }
         }
-        if constexpr (!DYN) break;
+        if (!DYN || n_items <= int(gridDim.x)) break;
         __syncthreads();  // every thread is done with this item's LDS
         if (tid == 0) next_item = atomicAdd(a.batch_order + a.batch, 1) + int(gridDim.x);
         __syncthreads();
@@ -838,7 +847,7 @@ __device__ __forceinline__ bool chunk_merge(const fa_kvcache_args &a, int32_t *c
 
 template <int HD, bool EXT>
 __global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcache_args a, const int row_tiles,
-                                                                 int32_t *const count) {
+                                                                 int32_t *const count, const bool ranked) {
     constexpr int BN = kChunkKeys, TILE = BN * HD * 2, STAGE = 2 * TILE;
     __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
     __shared__ int pages[kChunkPages];
@@ -860,7 +869,7 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcach
     const int hk = rest % a.nheads_k;
     rest /= a.nheads_k;
     const int split = rest % S;
-    const int b = a.batch_order[rest / S];
+    const int b = ranked ? a.batch_order[rest / S] : rest / S;
 
     const KvSeq sq = kv_seq(a, b);
     if (sq.err && a.status && tid == 0) atomicOr(a.status, sq.err);
@@ -1200,24 +1209,6 @@ int check_split(const fa_kvcache_args &a) {
 // with split counts and more than one split.
 bool fused_combine(const fa_kvcache_args &a) { return a.batch_order && a.split_count && a.num_splits > 1; }
 
-// kv_prep_kernel over the append's chunks (append) after one ordering workgroup (order).
-int launch_prep(const fa_kvcache_args &a, bool append, bool order, hipStream_t s) {
-    const int64_t chunks = append ? int64_t(a.batch) * a.seqlen_new * a.nheads_k * (a.head_dim / 8) : 0;
-    const int order_wgs = order ? 1 : 0;
-    const int64_t blocks = order_wgs + (chunks + kOrderThreads - 1) / kOrderThreads;
-    if (blocks == 0) return FA_OK;
-    if (blocks > 0x7fffffff) return FA_ERR_INVALID_ARG;
-    int32_t *count = order && fused_combine(a) ? a.split_count : nullptr;
-    const int n_count = count ? int(fa_kv_split_count_len(&a)) : 0;
-    if (a.head_dim == 128)
-        hipLaunchKernelGGL(kv_prep_kernel<128>, dim3(unsigned(blocks)), dim3(kOrderThreads), 0, s, a, order_wgs, count,
-                           n_count);
-    else
-        hipLaunchKernelGGL(kv_prep_kernel<64>, dim3(unsigned(blocks)), dim3(kOrderThreads), 0, s, a, order_wgs, count,
-                           n_count);
-    return int(hipGetLastError());
-}
-
 // KV heads per work item of the resident split kernel without options: in a
 // head-interleaved cache (head stride = head_dim) enough adjacent heads that
 // one key position's rows of an item are 512 contiguous bytes (HBM reads of
@@ -1250,14 +1241,45 @@ bool use_chunk(const fa_kvcache_args &a) {
     return !a.block_table || (a.page_block_size % kChunkKeys == 0 && a.cache_capacity > 0 &&
                               a.cache_capacity / a.page_block_size <= kChunkPages);
 }
+int64_t chunk_items(const fa_kvcache_args &a) {
+    const int row_tiles = ((a.nheads / a.nheads_k) * a.seqlen_q + kChunkRows - 1) / kChunkRows;
+    return int64_t(a.batch) * a.nheads_k * row_tiles * a.num_splits;
+}
+
+// Whether the split kernel's items come in the order of batch_order: there are
+// more of them than CUs.
+bool kv_ranked(const fa_kvcache_args &a) {
+    const int64_t n = use_chunk(a) ? chunk_items(a) : split_items(a) / kv_heads_per_item(a);
+    return a.batch_order && n > int64_t(device_cus());
+}
+
+// kv_prep_kernel over the append's chunks (append) after one ordering workgroup (order).
+int launch_prep(const fa_kvcache_args &a, bool append, bool order, hipStream_t s) {
+    const int64_t chunks = append ? int64_t(a.batch) * a.seqlen_new * a.nheads_k * (a.head_dim / 8) : 0;
+    int32_t *count = order && fused_combine(a) ? a.split_count : nullptr;
+    const int n_count = count ? int(fa_kv_split_count_len(&a)) : 0;
+    const bool rank = order && kv_ranked(a);
+    const int order_wgs = rank || count ? 1 : 0;
+    const int64_t blocks = order_wgs + (chunks + kOrderThreads - 1) / kOrderThreads;
+    if (blocks == 0) return FA_OK;
+    if (blocks > 0x7fffffff) return FA_ERR_INVALID_ARG;
+    if (a.head_dim == 128)
+        hipLaunchKernelGGL(kv_prep_kernel<128>, dim3(unsigned(blocks)), dim3(kOrderThreads), 0, s, a, order_wgs, rank, count,
+                           n_count);
+    else
+        hipLaunchKernelGGL(kv_prep_kernel<64>, dim3(unsigned(blocks)), dim3(kOrderThreads), 0, s, a, order_wgs, rank, count,
+                           n_count);
+    return int(hipGetLastError());
+}
+
 int launch_chunk(const fa_kvcache_args &a, hipStream_t s) {
     const int row_tiles = ((a.nheads / a.nheads_k) * a.seqlen_q + kChunkRows - 1) / kChunkRows;
-    const int64_t n = int64_t(a.batch) * a.nheads_k * row_tiles * a.num_splits;
+    const int64_t n = chunk_items(a);
     if (n == 0) return FA_OK;
-    const bool ext = a.local_window || a.softcap > 0.f || a.cache_leftpad || a.alibi_slopes || a.rotary_dim > 0;
+    const bool ranked = kv_ranked(a), ext = a.local_window || a.softcap > 0.f || a.cache_leftpad || a.alibi_slopes || a.rotary_dim > 0;
     auto go = [&](auto hd_tag, auto ext_tag) {
         hipLaunchKernelGGL((kv_chunk_kernel<decltype(hd_tag)::value, decltype(ext_tag)::value>), dim3(unsigned(n)),
-                           dim3(kKvThreads), 0, s, a, row_tiles, a.split_count);
+                           dim3(kKvThreads), 0, s, a, row_tiles, a.split_count, ranked);
     };
     using H128 = std::integral_constant<int, 128>;
     using H64 = std::integral_constant<int, 64>;
@@ -1281,12 +1303,13 @@ int launch_split(const fa_kvcache_args &a, hipStream_t s) {
     const bool dyn = a.batch_order != nullptr;
     const unsigned grid = unsigned(dyn ? std::min<int64_t>(gx, 2 * int64_t(device_cus())) : gx);
     int32_t *count = fused_combine(a) ? a.split_count : nullptr;
+    const bool ranked = kv_ranked(a);
     const bool ext = a.local_window || a.softcap > 0.f || a.cache_leftpad || a.alibi_slopes || a.rotary_dim > 0;
     auto go = [&](auto hd_tag, auto dyn_tag, auto ext_tag, auto hpi_tag) {
         constexpr int HD = decltype(hd_tag)::value, HPI = decltype(hpi_tag)::value;
         constexpr bool DYN = decltype(dyn_tag)::value, EXT = decltype(ext_tag)::value;
         hipLaunchKernelGGL((kv_splitkv_kernel<HD, DYN, EXT, HPI>), dim3(grid), dim3(kKvThreads), 0, s, a, row_tiles,
-                           n_items, count);
+                           n_items, count, ranked);
     };
     using H128 = std::integral_constant<int, 128>;
     using H64 = std::integral_constant<int, 64>;
