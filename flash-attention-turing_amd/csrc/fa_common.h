@@ -456,6 +456,16 @@ __device__ __forceinline__ void zero_gaps(const fa_tensor &t, const int32_t *cu,
 }
 constexpr int kZeroBlocks = 64;  // workgroups that zero gaps beside an order kernel's own
 
+// Place in a longest-first list of workgroup bid when all gridDim.x of them are
+// on the chip from the start, one layer of cus workgroups after another (cus is
+// 0 when they are not): every other layer is taken backwards, so that the CUs
+// with the longest items get the shortest ones beside them.
+__device__ __forceinline__ int paired_place(int bid, int n, int cus) {
+    if (cus == 0) return bid;
+    const int layer = bid / cus;
+    return layer & 1 ? layer * cus + min(n, (layer + 1) * cus) - 1 - bid : bid;
+}
+
 // Per-batch extents of a dense or packed (varlen) batch.
 struct SeqInfo {
     int q_start, sq, k_start, sk;

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import fa_capi
-from helpers import assert_2x, check_varlen, cu_from_lengths, randn16
+from helpers import assert_2x, check_fwd_bwd, check_varlen, cu_from_lengths, randn16
 from oracle.attention import attention_bwd, attention_fwd, bwd_fp32_noise
 from oracle.twin import bwd_twin, fwd_twin
 
@@ -116,3 +116,22 @@ def test_split_bytes_rule():
     assert size(1, 8192, 8192, 32, 8, 128, True) > 0
     for case in CASES + [(1, 1 << 20, 1 << 20, 8, 1, 128, True), (1, 16384, 16384, 32, 8, 128, True)]:
         assert size(*case) <= (256 << 20) + (1 << 20)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,sq,sk,h,hk,hd", [(3, 700, 700, 16, 16, 64), (3, 600, 777, 20, 20, 128)])
+def test_paired_items(device, b, sq, sk, h, hk, hd):
+    """Causal grids between one and two workgroups per CU, whose second layer is taken backwards (an odd number of
+    items in it): every query and key block once, against the oracle."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for blocks in ((sq + 127) // 128, (sk + 127) // 128):
+        assert cus < blocks * b * h <= 2 * cus and sk > 512, "the shape must select the pairing"
+    g = torch.Generator().manual_seed(8900 + sq + hd)
+    q, do = randn16((b, sq, h, hd), g), randn16((b, sq, h, hd), g)
+    k, v = randn16((b, sk, hk, hd), g), randn16((b, sk, hk, hd), g)
+    s = hd ** -0.5
+    print(f"case paired sq={sq} sk={sk} hd={hd}", flush=True)
+    ba, o, lse, grads = _args(*(t.to(device) for t in (q, k, v, do)), s, True)
+    fa_capi.call("fa_bwd", ba)
+    torch.cuda.synchronize()
+    check_fwd_bwd("paired", q, k, v, do, o.cpu(), lse.cpu(), tuple(t.cpu() for t in grads), s, True)
