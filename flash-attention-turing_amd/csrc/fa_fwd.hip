@@ -27,8 +27,8 @@
 //     VALU while the other group's MFMAs run on the matrix cores;
 //   * fwd_kernel (head_dim 64 and small grids): 4 waves, two (head_dim 128)
 //     or three (head_dim 64) independent workgroups per CU; on grids too small
-//     for that, two groups of 4 waves per workgroup and several workgroups per
-//     query block share the key blocks (fwd_plan).
+//     for that, two groups of 4 or 2 waves per workgroup, and several workgroups
+//     per query block, share the key blocks (fwd_plan).
 #include <type_traits>
 
 #include "fa_common.h"
@@ -350,24 +350,26 @@ struct KvLoader {
 // a score costs half the MFMA work of head_dim 128 for the same reads of V;
 // measured 3-6 % faster at seqlen 8192); two workgroups of 256 queries per
 // CU.  The per-tile arithmetic is the same, so the results are the same bits.
-// NG = 2: two groups of 4 waves over the same rows take the key blocks in turn,
-// each through its own LDS stages, and merge their results through LDS at the
-// end.  SPLIT: S workgroups per query block do the same and merge through
+// NG = 2: two groups of RW waves (RW = 4: 128 rows, 2: 64 rows) over the same rows
+// take the key blocks in turn, each through its own LDS stages, and merge their
+// results through LDS at the end.  SPLIT: S workgroups per query block do the same and merge through
 // split_ws.  A block's place in that order depends on its key position alone.
-template <int HD, bool CAUSAL, int QT, int NG, bool SPLIT>
-__global__ __launch_bounds__(256 * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 2 : 3) void fwd_kernel(
+template <int HD, bool CAUSAL, int QT, int NG, int RW, bool SPLIT>
+__global__ __launch_bounds__(64 * RW * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 2 : 3) void fwd_kernel(
     const fa_fwd_args a, const int num_m_blocks, const int lg, const int S) {
-    constexpr int NT = 256;  // threads of a wave group
+    constexpr int NT = 256;        // threads that copy a tile together
+    constexpr int GT = 64 * RW;    // threads of a wave group
     static_assert(QT == 1 || NG == 1, "two groups: one tile per wave");
     static_assert(NG == 2 || !SPLIT, "splits: two groups");
+    static_assert(RW == 4 || (RW == 2 && NG == 2 && !SPLIT), "two row waves: two groups, no splits");
     using C = FwdCfg<HD, NT>;
-    constexpr int BM = C::BM * QT, BN = C::BN;
+    constexpr int BM = 32 * RW * QT, BN = C::BN;
     __shared__ __attribute__((aligned(16))) char smem[NG * 2 * C::STAGE];
     __shared__ int ticket;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
-    const int wave = NG == 1 ? wave8 : wave8 & 3, grp = NG == 1 ? 0 : wave8 >> 2;
+    const int wave = NG == 1 ? wave8 : wave8 & (RW - 1), grp = NG == 1 ? 0 : wave8 / RW;
     const int g0 = grp * 2 * C::STAGE;  // the group's LDS stages
     const int hh = lane >> 5;
     FwdWork w;
@@ -399,12 +401,26 @@ __global__ __launch_bounds__(256 * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 2 : 
     TileReader<HD> rd;
     rd.init(lane);
     KvLoader<HD, NT> ld;
-    ld.init(a, wave, lane);
+    ld.init(a, RW == 4 ? wave : wave8, lane);
     const int part_step = SPLIT ? S : 1, step = NG * part_step;  // of the workgroup's blocks and of the group's
     const int nb0 = part + part_step * grp;                      // the group's first block
+    // Copies of the group's block nb into stage st; with two row waves a group,
+    // all four waves copy the blocks of both groups.
     auto issue = [&](int nb, int st) FA_INLINE {
-        ld.k(a, w, smem, g0 + st * C::STAGE, nb, wave, lane);
-        ld.v(a, w, smem, g0 + st * C::STAGE + C::TILE, nb, wave, lane);
+        if constexpr (RW == 4) {
+            if (nb >= w.n_blocks) return;
+            ld.k(a, w, smem, g0 + st * C::STAGE, nb, wave, lane);
+            ld.v(a, w, smem, g0 + st * C::STAGE + C::TILE, nb, wave, lane);
+        } else {
+            const int first = nb - part_step * grp;
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                if (first + part_step * g >= w.n_blocks) return;
+                const int off = (2 * g + st) * C::STAGE;
+                ld.k(a, w, smem, off, first + part_step * g, wave8, lane);
+                ld.v(a, w, smem, off + C::TILE, first + part_step * g, wave8, lane);
+            }
+        }
     };
 
     // One key block: S^T = K Q^T, online softmax, O^T += V^T P^T.  MASK is a
@@ -418,7 +434,7 @@ __global__ __launch_bounds__(256 * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 2 : 
         const int buf = it & 1, nb = it * step + nb0;
         wait_vmem();
         __syncthreads();  // block nb is in LDS; every wave is done with stage buf ^ 1
-        if (nb + step < w.n_blocks) issue(nb + step, buf ^ 1);
+        issue(nb + step, buf ^ 1);
         if (NG > 1 && nb >= w.n_blocks) return;
         const int n0 = nb * BN;
         if (CAUSAL && MASK && n0 > q_lo + 32 * QT - 1 + w.causal_off) return;  // no visible key for this wave
@@ -497,7 +513,7 @@ __global__ __launch_bounds__(256 * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 2 : 
     if (CAUSAL) n_full = min(n_full, max(0, (w.m0 + w.causal_off + 1) / BN));
     // Iterations in which every group has a block, and one without a mask.
     const int last0 = nb0 - part_step * grp + part_step * (NG - 1);  // the last group's first block
-    if (nb0 < w.n_blocks) issue(nb0, 0);
+    issue(nb0, 0);
     const int it_full = n_full > last0 ? (n_full - 1 - last0) / step + 1 : 0;
     const int n_it = w.n_blocks > part ? (w.n_blocks - 1 - part) / step + 1 : 0;
     for (int it = 0; it < it_full; ++it) block(it, std::false_type{});
@@ -509,28 +525,28 @@ __global__ __launch_bounds__(256 * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 2 : 
         // Each group finishes half of the head's dimensions: it hands the other
         // half of its O, and its maxima and sums, to the other group.
         constexpr int H = HD / 64;  // 32-wide dimension tiles of a half
-        const int t4 = tid & 255, r = 32 * wave + (lane & 31);
+        const int t4 = tid & (GT - 1), r = 32 * wave + (lane & 31);
         const float l_own = sum_xor32(row[0].l_p), m_own = row[0].m_t;
-        f32x4 *xo = reinterpret_cast<f32x4 *>(smem);                          // [group][4 H][256 threads]
-        f32x2 *xr = reinterpret_cast<f32x2 *>(smem + 2 * 4 * H * 256 * 16);   // [group][128 rows]
+        f32x4 *xo = reinterpret_cast<f32x4 *>(smem);                        // [group][4 H][GT threads]
+        f32x2 *xr = reinterpret_cast<f32x2 *>(smem + 2 * 4 * H * GT * 16);  // [group][BM rows]
         __syncthreads();  // every wave is done with the tiles
-        if (hh == 0) xr[grp * 128 + r] = f32x2{m_own, l_own};
+        if (hh == 0) xr[grp * BM + r] = f32x2{m_own, l_own};
         auto finish = [&](auto grp_tag) FA_INLINE {
             constexpr int GRP = decltype(grp_tag)::value;
 #pragma unroll
             for (int i = 0; i < 4 * H; ++i) {
                 const f32x16 &t = o[0][(1 - GRP) * H + i / 4];
-                xo[(GRP * 4 * H + i) * 256 + t4] = f32x4{t[4 * (i & 3)], t[4 * (i & 3) + 1], t[4 * (i & 3) + 2],
+                xo[(GRP * 4 * H + i) * GT + t4] = f32x4{t[4 * (i & 3)], t[4 * (i & 3) + 1], t[4 * (i & 3) + 2],
                                                          t[4 * (i & 3) + 3]};
             }
             __syncthreads();
-            const f32x2 other = xr[(1 - GRP) * 128 + r];
+            const f32x2 other = xr[(1 - GRP) * BM + r];
             float m = fmaxf(m_own, other[0]);
             const float a_own = m_own == -INFINITY ? 0.f : exp2_fast(m_own - m);
             const float a_other = other[0] == -INFINITY ? 0.f : exp2_fast(other[0] - m);
 #pragma unroll
             for (int i = 0; i < 4 * H; ++i) {
-                const f32x4 x = xo[((1 - GRP) * 4 * H + i) * 256 + t4];
+                const f32x4 x = xo[((1 - GRP) * 4 * H + i) * GT + t4];
                 f32x16 &t = o[0][GRP * H + i / 4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) t[4 * (i & 3) + e] = fmaf(x[e], a_other, t[4 * (i & 3) + e] * a_own);
@@ -767,39 +783,48 @@ static int fwd_pack_log2(const fa_fwd_args &a, int BM) {
     return lg;
 }
 
-// How the 128-row kernel runs: wave groups per workgroup and workgroups (splits)
-// per query block.  W: 128-row blocks (counted in 32-row tiles, so that a GQA
-// group packed into workgroups and its expanded heads get the same plan and
-// bits), NB: key blocks of the longest row.  Measured on MI355X, us at one group
-// and split -> as planned (groups x splits), head_dim 128 unless noted:
+// How fwd_kernel runs: row waves per wave group (32 rows each), wave groups per
+// workgroup and workgroups (splits) per query block.  W: 128-row blocks (counted
+// in 32-row tiles, so that a GQA group packed into workgroups and its expanded
+// heads get the same plan and bits), NB: key blocks of the longest row.  Measured
+// on MI355X, us at one group of 4 row waves -> as planned (row waves x groups x
+// splits), head_dim 128 unless noted:
 //   one workgroup per CU leaves each SIMD one wave; a second group halves the
 //   chain of key blocks (1.82 us for a pair of blocks against 2 x 1.22):
-//     b1 s1024 32/8 causal (W 256): 26.9 -> 23.5 (2 x 1)   s509: 16.7 -> 15.7 (2 x 1)
-//     b1 s4096 16/16 causal (W 512): 104 -> 89 (2 x 1)     s2048 16/16: 45.7 -> 38.3 (2 x 1)
-//     1024 rows x 16384 keys 32/8 (W 256): 328 -> 294 (2 x 1)
+//     b1 s1024 32/8 causal (W 256): 26.9 -> 23.9 (4 x 2 x 1)   s2048 16/16: 45.7 -> 38.3
+//     b1 s4096 16/16 causal (W 512): 104 -> 89                 1024 x 16384 keys 32/8: 328 -> 294
 //   it loses when two workgroups per CU fill the chip without a mask (W 512,
-//   s4096: 153 -> 159), on short chains (W 256, s256: 11.8 -> 12.7) and past W 512
+//   s4096: 153 -> 159), on short chains (W 256, s256: 11.8 -> 12.3) and past W 512
 //   (W 768, s2048: 74.5 -> 82);
-//   with idle CUs, splits take the rest (one launch to clear the counters and a
-//   merge: about 8 us, 2 more per split; a block pair takes 1.84 us, 1.31 at 64):
-//     512 rows x 16384 keys 32/8: 311 -> 160 (2 x 2)       128 rows: 309 -> 60 (2 x 8)
-//     b1 s2048 8/8 causal: 45.3 -> 30.2 (2 x 2)            512 x 8192 16/4 d64: 127 -> 38 (2 x 4)
+//   where half of the CUs would idle, two groups of 2 row waves use them all and
+//   read half as much LDS a CU (1.58 us a pair; 0.9 at head_dim 64):
+//     b1 s509 32/8 causal (W 128): 16.7 -> 13.5 (2 x 2 x 1)    s256: 11.5 -> 9.7
+//     b1 s700 32/8 causal (W 176): 20.9 -> 18.1                s1024 8/8 no mask: 25.7 -> 19.7
+//     d64 b1 s2048 16/16 causal (W 256): 35.1 -> 24.6          b4 s512 no mask: 12.8 -> 11.9
+//   not at W 256 at head_dim 128 (s1024 32/8: 23.9 -> 26.8), nor on long unmasked
+//   chains there (d64 b1 s2048: 29.3 -> 32.9);
+//   with CUs still idle and long chains, splits take them (one launch to clear the
+//   counters and a merge: about 8 us, 2 more per split):
+//     512 rows x 16384 keys 32/8: 311 -> 160 (4 x 2 x 2)       128 rows: 309 -> 60 (4 x 2 x 8)
+//     512 x 8192 16/4 d64: 127 -> 38 (4 x 2 x 4)
 struct FwdPlan {
-    int groups, splits;
+    int row_waves, groups, splits;
 };
 static FwdPlan fwd_plan(const fa_fwd_args &a) {
     const int64_t W = (int64_t(a.batch) * a.nheads * ((int64_t(a.lse_seqlen) + 31) / 32) + 3) / 4, cus = device_cus();
     const int NB = (a.seqlen_k + kFwdBN - 1) / kFwdBN;
-    FwdPlan plan = {1, 1};
+    FwdPlan plan = {4, 1, 1};
     if (2 * W <= cus ? NB >= 8 : W <= cus ? NB >= 12 : W <= 2 * cus && a.causal && NB >= 32) plan.groups = 2;
-    if (plan.groups == 1 || 2 * W > cus || a.cu_seqlens_q) return plan;
+    const bool narrow = 2 * W <= cus || (a.head_dim == 64 ? W <= cus && (a.causal || NB <= 16) : 4 * W <= 3 * cus && a.causal);
+    if (a.cu_seqlens_q || !narrow) return plan;  // varlen work orders list 128-row blocks
+    plan = {2, 2, 1};
     const double pairs = 0.5 * NB, unit = a.head_dim == 128 ? 1.84 : 1.31;
-    double best = pairs * unit;
+    double best = pairs * (a.head_dim == 128 ? 1.58 : 0.9);
     for (int S = 2; S <= 16 && W * S <= cus; ++S) {
         const double t = pairs / S * unit + 6 + 2 * S;
         if (t < best) {
             best = t;
-            plan.splits = S;
+            plan = {4, 2, S};
         }
     }
     return plan;
@@ -855,10 +880,21 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
             if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
             const int rc = launch_order(a, int(m_blocks), P, stream);
             if (rc) return rc;
-            hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 2, 1, false>), dim3(unsigned(grid)), dim3(256), 0, stream, a,
+            hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 2, 1, 4, false>), dim3(unsigned(grid)), dim3(256), 0, stream, a,
                                int(m_blocks), lg, 1);
             return int(hipGetLastError());
         }
+    }
+    const FwdPlan plan = fwd_plan(a);
+    if (plan.row_waves == 2) {
+        const int lg = fwd_pack_log2(a, 64), P = 64 >> lg;
+        const int m_blocks = (a.lse_seqlen + P - 1) / P;
+        const int64_t grid = int64_t(m_blocks) * a.batch * (a.nheads >> lg);
+        if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
+        if (grid == 0) return FA_OK;
+        hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 1, 2, 2, false>), dim3(unsigned(grid)), dim3(256), 0, stream, a,
+                           m_blocks, lg, 1);
+        return int(hipGetLastError());
     }
     constexpr int BM = FwdCfg<HD, 256>::BM;
     const int lg = fwd_pack_log2(a, BM), P = BM >> lg;
@@ -867,7 +903,6 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
     if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
     const int rc = launch_order(a, num_m_blocks, P, stream);
     if (rc || grid == 0) return rc;
-    const FwdPlan plan = fwd_plan(a);
     const int S = a.split_ws && a.split_ws_bytes >= int64_t(fwd_split_bytes(a, plan.splits)) ? plan.splits : 1;
     if (S > 1) {
         hipLaunchKernelGGL(zero_counts_kernel, dim3(unsigned((2 * grid + 255) / 256)), dim3(256), 0, stream,
@@ -877,7 +912,7 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
     }
     auto go = [&](auto ng_tag, auto split_tag) {
         constexpr int NG = decltype(ng_tag)::value;
-        hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 1, NG, decltype(split_tag)::value>), dim3(unsigned(grid * S)),
+        hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 1, NG, 4, decltype(split_tag)::value>), dim3(unsigned(grid * S)),
                            dim3(256 * NG), 0, stream, a, num_m_blocks, lg, S);
     };
     using G1 = std::integral_constant<int, 1>;
