@@ -892,12 +892,21 @@ static size_t dkdv_ws_bytes(const fa_bwd_args &a, int S) {
     return S > 1 ? size_t(dkdv_count_bytes(items) + items * S * 2 * 128 * a.head_dim * int64_t(sizeof(float))) : 0;
 }
 
+// The arguments as the kernels take them: split_ws is set only when the grid is
+// split and the workspace holds all of it (every kernel that sees it writes to it).
+static fa_bwd_args usable_split_ws(const fa_bwd_args &args) {
+    fa_bwd_args a = args;
+    const size_t bytes = a.split_ws ? fa_bwd_split_bytes(&a) : 0;
+    if (bytes == 0 || a.split_ws_bytes < int64_t(bytes)) a.split_ws = nullptr;
+    return a;
+}
+
 template <int HD, bool CAUSAL>
 static int launch_dkdv(const fa_bwd_args &a, hipStream_t s) {
     // seqlen_k bounds every sequence's key count (max_seqlen_k for varlen).
     static_assert(DkvCfg<HD>::BN == 128, "bwd_order_kernel and fa_bwd_order_len assume 128-key blocks");
     const int nnb = (a.seqlen_k + DkvCfg<HD>::BN - 1) / DkvCfg<HD>::BN;
-    const int S = a.split_ws && a.split_ws_bytes >= int64_t(dkdv_ws_bytes(a, dkdv_splits(a))) ? dkdv_splits(a) : 1;
+    const int S = a.split_ws ? dkdv_splits(a) : 1;
     const int64_t grid = int64_t(nnb) * a.batch * a.nheads_k * S;
     if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
     if (a.cu_seqlens_k && (a.work_order || a.dkv_rows > 0)) {
@@ -930,15 +939,16 @@ extern "C" int fa_bwd_preprocess(const fa_bwd_args *args, void *stream) {
     int rc = fa::check_bwd(args);
     if (rc) return rc;
     if ((rc = check_bwd_tensors(args))) return rc;
+    const fa_bwd_args a = fa::usable_split_ws(*args);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    return args->head_dim == 128 ? fa::launch_preprocess<128>(*args, s) : fa::launch_preprocess<64>(*args, s);
+    return a.head_dim == 128 ? fa::launch_preprocess<128>(a, s) : fa::launch_preprocess<64>(a, s);
 }
 
 extern "C" int fa_bwd_dq(const fa_bwd_args *args, void *stream) {
     int rc = fa::check_bwd(args);
     if (rc) return rc;
     if ((rc = check_bwd_tensors(args))) return rc;
-    const fa_bwd_args &a = *args;
+    const fa_bwd_args a = fa::usable_split_ws(*args);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (a.head_dim == 128) return a.causal ? fa::launch_dq<128, true>(a, s) : fa::launch_dq<128, false>(a, s);
     return a.causal ? fa::launch_dq<64, true>(a, s) : fa::launch_dq<64, false>(a, s);
@@ -948,7 +958,7 @@ extern "C" int fa_bwd_dkdv(const fa_bwd_args *args, void *stream) {
     int rc = fa::check_bwd(args);
     if (rc) return rc;
     if ((rc = check_bwd_tensors(args))) return rc;
-    const fa_bwd_args &a = *args;
+    const fa_bwd_args a = fa::usable_split_ws(*args);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (a.head_dim == 128) return a.causal ? fa::launch_dkdv<128, true>(a, s) : fa::launch_dkdv<128, false>(a, s);
     return a.causal ? fa::launch_dkdv<64, true>(a, s) : fa::launch_dkdv<64, false>(a, s);

@@ -102,6 +102,28 @@ def test_split_dkdv_varlen(device, ordered):
     check_varlen("split varlen", cu_q, cu_k, q, k, v, do, o.cpu(), lse.cpu(), tuple(t.cpu() for t in grads), s, True)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("short_by", [1, None])
+def test_small_workspace_is_not_touched(device, short_by):
+    """A split_ws below fa_bwd_split_bytes (by a byte, or all but 8 bytes of it) gives the unsplit kernel's bits and is
+    not written (the buffer behind the pointer has the whole size)."""
+    b, sq, sk, h, hk, hd = 1, 512, 512, 8, 2, 128
+    g = torch.Generator().manual_seed(8300)
+    q, do = randn16((b, sq, h, hd), g).to(device), randn16((b, sq, h, hd), g).to(device)
+    k, v = randn16((b, sk, hk, hd), g).to(device), randn16((b, sk, hk, hd), g).to(device)
+    print(f"case small workspace short_by={short_by}", flush=True)
+    ba, o, lse, grads = _args(q, k, v, do, hd ** -0.5, True)
+    fa_capi.call("fa_bwd", ba)
+    plain = [t.clone() for t in grads]
+    ws = _split_ws(ba, device)
+    ba.split_ws_bytes = ws.numel() - short_by if short_by else 8
+    for entry in ("fa_bwd", "fa_bwd_preprocess"):
+        fa_capi.call(entry, ba)
+        torch.cuda.synchronize()
+        assert bool((ws == 255).all()), entry
+        assert all(torch.equal(x, y) for x, y in zip(grads, plain))
+
+
 def test_split_bytes_rule():
     """Sizes that fill the chip by themselves take no workspace; the partials stay within 256 MiB."""
     def size(b, sq, sk, h, hk, hd, causal):
