@@ -104,14 +104,31 @@ int num_cus(int device) {
     return n;
 }
 
-// The workspace in which workgroups that share a query or key block sum their
-// results (undefined when the grid needs no sharing).
-template <class Args>
-at::Tensor split_workspace(Args &a, size_t bytes, const at::Tensor &like) {
+// The workspace in which workgroups that share a query block sum their results
+// (undefined when the grid needs no sharing).
+at::Tensor fwd_workspace(fa_fwd_args &a, const at::Tensor &like) {
+    const size_t bytes = fa_fwd_split_bytes(&a);
     if (bytes == 0) return at::Tensor();
     at::Tensor ws = at::empty({int64_t(bytes)}, like.options().dtype(at::kByte));
     a.split_ws = ws.data_ptr();
     a.split_ws_bytes = int64_t(bytes);
+    return ws;
+}
+
+// The backward's workspaces in one tensor: -D and LSE*log2(e) (dsum), then, at
+// the next 256 bytes, the one in which workgroups that share a key block sum
+// their results (when there are such).  Calls of a few tens of microseconds of
+// GPU time wait for the host, and a second allocation was part of that (forward
+// and backward, b1 s700 16/16 d64: 85.6 -> 81.3 us; b2 s200 16/4: 95.4 -> 90.8).
+at::Tensor bwd_workspace(fa_bwd_args &a, const at::Tensor &l) {
+    const int64_t split = int64_t(fa_bwd_split_bytes(&a));
+    const int64_t dsum = 2 * l.numel(), at_split = split > 0 ? (dsum + 63) / 64 * 64 : dsum;  // in floats
+    at::Tensor ws = at::empty({at_split + (split + 3) / 4}, l.options());
+    a.dsum = ws.data_ptr<float>();
+    if (split > 0) {
+        a.split_ws = a.dsum + at_split;
+        a.split_ws_bytes = split;
+    }
     return ws;
 }
 
@@ -153,7 +170,7 @@ std::vector<at::Tensor> mha_fwd(at::Tensor q, at::Tensor k, at::Tensor v, const 
     a.lse_seqlen = i32(seqlen_q, "seqlen_q");
     a.softmax_scale = softmax_scale;
     a.causal = is_causal ? 1 : 0;
-    at::Tensor split_ws = split_workspace(a, fa_fwd_split_bytes(&a), q);
+    at::Tensor split_ws = fwd_workspace(a, q);
     check_rc(fa_fwd(&a, current_stream()), "fa_fwd");
     return {o, l};
 }
@@ -186,7 +203,6 @@ std::vector<at::Tensor> mha_bwd(at::Tensor q, at::Tensor k, at::Tensor v, at::Te
 
     GradOut dq = grad_out(dq_, q, false, false, "dq"), dk = grad_out(dk_, k, false, false, "dk"),
             dv = grad_out(dv_, v, false, false, "dv");
-    at::Tensor dsum = at::empty({2, l.numel()}, l.options());  // -D, then LSE*log2(e)
 
     fa_bwd_args a{};
     a.q = desc4(q);
@@ -198,7 +214,6 @@ std::vector<at::Tensor> mha_bwd(at::Tensor q, at::Tensor k, at::Tensor v, at::Te
     a.dk = desc4(dk.buf);
     a.dv = desc4(dv.buf);
     a.lse = l.data_ptr<float>();
-    a.dsum = dsum.data_ptr<float>();
     a.batch = i32(batch_size, "batch_size");
     a.seqlen_q = i32(seqlen_q, "seqlen_q");
     a.seqlen_k = i32(seqlen_k, "seqlen_k");
@@ -208,7 +223,7 @@ std::vector<at::Tensor> mha_bwd(at::Tensor q, at::Tensor k, at::Tensor v, at::Te
     a.lse_seqlen = i32(seqlen_q, "seqlen_q");
     a.softmax_scale = softmax_scale;
     a.causal = is_causal ? 1 : 0;
-    at::Tensor split_ws = split_workspace(a, fa_bwd_split_bytes(&a), q);
+    at::Tensor ws = bwd_workspace(a, l);
     check_rc(fa_bwd(&a, current_stream()), "fa_bwd");
     for (auto *g : {&dq, &dk, &dv}) g->finish();
     return {dq.dst, dk.dst, dv.dst};
@@ -317,7 +332,6 @@ std::vector<at::Tensor> mha_varlen_bwd(at::Tensor q, at::Tensor k, at::Tensor v,
         if (dv.rest) dv.buf.zero_();
         dk.rest = dv.rest = false;
     }
-    at::Tensor dsum = at::empty({2, l.numel()}, l.options());  // -D, then LSE*log2(e)
 
     fa_bwd_args a{};
     a.q = desc3(q);
@@ -329,7 +343,6 @@ std::vector<at::Tensor> mha_varlen_bwd(at::Tensor q, at::Tensor k, at::Tensor v,
     a.dk = desc3(dk.buf);
     a.dv = desc3(dv.buf);
     a.lse = l.data_ptr<float>();
-    a.dsum = dsum.data_ptr<float>();
     a.cu_seqlens_q = cu_seqlens_q.data_ptr<int32_t>();
     a.cu_seqlens_k = cu_seqlens_k.data_ptr<int32_t>();
     a.batch = i32(batch_size, "batch_size");
@@ -346,7 +359,7 @@ std::vector<at::Tensor> mha_varlen_bwd(at::Tensor q, at::Tensor k, at::Tensor v,
     // dQ and dK/dV work items ordered longest first on the device (sequences of mixed lengths).
     at::Tensor work_order = at::empty({int64_t(std::max<size_t>(fa_bwd_order_len(&a), 1))}, cu_seqlens_k.options());
     a.work_order = work_order.data_ptr<int32_t>();
-    at::Tensor split_ws = split_workspace(a, fa_bwd_split_bytes(&a), q);
+    at::Tensor ws = bwd_workspace(a, l);
     check_rc(fa_bwd(&a, current_stream()), "fa_bwd (varlen)");
     for (auto *g : {&dq, &dk, &dv}) g->finish();
     return {dq.dst, dk.dst, dv.dst};
@@ -629,7 +642,7 @@ std::vector<at::Tensor> mha_fwd_kvcache(at::Tensor q, at::Tensor k_cache, at::Te
     f.causal = is_causal ? 1 : 0;
     f.k_batch = i32(batch_size_cache, "cache batch size");
     f.status = status;
-    at::Tensor split_ws = split_workspace(f, fa_fwd_split_bytes(&f), q);
+    at::Tensor split_ws = fwd_workspace(f, q);
     check_rc(fa_fwd(&f, stream), "fa_fwd (kv-cache chunk)");
     return {out, lse};
 }
