@@ -30,20 +30,20 @@ constexpr int kBwdThreads = 256;
 // 128; 3 at head_dim 64, whose registers then allow three workgroups per CU).
 constexpr int kDqPipe = 4;
 
-// Split dK/dV (bwd_dkdv_kernel, SPLIT): the workspace starts with two int32
-// counters per (batch, key block, KV head) item, then (256-byte aligned) the
-// fp32 partial sums.
+// Split dK/dV (bwd_dkdv_kernel, SPLIT): the workspace starts with an int32
+// counter per (batch, key block, KV head) item, then (256-byte aligned) the fp32
+// partial sums.
 __host__ __device__ __forceinline__ int64_t dkdv_items(const fa_bwd_args &a) {
     return int64_t((a.seqlen_k + 127) / 128) * a.batch * a.nheads_k;
 }
-__host__ __device__ __forceinline__ int64_t dkdv_count_bytes(int64_t items) { return (items * 8 + 255) & ~int64_t(255); }
+__host__ __device__ __forceinline__ int64_t dkdv_count_bytes(int64_t items) { return (items * 4 + 255) & ~int64_t(255); }
 
 // Zeroes those counters: run by every workgroup of the kernel that fills dsum
 // (the dQ or the preprocess kernel), which precedes dK/dV on the stream.
 __device__ __forceinline__ void zero_dkdv_counts(const fa_bwd_args &a, int block, int n_blocks) {
     if (!a.split_ws) return;
     int32_t *count = reinterpret_cast<int32_t *>(a.split_ws);
-    const int64_t n = 2 * dkdv_items(a);
+    const int64_t n = dkdv_items(a);
     for (int64_t i = int64_t(block) * kBwdThreads + threadIdx.x; i < n; i += int64_t(n_blocks) * kBwdThreads)
         count[i] = 0;
 }
@@ -386,53 +386,44 @@ __global__ __launch_bounds__(kOrderThreads) void dq_order_kernel(const fa_bwd_ar
     }, a.work_order + int64_t(a.batch) * nnb, false);
 }
 
-// Sums the S partial dK / dV tiles of an item.  The first S - 1 of its
-// workgroups to get here (count[0]) store theirs and count them stored
-// (count[1]); the last one waits for those stores, which are under way, and
-// adds the partials in the order of their shares, so the sum does not depend
-// on who came last.  Returns whether this workgroup holds the sum.  Partials
-// are stored and loaded at agent scope (past the XCD's L2, as in the split KV
-// kernel), 8 bytes a lane, 512 contiguous bytes a wave.
+// Sums the S partial dK / dV tiles of an item.  Each of its workgroups stores
+// its own and then counts itself; the one that counts last finds all of them
+// stored and adds them in the order of their shares, so the sum does not depend
+// on who came last and no workgroup waits for another.  Returns whether this
+// workgroup holds the sum.  Partials are stored and loaded at agent scope (past
+// the XCD's L2, as in the split KV kernel), 8 bytes a lane, 512 contiguous bytes
+// a wave.
 template <int HD>
 __device__ __forceinline__ bool dkdv_reduce(const fa_bwd_args &a, int item, int part, int S, int *ticket,
                                             f32x16 (&dk)[HD / 32], f32x16 (&dv)[HD / 32]) {
     constexpr int N = HD / 2;  // pairs of floats a lane holds: dK, then dV
     const int tid = threadIdx.x;
-    int32_t *count = reinterpret_cast<int32_t *>(a.split_ws) + 2 * int64_t(item);
-    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    const bool last = *ticket == S - 1;
+    int32_t *count = reinterpret_cast<int32_t *>(a.split_ws) + item;
     uint64_t *slots = reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(a.split_ws) + dkdv_count_bytes(dkdv_items(a))) +
                       int64_t(item) * S * N * kDkvThreads + tid;
-    // The last workgroup adds to its own registers when its share is one of
-    // the first two (x0 + x1 = x1 + x0); otherwise it stores too and adds all
-    // shares from memory.
-    if (!last || part >= 2) {
-        uint64_t *slot = slots + int64_t(part) * N * kDkvThreads;
+    uint64_t *own = slots + int64_t(part) * N * kDkvThreads;
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            f32x16 &t = i < N / 2 ? dk[i / 8] : dv[i / 8 - N / 16];
-            const f32x2 x = {t[2 * (i & 7)], t[2 * (i & 7) + 1]};
-            __hip_atomic_store(slot + i * kDkvThreads, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        }
-        wait_vmem();
-        if (!last) {
-            __syncthreads();  // every wave's stores have completed
-            if (tid == 0) __hip_atomic_fetch_add(count + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
-        }
+    for (int i = 0; i < N; ++i) {
+        f32x16 &t = i < N / 2 ? dk[i / 8] : dv[i / 8 - N / 16];
+        const f32x2 x = {t[2 * (i & 7)], t[2 * (i & 7) + 1]};
+        __hip_atomic_store(own + i * kDkvThreads, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+    wait_vmem();
+    __syncthreads();  // every wave's stores have completed
+    if (tid == 0) {
+        *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // Ready for another dK/dV call on the same workspace.
+        if (*ticket == S - 1) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (*ticket != S - 1) return false;
+    // It adds to its own registers when its share is one of the first two (x0 +
+    // x1 = x1 + x0), and all shares from memory otherwise.
+    if (part >= 2) {
 #pragma unroll
         for (int i = 0; i < HD / 32; ++i) dk[i] = dv[i] = zero16();
     }
-    if (tid == 0) {
-        while (__hip_atomic_load(count + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < S - 1)
-            __builtin_amdgcn_s_sleep(1);
-        // Ready for another dK/dV call on the same workspace.
-        __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(count + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
     for (int p = 0; p < S; ++p) {
         if (p == part && part < 2) continue;
         const uint64_t *slot = slots + int64_t(p) * N * kDkvThreads;

@@ -237,49 +237,40 @@ __device__ __forceinline__ void store_row(const fa_fwd_args &a, const FwdWork &w
     }
 }
 
-// Splits (fwd_kernel, SPLIT): the workspace starts with two int32 counters per
+// Splits (fwd_kernel, SPLIT): the workspace starts with an int32 counter per
 // workgroup of the unsplit grid (an item: 128 rows), then, 256-byte aligned, the
 // items' S x 128 rows' (maximum, sum) and their S x 128 x HD partial O in fp32.
-__host__ __device__ __forceinline__ int64_t fwd_count_bytes(int64_t items) { return (items * 8 + 255) & ~int64_t(255); }
+__host__ __device__ __forceinline__ int64_t fwd_count_bytes(int64_t items) { return (items * 4 + 255) & ~int64_t(255); }
 
 // Sums the S partial results of an item over dimension tiles [D0, D1) of O.
-// The first S - 1 workgroups to get here (count[0]) store theirs and count them
-// stored (count[1]); the last one waits for those stores, which are under way,
-// and sums all in split order, its own from registers.  Returns whether this
-// workgroup holds the sum.
+// Every workgroup stores its own and then counts itself; the one that counts
+// last finds all of them stored and sums them in split order, its own from
+// registers, so no workgroup waits for another.  Returns whether this workgroup
+// holds the sum.
 template <int HD, int D0, int D1>
 __device__ __forceinline__ bool fwd_merge(const fa_fwd_args &a, int64_t items, int item, int part, int S, int r,
                                           int *ticket, f32x16 (&o)[HD / 32], float &m, float &l) {
     constexpr int N = 8 * (D1 - D0), NT = 512;  // pairs of floats a lane holds, threads
     const int tid = threadIdx.x, hh = (tid >> 5) & 1;
-    int32_t *count = reinterpret_cast<int32_t *>(a.split_ws) + 2 * int64_t(item);
-    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    const int got = *ticket;
+    int32_t *count = reinterpret_cast<int32_t *>(a.split_ws) + item;
     uint64_t *rows = reinterpret_cast<uint64_t *>(static_cast<char *>(a.split_ws) + fwd_count_bytes(items));
     uint64_t *pairs = rows + items * S * 128 + int64_t(item) * S * N * NT + tid;
     rows += int64_t(item) * S * 128 + r;
-    if (got < S - 1) {
-        uint64_t *slot = pairs + int64_t(part) * N * NT;
+    uint64_t *own = pairs + int64_t(part) * N * NT;
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const f32x16 &t = o[D0 + i / 8];
-            const f32x2 x = {t[2 * (i & 7)], t[2 * (i & 7) + 1]};
-            __hip_atomic_store(slot + i * NT, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (D0 == 0 && hh == 0)
-            __hip_atomic_store(rows + part * 128, __builtin_bit_cast(uint64_t, f32x2{m, l}), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        wait_vmem();
-        __syncthreads();  // every wave's stores have completed
-        if (tid == 0) __hip_atomic_fetch_add(count + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return false;
+    for (int i = 0; i < N; ++i) {
+        const f32x16 &t = o[D0 + i / 8];
+        const f32x2 x = {t[2 * (i & 7)], t[2 * (i & 7) + 1]};
+        __hip_atomic_store(own + i * NT, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (tid == 0)
-        while (__hip_atomic_load(count + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < S - 1)
-            __builtin_amdgcn_s_sleep(1);
+    if (D0 == 0 && hh == 0)
+        __hip_atomic_store(rows + part * 128, __builtin_bit_cast(uint64_t, f32x2{m, l}), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    wait_vmem();
+    __syncthreads();  // every wave's stores have completed
+    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
+    if (*ticket != S - 1) return false;
     auto row_of = [&](int p) {
         return p == part ? f32x2{m, l}
                          : __builtin_bit_cast(f32x2, __hip_atomic_load(rows + p * 128, __ATOMIC_RELAXED,
@@ -905,8 +896,8 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
     if (rc || grid == 0) return rc;
     const int S = a.split_ws && a.split_ws_bytes >= int64_t(fwd_split_bytes(a, plan.splits)) ? plan.splits : 1;
     if (S > 1) {
-        hipLaunchKernelGGL(zero_counts_kernel, dim3(unsigned((2 * grid + 255) / 256)), dim3(256), 0, stream,
-                           reinterpret_cast<int32_t *>(a.split_ws), int(2 * grid));
+        hipLaunchKernelGGL(zero_counts_kernel, dim3(unsigned((grid + 255) / 256)), dim3(256), 0, stream,
+                           reinterpret_cast<int32_t *>(a.split_ws), int(grid));
         const int rc2 = int(hipGetLastError());
         if (rc2) return rc2;
     }

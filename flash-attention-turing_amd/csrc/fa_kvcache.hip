@@ -773,12 +773,12 @@ __global__ __launch_bounds__(256, 2) void kv_splitkv_kernel(const fa_kvcache_arg
 constexpr int kChunkRows = 128, kChunkKeys = 64, kChunkPages = 1024;
 constexpr int kChunkMinRows = 64, kChunkMaxSplits = 32;
 
-// Merges the partial rows (O normalised, LSE) of a row tile's splits.  The
-// first S - 1 items to get here (count[0]) store theirs, lane by lane, and
-// count them stored (count[1]); the last one waits for those stores, which are
-// under way, and sums all in split order, its own from registers.  row0:
-// the tile's first row of a split's accumulators, rows_here x HD values from there.
-// Returns whether this item holds the sum.
+// Merges the partial rows (O normalised, LSE) of a row tile's splits.  Every
+// item stores its own, lane by lane, and then counts itself; the one that
+// counts last finds all of them stored and sums them in split order, its own
+// from registers, so no item waits for another.  row0: the tile's first row of
+// a split's accumulators, rows_here x HD values from there.  Returns whether
+// this item holds the sum.
 template <int HD>
 __device__ __forceinline__ bool chunk_merge(const fa_kvcache_args &a, int32_t *count, int split, int64_t row0,
                                             int rows_here, int row, int hh, int *ticket, f32x16 (&o)[HD / 32],
@@ -786,34 +786,27 @@ __device__ __forceinline__ bool chunk_merge(const fa_kvcache_args &a, int32_t *c
     constexpr int N = HD / 4;  // pairs of floats a lane holds
     const int S = a.num_splits, tid = threadIdx.x;
     const int64_t nrow = int64_t(a.batch) * a.nheads * a.seqlen_q;
-    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
     const bool live = row < rows_here;
     // Pair i of a lane: element (2 i + hh) * rows_here + row, 256 contiguous bytes a half wave.
     uint64_t *pairs = reinterpret_cast<uint64_t *>(a.out_accum + row0 * HD) + hh * rows_here + row;
     const int step = 2 * rows_here;
     float *lses = a.lse_accum + row0 + row;
-    if (*ticket < S - 1) {
-        if (live) {
-            uint64_t *slot = pairs + int64_t(split) * nrow * (HD / 2);
+    if (live) {
+        uint64_t *slot = pairs + int64_t(split) * nrow * (HD / 2);
 #pragma unroll
-            for (int i = 0; i < N; ++i) {
-                const f32x2 x = {o[i / 8][2 * (i & 7)], o[i / 8][2 * (i & 7) + 1]};
-                __hip_atomic_store(slot + i * step, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            }
-            if (hh == 0)
-                __hip_atomic_store(lses + int64_t(split) * nrow, lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int i = 0; i < N; ++i) {
+            const f32x2 x = {o[i / 8][2 * (i & 7)], o[i / 8][2 * (i & 7) + 1]};
+            __hip_atomic_store(slot + i * step, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
         }
-        wait_vmem();
-        __syncthreads();  // every wave's stores have completed
-        if (tid == 0) __hip_atomic_fetch_add(count + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return false;
+        if (hh == 0)
+            __hip_atomic_store(lses + int64_t(split) * nrow, lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (tid == 0)
-        while (__hip_atomic_load(count + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < S - 1)
-            __builtin_amdgcn_s_sleep(1);
+    wait_vmem();
+    __syncthreads();  // every wave's stores have completed
+    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
+    if (*ticket != S - 1) return false;
     if (!live) return true;
     auto lse_of = [&](int s) {
         return s == split ? lse
@@ -1063,7 +1056,7 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcach
     // before the block loop and held through it.
     int orow = row;
     asm volatile("" : "+v"(orow));
-    if (S == 1 || chunk_merge<HD>(a, count + 2 * tile, split, row0, rows_here, orow, hh, &ticket, o, lse)) {
+    if (S == 1 || chunk_merge<HD>(a, count + tile, split, row0, rows_here, orow, hh, &ticket, o, lse)) {
         if (orow < rows_here) {
             const int oq = (first + orow) / G, oh = hk * G + (first + orow) % G;
             f16 *op = (f16 *)a.o.ptr + int64_t(b) * a.o.batch_stride + int64_t(oq) * a.o.row_stride +
@@ -1395,7 +1388,8 @@ extern "C" int fa_fwd_kvcache(const fa_kvcache_args *args, void *stream) {
 // calls: the split kernel writes every partial it later combines, and the
 // ordering workgroup resets the work counter and the split counts.  Calls on
 // one device share the array, so calls that overlap on a device (different
-// streams) race.
+// streams) race; their results are undefined, but no workgroup waits for another
+// one's counts, so every kernel ends.
 static __device__ __align__(256) char scratch[FA_NOALLOC_SCRATCH_BYTES];
 
 namespace {

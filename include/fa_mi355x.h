@@ -258,7 +258,9 @@ int fa_fwd_kvcache(const fa_kvcache_args *args, void *stream);
  * that, i.e. fa_kv_workspace_bytes(args) + 4 * (batch + 1 +
  * fa_kv_split_count_len(args)) bytes, returns FA_ERR_SCRATCH.
  * No allocation or free happens in the call.  Calls on one device share its
- * array: calls that overlap on one device (on different streams) race.
+ * array: calls that overlap on one device (on different streams) race, and
+ * their results are undefined.  (No kernel waits for a word in memory, so the
+ * kernels end all the same.)
  */
 #define FA_NOALLOC_SCRATCH_BYTES (16u << 20)
 int fa_fwd_kvcache_noalloc(const fa_kvcache_args *args, void *stream);
