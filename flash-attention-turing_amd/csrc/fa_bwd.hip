@@ -38,8 +38,9 @@ __host__ __device__ __forceinline__ int64_t dkdv_items(const fa_bwd_args &a) {
 }
 __host__ __device__ __forceinline__ int64_t dkdv_count_bytes(int64_t items) { return (items * 4 + 255) & ~int64_t(255); }
 
-// Zeroes those counters: run by every workgroup of the kernel that fills dsum
-// (the dQ or the preprocess kernel), which precedes dK/dV on the stream.
+// Zeroes those counters: run by every workgroup of the dQ kernel, which precedes
+// dK/dV on the stream in fa_bwd (fa_bwd_dkdv by itself clears them in a launch of
+// its own).
 __device__ __forceinline__ void zero_dkdv_counts(const fa_bwd_args &a, int block, int n_blocks) {
     if (!a.split_ws) return;
     int32_t *count = reinterpret_cast<int32_t *>(a.split_ws);
@@ -59,7 +60,6 @@ __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const fa_bwd_args a
     constexpr int KCH = HD / 8;
     constexpr int ROWS = kBwdThreads / KCH;  // rows per workgroup
     const int b = blockIdx.z, h = blockIdx.y;
-    zero_dkdv_counts(a, (b * gridDim.y + h) * gridDim.x + blockIdx.x, gridDim.x * gridDim.y * gridDim.z);
     const bool packed = a.cu_seqlens_q != nullptr;
     const SeqInfo si = seq_info(b, a.seqlen_q, a.seqlen_k, a.cu_seqlens_q, a.cu_seqlens_k, nullptr, 0);
     const int i = blockIdx.x * ROWS + threadIdx.x / KCH;
@@ -411,11 +411,7 @@ __device__ __forceinline__ bool dkdv_reduce(const fa_bwd_args &a, int item, int 
     }
     wait_vmem();
     __syncthreads();  // every wave's stores have completed
-    if (tid == 0) {
-        *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // Ready for another dK/dV call on the same workspace.
-        if (*ticket == S - 1) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (*ticket != S - 1) return false;
     // It adds to its own registers when its share is one of the first two (x0 +
@@ -892,8 +888,9 @@ static fa_bwd_args usable_split_ws(const fa_bwd_args &args) {
     return a;
 }
 
+// cleared: the dQ kernel of the same call has zeroed split_ws's counters.
 template <int HD, bool CAUSAL>
-static int launch_dkdv(const fa_bwd_args &a, hipStream_t s) {
+static int launch_dkdv(const fa_bwd_args &a, bool cleared, hipStream_t s) {
     // seqlen_k bounds every sequence's key count (max_seqlen_k for varlen).
     static_assert(DkvCfg<HD>::BN == 128, "bwd_order_kernel and fa_bwd_order_len assume 128-key blocks");
     const int nnb = (a.seqlen_k + DkvCfg<HD>::BN - 1) / DkvCfg<HD>::BN;
@@ -908,6 +905,10 @@ static int launch_dkdv(const fa_bwd_args &a, hipStream_t s) {
         if (rc) return rc;
     }
     if (grid == 0) return FA_OK;
+    if (S > 1 && !cleared) {
+        const int rc = clear_counts(a.split_ws, dkdv_items(a), s);
+        if (rc) return rc;
+    }
     if (S > 1)
         hipLaunchKernelGGL((bwd_dkdv_kernel<HD, CAUSAL, true>), dim3(unsigned(grid)), dim3(kDkvThreads), 0, s, a, nnb,
                            S, paired_cus(a, grid));
@@ -930,9 +931,8 @@ extern "C" int fa_bwd_preprocess(const fa_bwd_args *args, void *stream) {
     int rc = fa::check_bwd(args);
     if (rc) return rc;
     if ((rc = check_bwd_tensors(args))) return rc;
-    const fa_bwd_args a = fa::usable_split_ws(*args);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    return a.head_dim == 128 ? fa::launch_preprocess<128>(a, s) : fa::launch_preprocess<64>(a, s);
+    return args->head_dim == 128 ? fa::launch_preprocess<128>(*args, s) : fa::launch_preprocess<64>(*args, s);
 }
 
 extern "C" int fa_bwd_dq(const fa_bwd_args *args, void *stream) {
@@ -945,15 +945,18 @@ extern "C" int fa_bwd_dq(const fa_bwd_args *args, void *stream) {
     return a.causal ? fa::launch_dq<64, true>(a, s) : fa::launch_dq<64, false>(a, s);
 }
 
-extern "C" int fa_bwd_dkdv(const fa_bwd_args *args, void *stream) {
+static int run_dkdv(const fa_bwd_args *args, bool cleared, void *stream) {
     int rc = fa::check_bwd(args);
     if (rc) return rc;
     if ((rc = check_bwd_tensors(args))) return rc;
     const fa_bwd_args a = fa::usable_split_ws(*args);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (a.head_dim == 128) return a.causal ? fa::launch_dkdv<128, true>(a, s) : fa::launch_dkdv<128, false>(a, s);
-    return a.causal ? fa::launch_dkdv<64, true>(a, s) : fa::launch_dkdv<64, false>(a, s);
+    if (a.head_dim == 128)
+        return a.causal ? fa::launch_dkdv<128, true>(a, cleared, s) : fa::launch_dkdv<128, false>(a, cleared, s);
+    return a.causal ? fa::launch_dkdv<64, true>(a, cleared, s) : fa::launch_dkdv<64, false>(a, cleared, s);
 }
+
+extern "C" int fa_bwd_dkdv(const fa_bwd_args *args, void *stream) { return run_dkdv(args, false, stream); }
 
 extern "C" size_t fa_bwd_order_len(const fa_bwd_args *a) {
     if (!a || a->batch <= 0) return 0;
@@ -973,5 +976,5 @@ extern "C" int fa_bwd(const fa_bwd_args *args, void *stream) {
     // The dQ kernel also writes -D = -rowsum(dO * O) for the dK/dV kernel.
     int rc = fa_bwd_dq(args, stream);
     if (rc) return rc;
-    return fa_bwd_dkdv(args, stream);
+    return run_dkdv(args, true, stream);
 }

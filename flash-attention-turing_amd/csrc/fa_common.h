@@ -466,6 +466,18 @@ __device__ __forceinline__ int paired_place(int bid, int n, int cus) {
     return layer & 1 ? layer * cus + min(n, (layer + 1) * cus) - 1 - bid : bid;
 }
 
+// Clears the counters (n int32s at ws) of the items that workgroups share, by a
+// kernel: a memset node in a captured graph has misbehaved on replay.
+static __global__ void zero_counts_kernel(int32_t *count, int64_t n) {
+    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (i < n) count[i] = 0;
+}
+static inline int clear_counts(void *ws, int64_t n, hipStream_t stream) {
+    hipLaunchKernelGGL(zero_counts_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, stream,
+                       static_cast<int32_t *>(ws), n);
+    return int(hipGetLastError());
+}
+
 // Per-batch extents of a dense or packed (varlen) batch.
 struct SeqInfo {
     int q_start, sq, k_start, sk;

@@ -830,12 +830,6 @@ static size_t fwd_split_bytes(const fa_fwd_args &a, int S) {
     return S > 1 ? size_t(fwd_count_bytes(items) + items * S * 128 * (8 + 4 * int64_t(a.head_dim))) : 0;
 }
 
-// Clears the splits' counters before fwd_kernel.
-__global__ void zero_counts_kernel(int32_t *count, int n) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) count[i] = 0;
-}
-
 template <int HD, bool CAUSAL>
 static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
     // The ping-pong kernel when its grid fills the chip at least twice over
@@ -896,9 +890,7 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
     if (rc || grid == 0) return rc;
     const int S = a.split_ws && a.split_ws_bytes >= int64_t(fwd_split_bytes(a, plan.splits)) ? plan.splits : 1;
     if (S > 1) {
-        hipLaunchKernelGGL(zero_counts_kernel, dim3(unsigned((grid + 255) / 256)), dim3(256), 0, stream,
-                           reinterpret_cast<int32_t *>(a.split_ws), int(grid));
-        const int rc2 = int(hipGetLastError());
+        const int rc2 = clear_counts(a.split_ws, grid, stream);
         if (rc2) return rc2;
     }
     auto go = [&](auto ng_tag, auto split_tag) {

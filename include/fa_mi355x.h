@@ -125,8 +125,8 @@ typedef struct fa_bwd_args {
     /* Optional workspace of split_ws_bytes >= fa_bwd_split_bytes(args) bytes,
      * 256-byte aligned, when that is not 0: the grid of dK/dV key blocks is too
      * small for the chip, and several workgroups then share each key block's
-     * queries and sum their fp32 partial dK / dV in it.  fa_bwd_dq or
-     * fa_bwd_preprocess clears its counters, fa_bwd_dkdv leaves them cleared.
+     * queries and sum their fp32 partial dK / dV in it.  Only dK/dV reads it, and
+     * every call clears its counters itself, whatever ran before.
      * NULL (or a smaller one) gives each key block to one workgroup. */
     void *split_ws;
     int64_t split_ws_bytes;

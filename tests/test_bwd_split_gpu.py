@@ -157,3 +157,30 @@ def test_paired_items(device, b, sq, sk, h, hk, hd):
     fa_capi.call("fa_bwd", ba)
     torch.cuda.synchronize()
     check_fwd_bwd("paired", q, k, v, do, o.cpu(), lse.cpu(), tuple(t.cpu() for t in grads), s, True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("before", ["fa_bwd_dq", "fa_bwd_preprocess"])
+def test_dkdv_clears_its_own_counters(device, before):
+    """fa_bwd_dkdv with a workspace that the call before it did not have, then once more on the same one."""
+    b, sq, sk, h, hk, hd = 1, 512, 400, 8, 2, 64
+    g = torch.Generator().manual_seed(8400)
+    q, do = randn16((b, sq, h, hd), g).to(device), randn16((b, sq, h, hd), g).to(device)
+    k, v = randn16((b, sk, hk, hd), g).to(device), randn16((b, sk, hk, hd), g).to(device)
+    print(f"case own counters before={before}", flush=True)
+    ba, o, lse, grads = _args(q, k, v, do, hd ** -0.5, True)
+    fa_capi.call(before, ba)
+    ws = _split_ws(ba, device)  # its counters hold -1
+    got = []
+    for _ in range(2):
+        for t in grads[1:]:
+            t.fill_(7.0)
+        fa_capi.call("fa_bwd_dkdv", ba)
+        torch.cuda.synchronize()
+        got.append([t.clone() for t in grads[1:]])
+    fa_capi.call(before, ba)
+    ws.zero_()
+    fa_capi.call("fa_bwd_dkdv", ba)
+    torch.cuda.synchronize()
+    for x, y, z in zip(*got, grads[1:]):
+        assert torch.equal(x, z) and torch.equal(y, z)
