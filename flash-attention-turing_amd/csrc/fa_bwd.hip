@@ -773,7 +773,7 @@ static int check_bwd(const fa_bwd_args *p) {
     const fa_bwd_args &a = *p;
     if (a.head_dim != 64 && a.head_dim != 128) return FA_ERR_UNSUPPORTED;
     if (a.batch < 0 || a.seqlen_q < 0 || a.seqlen_k < 0 || a.nheads <= 0 || a.nheads_k <= 0 ||
-        a.nheads % a.nheads_k != 0 || !a.lse || a.lse_seqlen < a.seqlen_q)
+        a.nheads % a.nheads_k != 0 || !a.lse || a.lse_seqlen < a.seqlen_q || !split_ws_aligned(a.split_ws))
         return FA_ERR_INVALID_ARG;
     if (!a.dsum) return FA_ERR_WORKSPACE;
     return FA_OK;

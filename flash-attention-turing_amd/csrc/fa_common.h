@@ -22,7 +22,19 @@
 
 #include "fa_mi355x.h"
 
+// Workgroups that share an item (the KV split kernel's fused combine, the prompt
+// chunks', the forward's and the dK/dV kernel's shares) publish their partial
+// results with relaxed agent-scope atomics and rely on gfx950's write-through of
+// agent-scope stores (the reasons stand in kv_splitkv_kernel).
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "these kernels target gfx950: shared items rely on its agent-scope store visibility"
+#endif
+
 namespace fa {
+
+// split_ws of fa_fwd_args / fa_bwd_args (or NULL): its partial results are read
+// and written as 64-bit atomics at offsets that are multiples of 256 bytes.
+inline bool split_ws_aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 255u) == 0; }
 
 // Compute units of the current device (host; fa_abi.hip).
 int device_cus();

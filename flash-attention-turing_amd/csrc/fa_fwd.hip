@@ -914,7 +914,7 @@ extern "C" int fa_fwd(const fa_fwd_args *args, void *stream) {
     const fa_fwd_args &a = *args;
     if (a.head_dim != 64 && a.head_dim != 128) return FA_ERR_UNSUPPORTED;
     if (a.batch < 0 || a.seqlen_q < 0 || a.seqlen_k < 0 || a.nheads <= 0 || a.nheads_k <= 0 ||
-        a.nheads % a.nheads_k != 0 || !a.lse || a.lse_seqlen < a.seqlen_q)
+        a.nheads % a.nheads_k != 0 || !a.lse || a.lse_seqlen < a.seqlen_q || !fa::split_ws_aligned(a.split_ws))
         return FA_ERR_INVALID_ARG;
     if (fa::check_tensor(a.q, true) || fa::check_tensor(a.k, true) || fa::check_tensor(a.v, true) ||
         fa::check_tensor(a.o, true))

@@ -42,13 +42,6 @@
 
 #include "fa_common.h"
 
-// The split kernel's fused combine publishes partials with relaxed agent-scope
-// atomics and relies on gfx950's write-through of agent-scope stores (see
-// kv_splitkv_kernel); this file is built for gfx950 only.
-#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
-#error "fa_kvcache.hip targets gfx950: its fused combine relies on gfx950's agent-scope store visibility"
-#endif
-
 namespace fa {
 
 constexpr int kKvThreads = 256;
@@ -708,7 +701,7 @@ __global__ __launch_bounds__(256, 2) void kv_splitkv_kernel(const fa_kvcache_arg
             // model (the atomics are relaxed): an agent-scope store is written
             // past the XCD's L2 before its vmcnt completes, and an agent-scope
             // load does not hit another XCD's stale L2 copy; the #error at the
-            // top of this file keeps other targets from building it.  The count
+            // top of fa_common.h keeps other targets from building it.  The count
             // of a row tile of a head group sits at its first head's slot.
             wait_vmem();
             __syncthreads();

@@ -75,7 +75,7 @@ typedef struct fa_fwd_args {
      * NULL keeps the natural order.  Results are the same either way. */
     int32_t *work_order;
     /* Optional workspace of split_ws_bytes >= fa_fwd_split_bytes(args) bytes,
-     * 256-byte aligned, when that is not 0: the grid of query blocks is too small
+     * 256-byte aligned (else FA_ERR_INVALID_ARG), when that is not 0: the grid of query blocks is too small
      * for the chip, and several workgroups then share each block's keys and sum
      * their fp32 partial results in it.  NULL (or a smaller one): one each. */
     void *split_ws;
@@ -123,7 +123,7 @@ typedef struct fa_bwd_args {
      * either way (each item is computed independently). */
     int32_t *work_order;
     /* Optional workspace of split_ws_bytes >= fa_bwd_split_bytes(args) bytes,
-     * 256-byte aligned, when that is not 0: the grid of dK/dV key blocks is too
+     * 256-byte aligned (else FA_ERR_INVALID_ARG), when that is not 0: the grid of dK/dV key blocks is too
      * small for the chip, and several workgroups then share each key block's
      * queries and sum their fp32 partial dK / dV in it.  Only dK/dV reads it, and
      * every call clears its counters itself, whatever ran before.

@@ -235,3 +235,24 @@ def test_validation_errors_before_any_launch(lib):
     assert split(ctypes.byref(kv), None) == -1  # misaligned sin table
     kv.rotary_sin, kv.rotary_seqlen = P, 0
     assert split(ctypes.byref(kv), None) == -1  # empty table
+
+
+@pytest.mark.parametrize("off", [4, 8, 128])
+def test_split_workspace_alignment(lib, off):
+    # The shares' partial results are 64-bit atomics: a workspace that is not
+    # 256-byte aligned is refused before any launch.
+    fa_capi = _capi()
+    P = 1 << 20
+    t = fa_capi.FaTensor(P, 0, 1024, 128)
+    f, b = fa_capi.FaFwdArgs(), fa_capi.FaBwdArgs()
+    f.q = f.k = f.v = f.o = t
+    b.q = b.k = b.v = b.o = b.dout = b.dq = b.dk = b.dv = t
+    b.dsum = P
+    for a, names in ((f, ("fa_fwd",)), (b, ("fa_bwd", "fa_bwd_preprocess", "fa_bwd_dq", "fa_bwd_dkdv"))):
+        a.lse = P
+        a.batch, a.seqlen_q, a.seqlen_k, a.nheads, a.nheads_k, a.head_dim, a.lse_seqlen = 1, 8, 8, 4, 2, 128, 8
+        a.split_ws, a.split_ws_bytes = P + off, 1 << 30
+        for name in names:
+            entry = getattr(lib, name)
+            entry.argtypes = [ctypes.POINTER(type(a)), ctypes.c_void_p]
+            assert entry(ctypes.byref(a), None) == -1, name
