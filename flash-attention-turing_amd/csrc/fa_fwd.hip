@@ -838,13 +838,16 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
     // blocks waste less on causal diagonals and ragged sequence ends and deal
     // out more evenly (measured varlen causal, 32 / 8 heads: 64 x 1024 rows
     // +3 %, 64 x U[64, 1024] +14 %; 32 x 2048 even; 16 x 4096 -5 %).  Both
-    // give the same bits.
+    // give the bits of one wave group, and so does the two-tile kernel below;
+    // where the plan has two, neither is taken, however large the grid is that the
+    // unpacked heads make.
+    const FwdPlan plan = fwd_plan(a);
     if constexpr (HD == 128) {
         constexpr int BM = FwdCfg<HD, 512>::BM;
         const int lg = fwd_pack_log2(a, BM), P = BM >> lg;
         const int64_t pp_m_blocks = (a.lse_seqlen + P - 1) / P;
         const int64_t pp_grid = pp_m_blocks * a.batch * (a.nheads >> lg);
-        if (pp_grid >= 2 * int64_t(device_cus()) && a.lse_seqlen >= 2048) {
+        if (plan.groups == 1 && pp_grid >= 2 * int64_t(device_cus()) && a.lse_seqlen >= 2048) {
             if (pp_grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
             const int rc = launch_order(a, int(pp_m_blocks), P, stream);
             if (rc) return rc;
@@ -861,7 +864,7 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
         const int lg = min(fwd_pack_log2(a, BM2), 2), P = BM2 >> lg;
         const int64_t m_blocks = (a.lse_seqlen + P - 1) / P;
         const int64_t grid = m_blocks * a.batch * (a.nheads >> lg);
-        if (grid >= 2 * int64_t(device_cus())) {
+        if (plan.groups == 1 && grid >= 2 * int64_t(device_cus())) {
             if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
             const int rc = launch_order(a, int(m_blocks), P, stream);
             if (rc) return rc;
@@ -870,7 +873,6 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
             return int(hipGetLastError());
         }
     }
-    const FwdPlan plan = fwd_plan(a);
     if (plan.row_waves == 2) {
         const int lg = fwd_pack_log2(a, 64), P = 64 >> lg;
         const int m_blocks = (a.lse_seqlen + P - 1) / P;

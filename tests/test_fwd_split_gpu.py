@@ -75,6 +75,36 @@ def test_fwd_shares(device, b, sq, sk, h, hk, hd, causal, split):
     assert_lse(l1.cpu(), l_ref)
 
 
+# Few queries of many heads: packed into 128-row workgroups a group's heads leave CUs idle, expanded they fill the
+# chip (in 256-row blocks at head_dim 64).  Both take the same plan.
+PACKED = [
+    (32, 16, 2048, 16, 2, 64, False, False),
+    (32, 100, 2100, 16, 4, 64, True, False),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,sq,sk,h,hk,hd,causal,split", PACKED)
+def test_packed_heads_have_the_expanded_heads_bits(device, b, sq, sk, h, hk, hd, causal, split):
+    assert (_fa(b, sq, sk, h, hk, hd, causal) > 0) == split
+    assert (_fa(b, sq, sk, h, h, hd, causal) > 0) == split
+    g = torch.Generator().manual_seed(8550 + sq + 3 * sk + h + hd)
+    q, k, v = randn16((b, sq, h, hd), g), randn16((b, sk, hk, hd), g), randn16((b, sk, hk, hd), g)
+    k[:, sk // 2:] *= 4
+    s = hd ** -0.5
+    print(f"case packed b={b} sq={sq} sk={sk} h={h} hk={hk} hd={hd} causal={causal}", flush=True)
+    qd, kd, vd = (t.to(device) for t in (q, k, v))
+    out, lse = fai._flash_attn_forward(qd, kd, vd, s, causal)
+    mha, lse_m = fai._flash_attn_forward(
+        qd, *(t.repeat_interleave(h // hk, dim=2).contiguous() for t in (kd, vd)), s, causal)
+    torch.cuda.synchronize()
+    assert torch.equal(out, mha) and torch.equal(lse, lse_m)
+    for i in (0, b - 1):
+        o_ref, l_ref = attention_fwd(q[i:i + 1], k[i:i + 1], v[i:i + 1], s, causal)
+        assert_2x("out", out[i:i + 1].cpu(), o_ref, fwd_twin(q[i:i + 1], k[i:i + 1], v[i:i + 1], s, causal)[0])
+        assert_lse(lse[i:i + 1].cpu(), l_ref)
+
+
 @pytest.mark.gpu
 def test_fwd_groups_varlen(device):
     lens_q, lens_k, h, hk, hd, s = [700, 0, 33, 512], [800, 50, 0, 500], 8, 2, 128, 128 ** -0.5
