@@ -242,67 +242,62 @@ __device__ __forceinline__ void store_row(const fa_fwd_args &a, const FwdWork &w
 // items' S x 128 rows' (maximum, sum) and their S x 128 x HD partial O in fp32.
 __host__ __device__ __forceinline__ int64_t fwd_count_bytes(int64_t items) { return (items * 4 + 255) & ~int64_t(255); }
 
-// Sums the S partial results of an item over dimension tiles [D0, D1) of O.
-// Every workgroup stores its own and then counts itself; the one that counts
-// last finds all of them stored and sums them in split order, its own from
-// registers, so no workgroup waits for another.  Returns whether this workgroup
-// holds the sum.
+// A share's partial result over dimension tiles [D0, D1) of O, in the workspace:
+// store() writes share part's, sum() adds all S of an item up in the order of the
+// shares, so the sum does not depend on who came last.  Of the n_wgs
+// workgroups that have the item's shares, each stores its own and then counts
+// itself; the one that counts last finds all of them stored, so none waits for
+// another.  live: the lane's row r is a query of the sequence (the others' results
+// are not stored).
 template <int HD, int D0, int D1>
-__device__ __forceinline__ bool fwd_merge(const fa_fwd_args &a, int64_t items, int item, int part, int S, int r,
-                                          int *ticket, f32x16 (&o)[HD / 32], float &m, float &l) {
-    constexpr int N = 8 * (D1 - D0), NT = 512;  // pairs of floats a lane holds, threads
-    const int tid = threadIdx.x, hh = (tid >> 5) & 1;
-    int32_t *count = reinterpret_cast<int32_t *>(a.split_ws) + item;
-    uint64_t *rows = reinterpret_cast<uint64_t *>(static_cast<char *>(a.split_ws) + fwd_count_bytes(items));
-    uint64_t *pairs = rows + items * S * 128 + int64_t(item) * S * N * NT + tid;
-    rows += int64_t(item) * S * 128 + r;
-    uint64_t *own = pairs + int64_t(part) * N * NT;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const f32x16 &t = o[D0 + i / 8];
-        const f32x2 x = {t[2 * (i & 7)], t[2 * (i & 7) + 1]};
-        __hip_atomic_store(own + i * NT, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+struct FwdParts {
+    static constexpr int N = 8 * (D1 - D0), NT = 512;  // pairs of floats a lane holds, threads
+    uint64_t *rows, *pairs;
+    __device__ __forceinline__ FwdParts(const fa_fwd_args &a, int64_t items, int item, int S, int thread, int r) {
+        rows = reinterpret_cast<uint64_t *>(static_cast<char *>(a.split_ws) + fwd_count_bytes(items));
+        pairs = rows + items * S * 128 + int64_t(item) * S * N * NT + thread;
+        rows += int64_t(item) * S * 128 + r;
     }
-    if (D0 == 0 && hh == 0)
-        __hip_atomic_store(rows + part * 128, __builtin_bit_cast(uint64_t, f32x2{m, l}), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    wait_vmem();
-    __syncthreads();  // every wave's stores have completed
-    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (*ticket != S - 1) return false;
-    auto row_of = [&](int p) {
-        return p == part ? f32x2{m, l}
-                         : __builtin_bit_cast(f32x2, __hip_atomic_load(rows + p * 128, __ATOMIC_RELAXED,
-                                                                       __HIP_MEMORY_SCOPE_AGENT));
-    };
-    float mx = -INFINITY, sum = 0.f;
-    for (int p = 0; p < S; ++p) mx = fmaxf(mx, row_of(p)[0]);
-    f32x16 acc[D1 - D0];
-#pragma unroll
-    for (int i = 0; i < D1 - D0; ++i) acc[i] = zero16();
-    for (int p = 0; p < S; ++p) {
-        const f32x2 ml = row_of(p);
-        const float wt = ml[0] == -INFINITY ? 0.f : exp2_fast(ml[0] - mx);
-        sum = fmaf(ml[1], wt, sum);
-        const uint64_t *slot = pairs + int64_t(p) * N * NT;
+    __device__ __forceinline__ void store(int part, bool live, int hh, const f32x16 (&o)[HD / 32], float m,
+                                          float l) const {
+        if (!live) return;
+        uint64_t *own = pairs + int64_t(part) * N * NT;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            // (The own slot is read as well, and not used.)
-            const f32x2 x = __builtin_bit_cast(
-                f32x2, __hip_atomic_load(slot + i * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
             const f32x16 &t = o[D0 + i / 8];
-            f32x16 &c = acc[i / 8];
-            c[2 * (i & 7)] = fmaf(wt, p == part ? t[2 * (i & 7)] : x[0], c[2 * (i & 7)]);
-            c[2 * (i & 7) + 1] = fmaf(wt, p == part ? t[2 * (i & 7) + 1] : x[1], c[2 * (i & 7) + 1]);
+            const f32x2 x = {t[2 * (i & 7)], t[2 * (i & 7) + 1]};
+            __hip_atomic_store(own + i * NT, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (D0 == 0 && hh == 0)
+            __hip_atomic_store(rows + part * 128, __builtin_bit_cast(uint64_t, f32x2{m, l}), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void sum(int S, f32x16 (&o)[HD / 32], float &m, float &l) const {
+        auto row_of = [&](int p) {
+            return __builtin_bit_cast(f32x2, __hip_atomic_load(rows + p * 128, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        };
+        m = -INFINITY;
+        l = 0.f;
+        for (int p = 0; p < S; ++p) m = fmaxf(m, row_of(p)[0]);
+#pragma unroll
+        for (int i = D0; i < D1; ++i) o[i] = zero16();
+        for (int p = 0; p < S; ++p) {
+            const f32x2 ml = row_of(p);
+            const float wt = ml[0] == -INFINITY ? 0.f : exp2_fast(ml[0] - m);
+            l = fmaf(ml[1], wt, l);
+            const uint64_t *slot = pairs + int64_t(p) * N * NT;
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const f32x2 x = __builtin_bit_cast(
+                    f32x2, __hip_atomic_load(slot + i * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                f32x16 &c = o[D0 + i / 8];
+                c[2 * (i & 7)] = fmaf(wt, x[0], c[2 * (i & 7)]);
+                c[2 * (i & 7) + 1] = fmaf(wt, x[1], c[2 * (i & 7) + 1]);
+            }
         }
     }
-#pragma unroll
-    for (int i = 0; i < D1 - D0; ++i) o[D0 + i] = acc[i];
-    m = mx;
-    l = sum;
-    return true;
-}
+};
 
 // Copies of K / V block nb into an LDS tile by all NT threads.  A block that
 // runs past the sequence re-reads its last key for the missing rows (masked).
@@ -343,11 +338,14 @@ struct KvLoader {
 // CU.  The per-tile arithmetic is the same, so the results are the same bits.
 // NG = 2: two groups of RW waves (RW = 4: 128 rows, 2: 64 rows) over the same rows
 // take the key blocks in turn, each through its own LDS stages, and merge their
-// results through LDS at the end.  SPLIT: S workgroups per query block do the same and merge through
-// split_ws.  A block's place in that order depends on its key position alone.
+// results through LDS at the end.  SPLIT: a query block's key blocks are dealt out to S shares, each
+// walked as above, and the shares' results merge through split_ws; L of them, one after another, are
+// one workgroup's (1 where the grid then still has a CU for each, so the sum is the same for a GQA
+// group packed into a few workgroups and for its expanded heads in many).  A block's place in that
+// order depends on its key position alone.
 template <int HD, bool CAUSAL, int QT, int NG, int RW, bool SPLIT>
 __global__ __launch_bounds__(64 * RW * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 2 : 3) void fwd_kernel(
-    const fa_fwd_args a, const int num_m_blocks, const int lg, const int S) {
+    const fa_fwd_args a, const int num_m_blocks, const int lg, const int S, const int L) {
     constexpr int NT = 256;        // threads that copy a tile together
     constexpr int GT = 64 * RW;    // threads of a wave group
     static_assert(QT == 1 || NG == 1, "two groups: one tile per wave");
@@ -365,9 +363,11 @@ __global__ __launch_bounds__(64 * RW * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 
     const int hh = lane >> 5;
     FwdWork w;
     const int bp_count = a.batch * (a.nheads >> lg);
-    const int unit = SPLIT ? blockIdx.x / bp_count : 0;  // SPLIT: the S shares of a block of positions in turn
-    const int part = SPLIT ? unit % S : 0;
-    const int bid = SPLIT ? unit / S * bp_count + (blockIdx.x - unit * bp_count) : blockIdx.x;
+    const int unit = SPLIT ? blockIdx.x / bp_count : 0;  // SPLIT: the workgroups of a block of positions in turn
+    const int n_wgs = SPLIT ? (S + L - 1) / L : 1;       // ... n_wgs of them
+    int part = SPLIT ? unit % n_wgs * L : 0;             // the workgroup's shares: [part, part_end)
+    const int part_end = SPLIT ? min(S, part + L) : 1;
+    const int bid = SPLIT ? unit / n_wgs * bp_count + (blockIdx.x - unit * bp_count) : blockIdx.x;
     if (!fwd_work<BM, CAUSAL>(a, num_m_blocks, lg, bid, w)) return;
 
     // The wave's tiles QT * wave + t: one head (the launcher packs at most BM / 64 heads when QT = 2,
@@ -394,7 +394,7 @@ __global__ __launch_bounds__(64 * RW * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 
     KvLoader<HD, NT> ld;
     ld.init(a, RW == 4 ? wave : wave8, lane);
     const int part_step = SPLIT ? S : 1, step = NG * part_step;  // of the workgroup's blocks and of the group's
-    const int nb0 = part + part_step * grp;                      // the group's first block
+    int nb0 = part + part_step * grp;                            // the group's first block
     // Copies of the group's block nb into stage st; with two row waves a group,
     // all four waves copy the blocks of both groups.
     auto issue = [&](int nb, int st) FA_INLINE {
@@ -502,59 +502,95 @@ __global__ __launch_bounds__(64 * RW * NG, NG == 2 ? 1 : QT == 2 || HD == 128 ? 
     // is below the sequence end and at or below the diagonal of the first query.
     int n_full = min(w.n_blocks, w.sk / BN);
     if (CAUSAL) n_full = min(n_full, max(0, (w.m0 + w.causal_off + 1) / BN));
-    // Iterations in which every group has a block, and one without a mask.
-    const int last0 = nb0 - part_step * grp + part_step * (NG - 1);  // the last group's first block
-    issue(nb0, 0);
-    const int it_full = n_full > last0 ? (n_full - 1 - last0) / step + 1 : 0;
-    const int n_it = w.n_blocks > part ? (w.n_blocks - 1 - part) / step + 1 : 0;
-    for (int it = 0; it < it_full; ++it) block(it, std::false_type{});
-    for (int it = it_full; it < n_it; ++it) block(it, std::true_type{});
-    if constexpr (NG == 1) {
+    const int64_t items = num_m_blocks * bp_count;  // SPLIT: workgroups of the unsplit grid, and this one's
+    const int item = (w.b * (a.nheads >> lg) + (w.h >> lg)) * num_m_blocks + w.m0 / w.P;
+    for (;;) {
+        // Iterations in which every group has a block, and one without a mask.
+        const int last0 = nb0 - part_step * grp + part_step * (NG - 1);  // the last group's first block
+        issue(nb0, 0);
+        const int it_full = n_full > last0 ? (n_full - 1 - last0) / step + 1 : 0;
+        const int n_it = w.n_blocks > part ? (w.n_blocks - 1 - part) / step + 1 : 0;
+        for (int it = 0; it < it_full; ++it) block(it, std::false_type{});
+        for (int it = it_full; it < n_it; ++it) block(it, std::true_type{});
+        if constexpr (NG == 1) {
 #pragma unroll
-        for (int t = 0; t < QT; ++t) store_row<HD, 0, HD / 32>(a, w, qi[t], hh, o[t], row[t].m_t, sum_xor32(row[t].l_p));
-    } else {
-        // Each group finishes half of the head's dimensions: it hands the other
-        // half of its O, and its maxima and sums, to the other group.
-        constexpr int H = HD / 64;  // 32-wide dimension tiles of a half
-        const int t4 = tid & (GT - 1), r = 32 * wave + (lane & 31);
-        const float l_own = sum_xor32(row[0].l_p), m_own = row[0].m_t;
-        f32x4 *xo = reinterpret_cast<f32x4 *>(smem);                        // [group][4 H][GT threads]
-        f32x2 *xr = reinterpret_cast<f32x2 *>(smem + 2 * 4 * H * GT * 16);  // [group][BM rows]
-        __syncthreads();  // every wave is done with the tiles
-        if (hh == 0) xr[grp * BM + r] = f32x2{m_own, l_own};
-        auto finish = [&](auto grp_tag) FA_INLINE {
-            constexpr int GRP = decltype(grp_tag)::value;
+            for (int t = 0; t < QT; ++t)
+                store_row<HD, 0, HD / 32>(a, w, qi[t], hh, o[t], row[t].m_t, sum_xor32(row[t].l_p));
+        } else {
+            // Each group finishes half of the head's dimensions: it hands the other
+            // half of its O, and its maxima and sums, to the other group.
+            constexpr int H = HD / 64;  // 32-wide dimension tiles of a half
+            int t4 = tid & (GT - 1), r = 32 * wave + (lane & 31);
+            // SPLIT: opaque to the optimiser, so that the addresses below are formed
+            // here and not held through the next share's block loop.
+            if constexpr (SPLIT) asm volatile("" : "+v"(t4), "+v"(r));
+            const float l_own = sum_xor32(row[0].l_p), m_own = row[0].m_t;
+            f32x4 *xo = reinterpret_cast<f32x4 *>(smem);                        // [group][4 H][GT threads]
+            f32x2 *xr = reinterpret_cast<f32x2 *>(smem + 2 * 4 * H * GT * 16);  // [group][BM rows]
+            __syncthreads();  // every wave is done with the tiles
+            if (hh == 0) xr[grp * BM + r] = f32x2{m_own, l_own};
+            auto finish = [&](auto grp_tag) FA_INLINE {
+                constexpr int GRP = decltype(grp_tag)::value;
 #pragma unroll
-            for (int i = 0; i < 4 * H; ++i) {
-                const f32x16 &t = o[0][(1 - GRP) * H + i / 4];
-                xo[(GRP * 4 * H + i) * GT + t4] = f32x4{t[4 * (i & 3)], t[4 * (i & 3) + 1], t[4 * (i & 3) + 2],
-                                                         t[4 * (i & 3) + 3]};
-            }
+                for (int i = 0; i < 4 * H; ++i) {
+                    const f32x16 &t = o[0][(1 - GRP) * H + i / 4];
+                    xo[(GRP * 4 * H + i) * GT + t4] = f32x4{t[4 * (i & 3)], t[4 * (i & 3) + 1], t[4 * (i & 3) + 2],
+                                                             t[4 * (i & 3) + 3]};
+                }
+                __syncthreads();
+                const f32x2 other = xr[(1 - GRP) * BM + r];
+                float m = fmaxf(m_own, other[0]);
+                const float a_own = m_own == -INFINITY ? 0.f : exp2_fast(m_own - m);
+                const float a_other = other[0] == -INFINITY ? 0.f : exp2_fast(other[0] - m);
+#pragma unroll
+                for (int i = 0; i < 4 * H; ++i) {
+                    const f32x4 x = xo[((1 - GRP) * 4 * H + i) * GT + t4];
+                    f32x16 &t = o[0][GRP * H + i / 4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) t[4 * (i & 3) + e] = fmaf(x[e], a_other, t[4 * (i & 3) + e] * a_own);
+                }
+                // In group order, so that both groups have the same bits.
+                float l = GRP == 0 ? fmaf(other[1], a_other, l_own * a_own) : fmaf(l_own, a_own, other[1] * a_other);
+                if constexpr (SPLIT)
+                    FwdParts<HD, GRP * H, GRP * H + H>(a, items, item, S, GRP * GT + t4, r)
+                        .store(part, qi[0] < w.sq, hh, o[0], m, l);
+                else
+                    store_row<HD, GRP * H, GRP * H + H>(a, w, qi[0], hh, o[0], m, l);
+            };
+            if (grp == 0)
+                finish(std::integral_constant<int, 0>{});
+            else
+                finish(std::integral_constant<int, 1>{});
+        }
+        if (!SPLIT || ++part == part_end) break;
+        // The next share, from the start.
+        ++nb0;
+#pragma unroll
+        for (int i = 0; i < HD / 32; ++i) o[0][i] = zero16();
+        row[0] = SoftmaxRow();
+        __syncthreads();  // every wave has read what the groups exchanged
+    }
+    if constexpr (SPLIT) {
+        wait_vmem();
+        __syncthreads();  // every wave's stores have completed
+        if (n_wgs > 1) {
+            if (tid == 0)
+                ticket = __hip_atomic_fetch_add(reinterpret_cast<int32_t *>(a.split_ws) + item, 1, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
             __syncthreads();
-            const f32x2 other = xr[(1 - GRP) * BM + r];
-            float m = fmaxf(m_own, other[0]);
-            const float a_own = m_own == -INFINITY ? 0.f : exp2_fast(m_own - m);
-            const float a_other = other[0] == -INFINITY ? 0.f : exp2_fast(other[0] - m);
-#pragma unroll
-            for (int i = 0; i < 4 * H; ++i) {
-                const f32x4 x = xo[((1 - GRP) * 4 * H + i) * GT + t4];
-                f32x16 &t = o[0][GRP * H + i / 4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) t[4 * (i & 3) + e] = fmaf(x[e], a_other, t[4 * (i & 3) + e] * a_own);
-            }
-            // In group order, so that both groups have the same bits.
-            float l = GRP == 0 ? fmaf(other[1], a_other, l_own * a_own) : fmaf(l_own, a_own, other[1] * a_other);
-            if constexpr (SPLIT) {
-                const int item = (w.b * (a.nheads >> lg) + (w.h >> lg)) * num_m_blocks + w.m0 / w.P;
-                if (!fwd_merge<HD, GRP * H, GRP * H + H>(a, num_m_blocks * bp_count, item, part, S, r, &ticket, o[0], m, l))
-                    return;
-            }
-            store_row<HD, GRP * H, GRP * H + H>(a, w, qi[0], hh, o[0], m, l);
+            if (ticket != n_wgs - 1) return;
+        }
+        auto sum = [&](auto grp_tag) FA_INLINE {
+            constexpr int D0 = decltype(grp_tag)::value * (HD / 64), D1 = D0 + HD / 64;
+            float m = 0.f, l = 0.f;
+            if (qi[0] < w.sq)
+                FwdParts<HD, D0, D1>(a, items, item, S, tid, 32 * wave + (lane & 31)).sum(S, o[0], m, l);
+            store_row<HD, D0, D1>(a, w, qi[0], hh, o[0], m, l);
         };
         if (grp == 0)
-            finish(std::integral_constant<int, 0>{});
+            sum(std::integral_constant<int, 0>{});
         else
-            finish(std::integral_constant<int, 1>{});
+            sum(std::integral_constant<int, 1>{});
     }
 }
 
@@ -774,60 +810,97 @@ static int fwd_pack_log2(const fa_fwd_args &a, int BM) {
     return lg;
 }
 
-// How fwd_kernel runs: row waves per wave group (32 rows each), wave groups per
-// workgroup and workgroups (splits) per query block.  W: 128-row blocks (counted
-// in 32-row tiles, so that a GQA group packed into workgroups and its expanded
-// heads get the same plan and bits), NB: key blocks of the longest row.  Measured
-// on MI355X, us at one group of 4 row waves -> as planned (row waves x groups x
-// splits), head_dim 128 unless noted:
+// Causal calls whose longest row sees at most twice the average row's keys or so
+// (queries over at most as many earlier keys again), and those of a square.
+static bool causal_near(const fa_fwd_args &a) { return a.causal && a.seqlen_k <= 2 * int64_t(a.seqlen_q); }
+static bool causal_square(const fa_fwd_args &a) {
+    return a.causal && 10 * int64_t(a.seqlen_k) <= 11 * int64_t(a.seqlen_q);
+}
+
+// How the keys of a query block are shared: wave groups per workgroup and shares
+// (splits) per query block.  A group rounds P to fp16 against its own running
+// maximum, so a row's bits depend on this plan, and with it on batch, heads and
+// lengths.  They must not depend on how many heads share a workgroup (a GQA group
+// gives the bits of its expanded heads), so the rules count work that packing does
+// not change: W, 128-row blocks in 32-row tiles (what the packed heads of short
+// calls fill), and the 128- and 64-row blocks of unpacked heads (U, U64), the most
+// workgroups that any form of the call launches.  NB: key blocks of the longest row.
+// Measured on MI355X, us at one group of 4 row waves -> as planned (row waves x
+// groups x splits), head_dim 128 unless noted:
 //   one workgroup per CU leaves each SIMD one wave; a second group halves the
 //   chain of key blocks (1.82 us for a pair of blocks against 2 x 1.22):
-//     b1 s1024 32/8 causal (W 256): 26.9 -> 23.9 (4 x 2 x 1)   s2048 16/16: 45.7 -> 38.3
-//     b1 s4096 16/16 causal (W 512): 104 -> 89                 1024 x 16384 keys 32/8: 328 -> 294
-//   it loses when two workgroups per CU fill the chip without a mask (W 512,
-//   s4096: 153 -> 159), on short chains (W 256, s256: 11.8 -> 12.3) and past W 512
-//   (W 768, s2048: 74.5 -> 82);
-//   where half of the CUs would idle, two groups of 2 row waves use them all and
-//   read half as much LDS a CU (1.58 us a pair; 0.9 at head_dim 64):
-//     b1 s509 32/8 causal (W 128): 16.7 -> 13.5 (2 x 2 x 1)    s256: 11.5 -> 9.7
-//     b1 s700 32/8 causal (W 176): 20.9 -> 18.1                s1024 8/8 no mask: 25.7 -> 19.7
-//     d64 b1 s2048 16/16 causal (W 256): 35.1 -> 24.6          b4 s512 no mask: 12.8 -> 11.9
-//   not at W 256 at head_dim 128 (s1024 32/8: 23.9 -> 26.8), nor on long unmasked
-//   chains there (d64 b1 s2048: 29.3 -> 32.9);
+//     b1 s1024 32/8 causal (W 256): 28.3 -> 25.7 (4 x 2 x 1)   s2048 16/16: 45.7 -> 38.3
+//     b1 s4096 16/16 causal (W 512): 110 -> 93                 1024 x 16384 keys 32/8: 328 -> 294
+//   a workgroup of two groups has a CU to itself, so it loses where one-group ones
+//   would share CUs: without a causal square (W 512, s4096 no mask: 153 -> 159;
+//   256 x 4000 keys: 177 -> 208; 1024 x 2048 causal: 69 -> 72), past W 512 (W 768,
+//   s2048: 74.5 -> 82) and for unpacked heads of few queries (b16 32/32, 64 x 1300:
+//   69 -> 77; b32 16/16, 16 x 1400: 69 -> 75); and on short chains (W 256, s256:
+//   11.8 -> 12.3; one block: 5.0 -> 5.5);
 //   with CUs still idle and long chains, splits take them (one launch to clear the
 //   counters and a merge: about 8 us, 2 more per split):
 //     512 rows x 16384 keys 32/8: 311 -> 160 (4 x 2 x 2)       128 rows: 309 -> 60 (4 x 2 x 8)
 //     512 x 8192 16/4 d64: 127 -> 38 (4 x 2 x 4)
+//   and where heads do not pack, their workgroups walk the same shares in turn: 16
+//     queries x 8000 keys b8: 32/8 159 -> 61 (4 x 2 x 4), 32/32 188 -> 200
 struct FwdPlan {
-    int row_waves, groups, splits;
+    int groups, splits;
 };
 static FwdPlan fwd_plan(const fa_fwd_args &a) {
-    const int64_t W = (int64_t(a.batch) * a.nheads * ((int64_t(a.lse_seqlen) + 31) / 32) + 3) / 4, cus = device_cus();
+    const int64_t heads = int64_t(a.batch) * a.nheads, len = a.lse_seqlen, cus = device_cus();
+    const int64_t W = (heads * ((len + 31) / 32) + 3) / 4, U = heads * ((len + 127) / 128), U64 = heads * ((len + 63) / 64);
     const int NB = (a.seqlen_k + kFwdBN - 1) / kFwdBN;
-    FwdPlan plan = {4, 1, 1};
-    if (2 * W <= cus ? NB >= 8 : W <= cus ? NB >= 12 : W <= 2 * cus && a.causal && NB >= 32) plan.groups = 2;
-    const bool narrow = 2 * W <= cus || (a.head_dim == 64 ? W <= cus && (a.causal || NB <= 16) : 4 * W <= 3 * cus && a.causal);
-    if (a.cu_seqlens_q || !narrow) return plan;  // varlen work orders list 128-row blocks
-    plan = {2, 2, 1};
+    const bool half = 2 * W <= cus;  // half of the CUs would idle
+    // The least key blocks for two groups (64-row blocks, fwd_narrow, pay from 2 on).
+    const int least = half                ? !a.cu_seqlens_q && U64 <= cus ? 2 : 8
+                      : a.head_dim == 64 ? (causal_near(a) ? 6 : 8)
+                                         : (causal_near(a) ? 9 : 12);
+    FwdPlan plan = {1, 1};
+    if (W <= cus ? 2 * U <= 3 * cus && NB >= least : W <= 2 * cus && causal_square(a) && NB >= 32) plan.groups = 2;
+    if (!half || plan.groups == 1 || a.cu_seqlens_q) return plan;  // varlen: the work order lists unsplit blocks
     const double pairs = 0.5 * NB, unit = a.head_dim == 128 ? 1.84 : 1.31;
-    double best = pairs * (a.head_dim == 128 ? 1.58 : 0.9);
+    const double unsplit = pairs * (a.head_dim == 128 ? 1.58 : 0.9);
+    double best = unsplit;
     for (int S = 2; S <= 16 && W * S <= cus; ++S) {
         const double t = pairs / S * unit + 6 + 2 * S;
         if (t < best) {
             best = t;
-            plan = {4, 2, S};
+            plan.splits = S;
         }
     }
+    // Where the unpacked form of the call fills the chip by itself, it takes the
+    // shares one after another and gains nothing: only where they halve the packed
+    // form's time.
+    if (U >= cus && best > 0.5 * unsplit) plan.splits = 1;
     return plan;
 }
-// Workgroups of the unsplit 128-row grid.
-static int64_t fwd_items(const fa_fwd_args &a) {
-    const int lg = fwd_pack_log2(a, 128), P = 128 >> lg;
+// Workgroups of the unsplit grid of BM-row blocks.
+static int64_t fwd_items(const fa_fwd_args &a, int BM) {
+    const int lg = fwd_pack_log2(a, BM), P = BM >> lg;
     return int64_t((a.lse_seqlen + P - 1) / P) * a.batch * (a.nheads >> lg);
 }
 static size_t fwd_split_bytes(const fa_fwd_args &a, int S) {
-    const int64_t items = fwd_items(a);
+    const int64_t items = fwd_items(a, 128);
     return S > 1 ? size_t(fwd_count_bytes(items) + items * S * 128 * (8 + 4 * int64_t(a.head_dim))) : 0;
+}
+
+// Whether the two wave groups of an unsplit dense call have 2 row waves each
+// (64-row blocks) instead of 4: the same bits, read half as much LDS a workgroup
+// (1.58 us a pair of blocks against 1.82; 0.9 against 1.31 at head_dim 64), so they
+// win where their grid still has a CU for each workgroup, and a little past that
+// where a causal square's later workgroups are short.  Measured on MI355X, us in
+// 128-row -> 64-row blocks (workgroups of the latter), head_dim 128 unless noted:
+//   b1 s509 32/8 causal (256): 15.4 -> 13.5       b1 s1024 16/2 causal (256): 23.7 -> 21.3
+//   b1 s1200 16/2 causal (304): 26.7 -> 25.1      b1 s700 32/8 causal (352): 18.6 -> 18.1
+//   b2 s350 32/8 causal (352): 14.5 -> 16.6       700 x 1050 keys causal (352): 26.3 -> 29.9
+//   b1 s2048 8/8 causal (512): 41.8 -> 44.8       b4 200 x 8000 keys 32/4 (448): 144 -> 237
+//   d64 b2 s2048 8/8 causal (512): 29.7 -> 26.7   d64 1024 x 2048 keys causal (512): 30.6 -> 29.9
+//   d64 2048 x 6144 keys causal (512): 77 -> 79   d64 256 x 1024 keys no mask (384): 18.0 -> 19.1
+static bool fwd_narrow(const fa_fwd_args &a) {
+    const int64_t n = fwd_items(a, 64), cus = device_cus();
+    if (n <= cus) return true;
+    if (a.head_dim == 64) return n <= 2 * cus && causal_near(a);
+    return 2 * n <= 3 * cus && causal_square(a) && a.seqlen_k > 9 * kFwdBN;
 }
 
 template <int HD, bool CAUSAL>
@@ -869,18 +942,19 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
             const int rc = launch_order(a, int(m_blocks), P, stream);
             if (rc) return rc;
             hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 2, 1, 4, false>), dim3(unsigned(grid)), dim3(256), 0, stream, a,
-                               int(m_blocks), lg, 1);
+                               int(m_blocks), lg, 1, 1);
             return int(hipGetLastError());
         }
     }
-    if (plan.row_waves == 2) {
+    const int S = a.split_ws && a.split_ws_bytes >= int64_t(fwd_split_bytes(a, plan.splits)) ? plan.splits : 1;
+    if (plan.groups == 2 && S == 1 && !a.cu_seqlens_q && fwd_narrow(a)) {
         const int lg = fwd_pack_log2(a, 64), P = 64 >> lg;
         const int m_blocks = (a.lse_seqlen + P - 1) / P;
         const int64_t grid = int64_t(m_blocks) * a.batch * (a.nheads >> lg);
         if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
         if (grid == 0) return FA_OK;
         hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 1, 2, 2, false>), dim3(unsigned(grid)), dim3(256), 0, stream, a,
-                           m_blocks, lg, 1);
+                           m_blocks, lg, 1, 1);
         return int(hipGetLastError());
     }
     constexpr int BM = FwdCfg<HD, 256>::BM;
@@ -890,15 +964,19 @@ static int launch_fwd(const fa_fwd_args &a, hipStream_t stream) {
     if (grid > 0x7fffffff) return FA_ERR_INVALID_ARG;
     const int rc = launch_order(a, num_m_blocks, P, stream);
     if (rc || grid == 0) return rc;
-    const int S = a.split_ws && a.split_ws_bytes >= int64_t(fwd_split_bytes(a, plan.splits)) ? plan.splits : 1;
-    if (S > 1) {
+    // Shares that a workgroup takes one after another: few enough workgroups for
+    // one CU each (b32 8/8, 2 x 8000 keys, 256 blocks x 4 shares: 240 us in 1024
+    // workgroups, 216 in 256, 189 without shares).
+    int L = 1;
+    while (L < S && grid * ((S + L - 1) / L) > device_cus()) ++L;
+    if (L < S) {  // several workgroups a block: they count
         const int rc2 = clear_counts(a.split_ws, grid, stream);
         if (rc2) return rc2;
     }
     auto go = [&](auto ng_tag, auto split_tag) {
         constexpr int NG = decltype(ng_tag)::value;
-        hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 1, NG, 4, decltype(split_tag)::value>), dim3(unsigned(grid * S)),
-                           dim3(256 * NG), 0, stream, a, num_m_blocks, lg, S);
+        hipLaunchKernelGGL((fwd_kernel<HD, CAUSAL, 1, NG, 4, decltype(split_tag)::value>),
+                           dim3(unsigned(grid * ((S + L - 1) / L))), dim3(256 * NG), 0, stream, a, num_m_blocks, lg, S, L);
     };
     using G1 = std::integral_constant<int, 1>;
     using G2 = std::integral_constant<int, 2>;

@@ -76,10 +76,15 @@ def test_fwd_shares(device, b, sq, sk, h, hk, hd, causal, split):
 
 
 # Few queries of many heads: packed into 128-row workgroups a group's heads leave CUs idle, expanded they fill the
-# chip (in 256-row blocks at head_dim 64).  Both take the same plan.
+# chip (in 256-row blocks at head_dim 64).  Both take the same plan, one group, two, or shares, which the expanded form's
+# workgroups walk several of in turn (all of them; two of three or four).
 PACKED = [
     (32, 16, 2048, 16, 2, 64, False, False),
     (32, 100, 2100, 16, 4, 64, True, False),
+    (16, 64, 1300, 32, 8, 128, True, False),
+    (16, 2, 6500, 16, 4, 128, False, True),
+    (8, 33, 4100, 16, 2, 128, True, True),
+    (4, 150, 4000, 16, 4, 64, True, True),
 ]
 
 
