@@ -1096,12 +1096,29 @@ static int check_kv(const fa_kvcache_args *p) {
     return FA_OK;
 }
 
+// Whether many query rows (tiles of 128 rows over all sequences and KV heads) are
+// kv_chunk_kernel's: there are enough tiles that few splits fill the chip, or few
+// keys to split.  Otherwise (one or two KV heads, few sequences, long caches) it
+// needs more splits than one workgroup merges quickly, and kv_splitkv_kernel's four
+// waves share a tile's keys besides.  Measured on MI355X, us a call at each kernel's
+// best splits up to 16, split kernel -> this one (tiles):
+//   64/1 heads, 1 token, 5.5k keys (1): 39 -> 53       128/1, 1 x 210k (1): 141 -> 351
+//   32/2, 8 tokens, 7.8k (2): 38 -> 48                 b4 8/1, 16 x 63k (4): 60 -> 101
+//   32/8, 16 x 18k (8): 52 -> 60                       b1 64/4, 9 x 20k (8): 62 -> 71
+//   head_dim 64 32/8, 32 x 12k (8): 41 -> 44           16 tiles, > 16k keys: 1.2x faster
+//   17 - 32 tiles: 1.2 - 1.9x faster                   up to 4k keys: 1.03 - 1.57x faster
+static bool chunk_fills(int64_t tiles, int num_cus) { return 16 * tiles > std::max(num_cus, 1); }
+static bool chunk_pays(int64_t tiles, int64_t keys, int num_cus) {
+    return chunk_fills(tiles, num_cus) || (keys > 0 && keys <= 4096);
+}
+
 // Splits of the many-row kernel: the fewest key blocks on the busiest CU (a CU
 // with one workgroup is about 10 % slower per block) and 1.3 blocks' time for
 // every split to merge.  Measured on MI355X with 32 / 8 heads, head_dim 128, us
 // per call at 1 split -> the splits taken: 512 rows x 1 sequence of 8k keys
 // 226 -> 128 (4 splits), 128 x 1 x 8k 214 -> 59 (8), 32 x 8 x 8k 215 -> 82 (4),
-// 1024 x 1 x 15k 444 -> 410 (2).
+// 1024 x 1 x 15k 444 -> 410 (2).  At most 16: with the tiles that chunk_pays asks
+// for, that many fill the chip.
 static int chunk_num_splits(int64_t heads, int rows, int capacity, int num_cus) {
     const int64_t tiles = heads * ((rows + kChunkRows - 1) / kChunkRows), cus = std::max(num_cus, 1);
     const double blocks = (double(capacity) + kChunkKeys - 1) / kChunkKeys;
@@ -1138,7 +1155,9 @@ extern "C" int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_d
     if (requested > 0) return requested;
     if (batch <= 0 || nheads_k <= 0 || nheads <= 0 || seqlen_k_capacity <= 0) return 1;
     const int rows = (nheads / nheads_k) * seqlen_q;
-    if (rows >= fa::kChunkMinRows) return fa::chunk_num_splits(int64_t(batch) * nheads_k, rows, seqlen_k_capacity, num_cus);
+    const int64_t tiles = int64_t(batch) * nheads_k * ((rows + fa::kChunkRows - 1) / fa::kChunkRows);
+    if (rows >= fa::kChunkMinRows && fa::chunk_pays(tiles, seqlen_k_capacity, num_cus))
+        return fa::chunk_num_splits(int64_t(batch) * nheads_k, rows, seqlen_k_capacity, num_cus);
     const int64_t wgs = int64_t(batch) * nheads_k * ((rows + 31) / 32);
     const int64_t by_len = (int64_t(seqlen_k_capacity) + 4096) / 8192;
     const int64_t by_fill = (int64_t(std::max(num_cus, 1)) + wgs - 1) / std::max<int64_t>(wgs, 1);
@@ -1214,22 +1233,31 @@ int kv_heads_per_item(const fa_kvcache_args &a) {
     return hpi;
 }
 
+int64_t chunk_tiles(const fa_kvcache_args &a) {
+    return int64_t(a.batch) * a.nheads_k * (((a.nheads / a.nheads_k) * a.seqlen_q + kChunkRows - 1) / kChunkRows);
+}
+int64_t chunk_items(const fa_kvcache_args &a) { return chunk_tiles(a) * a.num_splits; }
+
 // Whether the split kernel of a call is kv_chunk_kernel: at least 64 query rows
 // per KV head (with 64 rows, 8 sequences of 8k keys, 32 / 8 heads: 71 us against
-// 114 at the best split counts; one sequence 50 against 49; with 32 rows the
-// other kernel reads K and V once as well and its waves share the keys), few
-// enough splits for one workgroup to merge, and the split counts to do it with.
-// Its 64-key blocks must not straddle pages, and its page ids fit in LDS.
+// 114 at the best split counts; with 32 rows the other kernel reads K and V once as
+// well and its waves share the keys) in enough tiles (chunk_pays; with softcap or
+// ALiBi, whose scores cost more arithmetic than the shared loads save, a short cache
+// is not reason enough: b1 8/1 304 rows x 3k keys 35 -> 42 us), few enough splits
+// for one workgroup to merge, and the split counts to do it with.  Its 64-key blocks
+// must not straddle pages, and its page ids fit in LDS.
 bool use_chunk(const fa_kvcache_args &a) {
     const int R = (a.nheads / a.nheads_k) * a.seqlen_q;
     if (R < kChunkMinRows || a.num_splits > kChunkMaxSplits || !a.batch_order || (a.num_splits > 1 && !a.split_count))
         return false;
+    // A left window leaves so many keys, as the caller's split count takes them.
+    int64_t keys = a.cache_capacity;
+    if (a.local_window && a.window_left >= 0) keys = std::min<int64_t>(keys, int64_t(a.window_left) + 1 + a.seqlen_q);
+    const bool natural = a.softcap > 0.f || a.alibi_slopes;
+    if (!(natural ? chunk_fills(chunk_tiles(a), device_cus()) : chunk_pays(chunk_tiles(a), keys, device_cus())))
+        return false;
     return !a.block_table || (a.page_block_size % kChunkKeys == 0 && a.cache_capacity > 0 &&
                               a.cache_capacity / a.page_block_size <= kChunkPages);
-}
-int64_t chunk_items(const fa_kvcache_args &a) {
-    const int row_tiles = ((a.nheads / a.nheads_k) * a.seqlen_q + kChunkRows - 1) / kChunkRows;
-    return int64_t(a.batch) * a.nheads_k * row_tiles * a.num_splits;
 }
 
 // Whether the split kernel's items come in the order of batch_order: there are

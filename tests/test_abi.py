@@ -256,3 +256,18 @@ def test_split_workspace_alignment(lib, off):
             entry = getattr(lib, name)
             entry.argtypes = [ctypes.POINTER(type(a)), ctypes.c_void_p]
             assert entry(ctypes.byref(a), None) == -1, name
+
+
+def test_num_splits_many_rows(lib):
+    # From 64 query rows per KV head on, the many-row kernel's count (at most 16) where its 128-row tiles are many
+    # enough (more than a sixteenth of the CUs) or the keys few; else the split kernel's, which fills the chip.
+    f = lib.fa_kv_num_splits
+    for (cap, d, sq, b, h, hk), least in {
+        (131072, 128, 1, 1, 64, 1): 32,  # one tile
+        (65536, 128, 4, 1, 32, 2): 32,  # two
+        (131072, 64, 16, 1, 32, 8): 16,  # eight
+    }.items():
+        assert f(0, cap, d, sq, b, h, hk, 256) >= least
+        assert f(0, 4096, d, sq, b, h, hk, 256) <= 16
+    assert f(0, 131072, 128, 16, 4, 32, 8, 256) <= 16  # 32 tiles
+    assert f(0, 300000, 128, 512, 2, 32, 8, 256) <= 2  # 256 tiles
