@@ -908,14 +908,18 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcach
             qB[g] = as_h8(v);
         }
     }
-    // Page ids of the walked keys (the launcher takes this kernel only when they fit).
+    // Page ids of the walked keys, kChunkPages of them at a time: those from block
+    // nb's page on, which serve the blocks below nb_staged.
     const int page = a.page_block_size;
-    const int pg0 = a.block_table ? nb0 * BN / page : 0;
-    if (a.block_table && nb1 > nb0) {
+    int pg0 = 0, nb_staged = nb1;
+    auto stage_pages = [&](int nb) {
+        pg0 = nb * BN / page;
         const int32_t *bt = a.block_table + int64_t(b) * a.block_table_stride + pg0;
-        const int n_pages = (nb1 * BN - 1) / page - pg0 + 1;
+        const int n_pages = min(kChunkPages, (nb1 * BN - 1) / page - pg0 + 1);
         for (int i = tid; i < n_pages; i += kKvThreads) pages[i] = bt[i];
-    }
+        nb_staged = int(min(int64_t(nb1), int64_t(pg0 + kChunkPages) * (page / BN)));
+    };
+    if (a.block_table && nb1 > nb0) stage_pages(nb0);
     wait_vmem();  // only the tile copies are in flight in the loop
     __syncthreads();
 
@@ -949,7 +953,13 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcach
     for (int nb = nb0; nb < nb1; ++nb) {
         wait_vmem();
         __syncthreads();  // block nb is in LDS; every wave is done with the other stage
-        if (nb + 1 < nb1) issue(nb + 1);
+        if (nb + 1 < nb1) {
+            if (nb + 1 >= nb_staged) {
+                stage_pages(nb + 1);  // (every wave has read the ids of the blocks up to nb)
+                __syncthreads();
+            }
+            issue(nb + 1);
+        }
         const int p0 = nb * BN;
         if (p0 >= any_hi || p0 + BN <= any_lo) continue;  // no key for this wave
         // The lane's read bases with this block's stage added (opaque, so the
@@ -1097,19 +1107,23 @@ static int check_kv(const fa_kvcache_args *p) {
 }
 
 // Whether many query rows (tiles of 128 rows over all sequences and KV heads) are
-// kv_chunk_kernel's: there are enough tiles that few splits fill the chip, or few
-// keys to split.  Otherwise (one or two KV heads, few sequences, long caches) it
-// needs more splits than one workgroup merges quickly, and kv_splitkv_kernel's four
-// waves share a tile's keys besides.  Measured on MI355X, us a call at each kernel's
-// best splits up to 16, split kernel -> this one (tiles):
-//   64/1 heads, 1 token, 5.5k keys (1): 39 -> 53       128/1, 1 x 210k (1): 141 -> 351
+// kv_chunk_kernel's: there are enough tiles that few splits fill the chip, few keys
+// to split, or so many that merging more splits does not weigh.  Otherwise (one or
+// two KV heads, few sequences) kv_splitkv_kernel's four waves share a tile's keys
+// and its many items merge faster.  natural: scores formed in natural units (softcap,
+// ALiBi), whose arithmetic costs this kernel more than the shared loads save.
+// Measured on MI355X, us a call at each kernel's own splits, split kernel -> this one
+// (tiles):
+//   64/1 heads, 1 token, 5.5k keys (1): 39 -> 53       128/1, 1 x 210k (1): 181 -> 351
 //   32/2, 8 tokens, 7.8k (2): 38 -> 48                 b4 8/1, 16 x 63k (4): 60 -> 101
-//   32/8, 16 x 18k (8): 52 -> 60                       b1 64/4, 9 x 20k (8): 62 -> 71
-//   head_dim 64 32/8, 32 x 12k (8): 41 -> 44           16 tiles, > 16k keys: 1.2x faster
-//   17 - 32 tiles: 1.2 - 1.9x faster                   up to 4k keys: 1.03 - 1.57x faster
-static bool chunk_fills(int64_t tiles, int num_cus) { return 16 * tiles > std::max(num_cus, 1); }
-static bool chunk_pays(int64_t tiles, int64_t keys, int num_cus) {
-    return chunk_fills(tiles, num_cus) || (keys > 0 && keys <= 4096);
+//   32/8, 16 x 18k (8): 52 -> 60                       64/4, 9 x 20k (8): 67 -> 71
+//   32/8, 32 x 106k (8): 274 -> 165                    64/2, 9 x 186k (6): 318 -> 211
+//   12 - 16 tiles: 1.0 - 1.9x faster; 17 and more: 1.2 - 1.9x; up to 4k keys: 1.0 - 1.4x
+//   natural: b4 16/1, 8 x 15k (4): 54 -> 86; 16 tiles: 0.77 - 1.3x; 1 - 8 tiles x 3k: 0.84x
+static bool chunk_pays(int64_t tiles, int64_t keys, bool natural, int num_cus) {
+    const int64_t cus = std::max(num_cus, 1);
+    if (natural) return 16 * tiles > cus;
+    return 24 * tiles > cus || (keys > 0 && keys <= 4096) || (48 * tiles > cus && keys >= 65536);
 }
 
 // Splits of the many-row kernel: the fewest key blocks on the busiest CU (a CU
@@ -1117,14 +1131,15 @@ static bool chunk_pays(int64_t tiles, int64_t keys, int num_cus) {
 // every split to merge.  Measured on MI355X with 32 / 8 heads, head_dim 128, us
 // per call at 1 split -> the splits taken: 512 rows x 1 sequence of 8k keys
 // 226 -> 128 (4 splits), 128 x 1 x 8k 214 -> 59 (8), 32 x 8 x 8k 215 -> 82 (4),
-// 1024 x 1 x 15k 444 -> 410 (2).  At most 16: with the tiles that chunk_pays asks
-// for, that many fill the chip.
-static int chunk_num_splits(int64_t heads, int rows, int capacity, int num_cus) {
-    const int64_t tiles = heads * ((rows + kChunkRows - 1) / kChunkRows), cus = std::max(num_cus, 1);
-    const double blocks = (double(capacity) + kChunkKeys - 1) / kChunkKeys;
+// 1024 x 1 x 15k 444 -> 410 (2).  At most 16 where there are enough tiles for those
+// to fill the chip (chunk_pays), 32 otherwise.
+static int chunk_num_splits(int64_t tiles, int64_t keys, int num_cus) {
+    const int64_t cus = std::max(num_cus, 1);
+    const double blocks = (double(keys) + kChunkKeys - 1) / kChunkKeys;
+    const int most = 24 * tiles > cus ? 16 : kChunkMaxSplits;
     int best = 1;
     double best_t = 0;
-    for (int S = 1; S <= 16 && (S == 1 || blocks >= 4 * S); ++S) {
+    for (int S = 1; S <= most && (S == 1 || blocks >= 4 * S); ++S) {
         const int64_t wgs = tiles * S;
         double t = double((wgs + cus - 1) / cus) * blocks / S;
         if (wgs <= cus) t *= 1.1;
@@ -1137,10 +1152,34 @@ static int chunk_num_splits(int64_t heads, int rows, int capacity, int num_cus) 
     return best;
 }
 
+static int64_t chunk_tiles(const fa_kvcache_args &a) {
+    return int64_t(a.batch) * a.nheads_k * (((a.nheads / a.nheads_k) * a.seqlen_q + kChunkRows - 1) / kChunkRows);
+}
+static int64_t chunk_items(const fa_kvcache_args &a) { return chunk_tiles(a) * a.num_splits; }
+
+// Key positions a call's splits divide at most (the live lengths are on the
+// device): with a left window, the window and the call's own tokens (64 sequences
+// of 1k - 16k tokens, 4096-key window: 192 us in the 2 splits of the whole capacity,
+// 182 in 1).
+static int64_t split_keys(const fa_kvcache_args &a) {
+    const int64_t keys = a.cache_capacity;
+    return a.local_window && a.window_left >= 0 ? std::min<int64_t>(keys, int64_t(a.window_left) + 1 + a.seqlen_q) : keys;
+}
+
+// Whether kv_chunk_kernel suits a call, if it is given the workspaces that the
+// kernel needs: at least 64 query rows per KV head (with 64 rows, 8 sequences of 8k
+// keys, 32 / 8 heads: 71 us against 114 at the best split counts; with 32 rows the
+// other kernel reads K and V once as well and its waves share the keys) in enough
+// tiles (chunk_pays).  Its 64-key blocks must not straddle pages.
+static bool chunk_suits(const fa_kvcache_args &a, int num_cus) {
+    if ((a.nheads / a.nheads_k) * a.seqlen_q < kChunkMinRows) return false;
+    if (a.block_table && a.page_block_size % kChunkKeys != 0) return false;
+    return chunk_pays(chunk_tiles(a), split_keys(a), a.softcap > 0.f || a.alibi_slopes, num_cus);
+}
+
 }  // namespace fa
 
-extern "C" int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_dim, int seqlen_q, int batch,
-                                int nheads, int nheads_k, int num_cus) {
+extern "C" int fa_kv_args_num_splits(const fa_kvcache_args *args, int requested, int num_cus) {
     // An explicit request is honoured (kvcache_native.cu:922-924).  Otherwise
     // (measured on MI355X over paged and contiguous decode shapes) a work item
     // streams best with about 8192 cache positions: fewer and the per-item
@@ -1151,20 +1190,38 @@ extern "C" int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_d
     // on few sequences: one sequence of 1024 positions, 32 / 8 heads, takes
     // 15.5 us per call in 16 splits against 20.3 in 2).  Only the capacity is
     // known on the host (the live lengths are on the device).
-    (void)head_dim;
     if (requested > 0) return requested;
-    if (batch <= 0 || nheads_k <= 0 || nheads <= 0 || seqlen_k_capacity <= 0) return 1;
-    const int rows = (nheads / nheads_k) * seqlen_q;
-    const int64_t tiles = int64_t(batch) * nheads_k * ((rows + fa::kChunkRows - 1) / fa::kChunkRows);
-    if (rows >= fa::kChunkMinRows && fa::chunk_pays(tiles, seqlen_k_capacity, num_cus))
-        return fa::chunk_num_splits(int64_t(batch) * nheads_k, rows, seqlen_k_capacity, num_cus);
-    const int64_t wgs = int64_t(batch) * nheads_k * ((rows + 31) / 32);
-    const int64_t by_len = (int64_t(seqlen_k_capacity) + 4096) / 8192;
+    if (!args || args->batch <= 0 || args->nheads_k <= 0 || args->nheads <= 0) return 1;
+    const fa_kvcache_args &a = *args;
+    const int64_t keys = fa::split_keys(a);
+    if (keys <= 0) return 1;
+    if (fa::chunk_suits(a, num_cus)) return fa::chunk_num_splits(fa::chunk_tiles(a), keys, num_cus);
+    const int rows = (a.nheads / a.nheads_k) * a.seqlen_q;
+    const int64_t wgs = int64_t(a.batch) * a.nheads_k * ((rows + 31) / 32);
+    const int64_t by_len = (keys + 4096) / 8192;
     const int64_t by_fill = (int64_t(std::max(num_cus, 1)) + wgs - 1) / std::max<int64_t>(wgs, 1);
-    int64_t max_by_len = seqlen_k_capacity / 512;
-    if (seqlen_k_capacity >= 512) max_by_len = std::max<int64_t>(max_by_len, std::min(16, seqlen_k_capacity / 64));
+    int64_t max_by_len = keys / 512;
+    if (keys >= 512) max_by_len = std::max<int64_t>(max_by_len, std::min<int64_t>(16, keys / 64));
     max_by_len = std::max<int64_t>(1, max_by_len);
-    return int(std::max<int64_t>(1, std::min<int64_t>({std::max(by_len, by_fill), max_by_len, 128})));
+    // One workgroup combines the splits of a tile's 32 rows: with many rows on few
+    // tiles that outweighs idle CUs (us in the splits that fill the chip -> 16: 64/1
+    // heads, 1 token on 70k keys 128: 271 -> 80; b2 16/1 d64, 4 tokens on 39k keys 64:
+    // 120 -> 45; at 225k keys b3 128/1 d64 254 in 16, 187 in 32).
+    const int64_t most = rows < fa::kChunkMinRows ? 128 : keys > 131072 ? 32 : 16;
+    return int(std::max<int64_t>(1, std::min<int64_t>({std::max(by_len, by_fill), max_by_len, most})));
+}
+
+extern "C" int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_dim, int seqlen_q, int batch,
+                                int nheads, int nheads_k, int num_cus) {
+    // The same for a call without options on a cache whose pages are multiples of 64 tokens.
+    fa_kvcache_args a{};
+    a.cache_capacity = seqlen_k_capacity;
+    a.head_dim = head_dim;
+    a.seqlen_q = seqlen_q;
+    a.batch = batch;
+    a.nheads = nheads;
+    a.nheads_k = nheads_k;
+    return fa_kv_args_num_splits(&a, requested, num_cus);
 }
 
 extern "C" size_t fa_kv_workspace_bytes(const fa_kvcache_args *a) {
@@ -1233,31 +1290,12 @@ int kv_heads_per_item(const fa_kvcache_args &a) {
     return hpi;
 }
 
-int64_t chunk_tiles(const fa_kvcache_args &a) {
-    return int64_t(a.batch) * a.nheads_k * (((a.nheads / a.nheads_k) * a.seqlen_q + kChunkRows - 1) / kChunkRows);
-}
-int64_t chunk_items(const fa_kvcache_args &a) { return chunk_tiles(a) * a.num_splits; }
-
-// Whether the split kernel of a call is kv_chunk_kernel: at least 64 query rows
-// per KV head (with 64 rows, 8 sequences of 8k keys, 32 / 8 heads: 71 us against
-// 114 at the best split counts; with 32 rows the other kernel reads K and V once as
-// well and its waves share the keys) in enough tiles (chunk_pays; with softcap or
-// ALiBi, whose scores cost more arithmetic than the shared loads save, a short cache
-// is not reason enough: b1 8/1 304 rows x 3k keys 35 -> 42 us), few enough splits
-// for one workgroup to merge, and the split counts to do it with.  Its 64-key blocks
-// must not straddle pages, and its page ids fit in LDS.
+// Whether the split kernel of a call is kv_chunk_kernel: it suits the call, there
+// are few enough splits for one workgroup to merge, and the split counts to do it
+// with.
 bool use_chunk(const fa_kvcache_args &a) {
-    const int R = (a.nheads / a.nheads_k) * a.seqlen_q;
-    if (R < kChunkMinRows || a.num_splits > kChunkMaxSplits || !a.batch_order || (a.num_splits > 1 && !a.split_count))
-        return false;
-    // A left window leaves so many keys, as the caller's split count takes them.
-    int64_t keys = a.cache_capacity;
-    if (a.local_window && a.window_left >= 0) keys = std::min<int64_t>(keys, int64_t(a.window_left) + 1 + a.seqlen_q);
-    const bool natural = a.softcap > 0.f || a.alibi_slopes;
-    if (!(natural ? chunk_fills(chunk_tiles(a), device_cus()) : chunk_pays(chunk_tiles(a), keys, device_cus())))
-        return false;
-    return !a.block_table || (a.page_block_size % kChunkKeys == 0 && a.cache_capacity > 0 &&
-                              a.cache_capacity / a.page_block_size <= kChunkPages);
+    return a.batch_order && a.num_splits <= kChunkMaxSplits && (a.num_splits == 1 || a.split_count) &&
+           chunk_suits(a, device_cus());
 }
 
 // Whether the split kernel's items come in the order of batch_order: there are

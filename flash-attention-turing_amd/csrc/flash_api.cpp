@@ -593,15 +593,7 @@ std::vector<at::Tensor> mha_fwd_kvcache(at::Tensor q, at::Tensor k_cache, at::Te
     // forward kernel with per-batch key counts and the batch remap.
     const bool use_split_kernel = has_block_table || num_splits > 1 || seqlen_q == 1 || options;
     if (use_split_kernel) {
-        // With a left window the splits divide the window and the call's own
-        // tokens (64 sequences of 1k - 16k tokens, 4096-key window: 192 us in the
-        // 2 splits of the whole capacity, 182 in 1).
-        const int64_t keys = a.window_left >= 0
-                                 ? std::min<int64_t>(seqlen_cache, int64_t(a.window_left) + 1 + seqlen_q)
-                                 : seqlen_cache;
-        a.num_splits = fa_kv_num_splits(num_splits, int(keys), int(head_size), int(seqlen_q),
-                                        int(batch_size), int(num_heads), int(num_heads_k),
-                                        num_cus(q.get_device()));
+        a.num_splits = fa_kv_args_num_splits(&a, num_splits, num_cus(q.get_device()));
         // Workspace: split accumulators (num_splits > 1), then the longest-first
         // sequence order the split kernel schedules by and its work counter, then
         // the split counts with which it combines the partials itself.  Append,

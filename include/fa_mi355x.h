@@ -226,7 +226,12 @@ typedef struct fa_kvcache_args {
 } fa_kvcache_args;
 
 /* Split count for a request (kvcache_native.cu:913-952 choose_num_splits);
- * requested > 0 is returned unchanged. */
+ * requested > 0 is returned unchanged.  fa_kv_args_num_splits takes the call itself
+ * (sizes, options, cache_capacity; num_splits and the workspaces are not read, and
+ * batch_order and split_count are taken to be given), fa_kv_num_splits only the sizes
+ * of a call without options.  fa_kv_args_num_splits has no counterpart in the
+ * reference. */
+int fa_kv_args_num_splits(const fa_kvcache_args *args, int requested, int num_cus);
 int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_dim, int seqlen_q,
                      int batch, int nheads, int nheads_k, int num_cus);
 /* Bytes of the split accumulators for args->num_splits (0 when num_splits == 1);

@@ -259,15 +259,42 @@ def test_split_workspace_alignment(lib, off):
 
 
 def test_num_splits_many_rows(lib):
-    # From 64 query rows per KV head on, the many-row kernel's count (at most 16) where its 128-row tiles are many
-    # enough (more than a sixteenth of the CUs) or the keys few; else the split kernel's, which fills the chip.
+    # From 64 query rows per KV head on, the many-row kernel's count where its 128-row tiles are many enough or the
+    # keys few; else the split kernel's, at most 16, or 32 past 131072 keys.
     f = lib.fa_kv_num_splits
     for (cap, d, sq, b, h, hk), least in {
-        (131072, 128, 1, 1, 64, 1): 32,  # one tile
-        (65536, 128, 4, 1, 32, 2): 32,  # two
+        (262144, 128, 1, 1, 64, 1): 32,  # one tile
+        (65536, 128, 4, 1, 32, 2): 16,  # two
         (131072, 64, 16, 1, 32, 8): 16,  # eight
     }.items():
         assert f(0, cap, d, sq, b, h, hk, 256) >= least
         assert f(0, 4096, d, sq, b, h, hk, 256) <= 16
     assert f(0, 131072, 128, 16, 4, 32, 8, 256) <= 16  # 32 tiles
     assert f(0, 300000, 128, 512, 2, 32, 8, 256) <= 2  # 256 tiles
+
+
+def test_num_splits_of_a_call(lib):
+    # fa_kv_args_num_splits knows what chooses the kernel besides the sizes: scores in natural units (softcap, ALiBi),
+    # the page size and a window; without those it agrees with fa_kv_num_splits.
+    fa_capi = _capi()
+    f, g = lib.fa_kv_args_num_splits, lib.fa_kv_num_splits
+    f.argtypes = [ctypes.POINTER(fa_capi.FaKvcacheArgs), ctypes.c_int, ctypes.c_int]
+
+    def call(cap, d, sq, b, h, hk, requested=0, **more):
+        a = fa_capi.FaKvcacheArgs()
+        a.cache_capacity, a.head_dim, a.seqlen_q, a.batch, a.nheads, a.nheads_k = cap, d, sq, b, h, hk
+        for name, x in more.items():
+            setattr(a, name, x)
+        return f(ctypes.byref(a), requested, 256)
+
+    assert f(None, 0, 256) == 1
+    for cap in (0, 1, 500, 4096, 10000, 70000, 300000):
+        for d, sq, b, h, hk in ((128, 1, 64, 32, 8), (128, 1, 1, 64, 1), (64, 16, 2, 32, 8), (128, 512, 2, 32, 8),
+                                (64, 100, 1, 8, 8)):
+            assert call(cap, d, sq, b, h, hk) == g(0, cap, d, sq, b, h, hk, 256)
+            assert call(cap, d, sq, b, h, hk, requested=9) == 9
+    many = (20000, 128, 16, 2, 32, 8)  # 16 tiles of 128 rows, 32 of 32
+    split = call(*many, softcap=30.0)
+    assert split == call(*many, alibi_slopes=1 << 20) == call(*many, block_table=1 << 20, page_block_size=32) == 8
+    assert call(*many) == call(*many, block_table=1 << 20, page_block_size=64) > split
+    assert call(*many, local_window=1, window_left=1000) == call(1017, *many[1:])

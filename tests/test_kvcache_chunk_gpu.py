@@ -9,6 +9,7 @@ import torch
 import flash_attention_interface as fai
 from helpers import assert_2x, assert_lse, kv_oracle, randn16
 from oracle import kvcache as okv
+from test_capi_paths_gpu import _kv_capi
 from test_kvcache_gpu import _paged_from_contiguous
 
 # batch, queries, heads, kv heads, head_dim, capacity, appended, lengths before the append, splits, causal, options.
@@ -88,3 +89,59 @@ def test_kvcache_chunk(device, case):
         else:  # the heuristic may cut another capacity into another number of splits
             assert_2x("out", plain[0], o_ref, o_ref.to(torch.float16))
             assert_2x("out", remap[0], o_ref, o_ref.to(torch.float16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [1, 2])
+def test_chunk_over_1024_pages(device, splits):
+    """1100 shuffled pages of 64 tokens: with one split its page ids do not fit in LDS at once and are staged anew on
+    the way; the contiguous cache of the same tokens gives the same bits (18 KV heads of one tile: this kernel)."""
+    g = torch.Generator().manual_seed(8400)
+    pages, page, sq, h, hd = 1100, 64, 64, 18, 64
+    cap, lens = pages * page, torch.tensor([pages * page - 21], dtype=torch.int32)
+    q = randn16((1, sq, h, hd), g)
+    gd = torch.Generator(device=device).manual_seed(8401)
+    kc, vc = (torch.randn((1, cap, h, hd), generator=gd, device=device, dtype=torch.float16) for _ in range(2))
+    table = torch.randperm(pages, generator=g).to(torch.int32)
+    kp, vp = (torch.empty((pages, page, h, hd), dtype=torch.float16, device=device) for _ in range(2))
+    for dst, src in ((kp, kc), (vp, vc)):
+        dst[table.long().to(device)] = src.view(pages, page, h, hd)
+    print(f"case over 1024 pages splits={splits}", flush=True)
+    kw = dict(causal=True, splits=splits, order=True, fused=splits > 1, calls=("fa_fwd_kvcache",))
+    out, lse, _, _ = _kv_capi(device, q, kp, vp, None, None, lens, table.view(1, pages), **kw)
+    out2, lse2, _, _ = _kv_capi(device, q, kc, vc, None, None, lens, None, **kw)
+    assert torch.equal(out, out2) and torch.equal(lse, lse2)
+    for i in (0, h - 1):
+        ku, vu = okv.materialize(kc[:, :, i:i + 1].cpu(), vc[:, :, i:i + 1].cpu(), lens, None, None)
+        o_ref, l_ref = okv.splitkv_attention(q[:, :, i:i + 1], ku, vu, lens, hd ** -0.5, True, 1)
+        assert_2x("out", out[:, :, i:i + 1], o_ref, o_ref.to(torch.float16))
+        assert_lse(lse[:, i:i + 1], l_ref)
+
+
+# Batches of chunks in more items than CUs (12 sequences x 8 KV heads x 2 tiles x 3 splits): sequences in the order of
+# their lengths, an empty one among them, later items starting while earlier ones merge.
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd,opt", [(128, ""), (64, "softcap alibi"), (128, "alibi window"), (64, "leftpad")])
+def test_chunk_ranked(device, hd, opt):
+    b, sq, h, hk, cap, new, splits = 12, 33, 32, 8, 640, 33, 3
+    assert b * hk * 2 * splits > torch.cuda.get_device_properties(0).multi_processor_count, "items must be ranked"
+    g = torch.Generator().manual_seed(8500 + hd + len(opt))
+    q, kc, vc = randn16((b, sq, h, hd), g), randn16((b, cap, hk, hd), g), randn16((b, cap, hk, hd), g)
+    k, v = randn16((b, new, hk, hd), g), randn16((b, new, hk, hd), g)
+    seqlens = torch.tensor([0, 607, 31, 300, 64, 600, 1, 450, 128, 95, 520, 200], dtype=torch.int32)
+    ends = seqlens + new
+    kw = dict(window_size=(150, 0) if "window" in opt else (-1, -1), softcap=15.0 if "softcap" in opt else 0.0,
+              alibi_slopes=2.0 ** -torch.arange(1, h + 1, dtype=torch.float32) / 4 if "alibi" in opt else None,
+              cache_leftpad=torch.arange(b, dtype=torch.int32) * 3 if "leftpad" in opt else None)
+    print(f"case ranked hd={hd} {opt}", flush=True)
+    _, _, kc_ref, vc_ref = kv_oracle(q, kc, vc, k, v, seqlens, None, None, True, 1, None)
+    ku, vu = okv.materialize(kc_ref, vc_ref, ends, None, None)
+    o_ref, l_ref = okv.splitkv_attention(q, ku, vu, ends, hd ** -0.5, True, 1, window=kw["window_size"],
+                                         softcap=kw["softcap"], alibi_slopes=kw["alibi_slopes"],
+                                         leftpad=kw["cache_leftpad"])
+    got = _call(device, q, kc, vc, k, v, seqlens, None, None, splits, True, kw)
+    again = _call(device, q, kc, vc, k, v, seqlens, None, None, splits, True, kw)
+    assert torch.equal(got[2], kc_ref) and torch.equal(got[3], vc_ref)
+    assert torch.equal(got[0], again[0]) and torch.equal(got[1], again[1])
+    assert_2x("out", got[0], o_ref, o_ref.to(torch.float16))
+    assert_lse(got[1], l_ref)
