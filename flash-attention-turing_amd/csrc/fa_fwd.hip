@@ -855,11 +855,15 @@ static FwdPlan fwd_plan(const fa_fwd_args &a) {
     const int least = half                ? !a.cu_seqlens_q && U64 <= cus ? 2 : 8
                       : a.head_dim == 64 ? (causal_near(a) ? 6 : 8)
                                          : (causal_near(a) ? 9 : 12);
+    const bool few = 2 * U <= 3 * cus, dense = !a.cu_seqlens_q;  // varlen: the work order lists unsplit blocks
     FwdPlan plan = {1, 1};
-    if (W <= cus ? 2 * U <= 3 * cus && NB >= least : W <= 2 * cus && causal_square(a) && NB >= 32) plan.groups = 2;
-    if (!half || plan.groups == 1 || a.cu_seqlens_q) return plan;  // varlen: the work order lists unsplit blocks
+    if (W > cus)
+        plan.groups = W <= 2 * cus && causal_square(a) && NB >= 32 ? 2 : 1;
+    else if (few || (half && dense && U <= 2 * cus))
+        plan.groups = NB >= least ? 2 : 1;
+    if (!half || plan.groups == 1 || !dense) return plan;
     const double pairs = 0.5 * NB, unit = a.head_dim == 128 ? 1.84 : 1.31;
-    const double unsplit = pairs * (a.head_dim == 128 ? 1.58 : 0.9);
+    const double unsplit = pairs * (a.head_dim == 128 ? 1.58 : 0.9), one_group = pairs * 2.44;
     double best = unsplit;
     for (int S = 2; S <= 16 && W * S <= cus; ++S) {
         const double t = pairs / S * unit + 6 + 2 * S;
@@ -868,10 +872,15 @@ static FwdPlan fwd_plan(const fa_fwd_args &a) {
             plan.splits = S;
         }
     }
-    // Where the unpacked form of the call fills the chip by itself, it takes the
-    // shares one after another and gains nothing: only where they halve the packed
-    // form's time.
-    if (U >= cus && best > 0.5 * unsplit) plan.splits = 1;
+    // Where the unpacked form of the call fills the chip by itself, it gains nothing
+    // by two groups or shares and takes the shares one after another (5 - 18 % slower,
+    // the more the shorter): only where the packed form gains much.  16 queries of b16
+    // 32/8 and 32/32 heads, us in one group -> as planned: 3000 keys 66 -> 46 and 137 ->
+    // 154, 20000 keys 392 -> 261 and (10000) 439 -> 465; head_dim 64, 8000 keys, where
+    // two groups do without shares: 122 -> 84 and 184 -> 194.
+    if (!few && a.head_dim == 64) plan.splits = 1;
+    if (!few && a.head_dim == 128 && best > 0.6 * one_group) plan = {1, 1};
+    if (few && U >= cus && best > 0.55 * unsplit) plan.splits = 1;
     return plan;
 }
 // Workgroups of the unsplit grid of BM-row blocks.
