@@ -18,6 +18,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stdint.h>
 
 #include "fa_mi355x.h"
@@ -244,18 +245,18 @@ __device__ __forceinline__ int swz(int row) {
 }
 
 // Copy rows [row0, row0 + ROWS) of a [rows][HD] fp16 source (row stride rs,
-// rows clamped to <= last_row) into a swizzled natural tile with DMA: the NT
+// rows clamped to [first_row, last_row]) into a swizzled natural tile with DMA: the NT
 // threads of the workgroup each move ROWS*HD/8/NT chunks.  General form (any
 // row0, clamping per row); TileCopier below is the fast path.
 template <int HD, int ROWS, int NT>
 __device__ __forceinline__ void dma_tile(char *tile, const f16 *src, int64_t rs, int row0, int last_row, int wave,
-                                         int lane) {
+                                         int lane, int first_row = INT_MIN) {
     constexpr int KCH = HD / 8, CPT = ROWS * KCH / NT, WAVES = NT / 64;
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
         const int base = (i * WAVES + wave) * 64;
         const int p = base + lane, row = p / KCH, cs = p % KCH;
-        const int64_t r = min(row0 + row, last_row);
+        const int64_t r = max(min(row0 + row, last_row), first_row);
         g2l16(src + r * rs + 8 * (cs ^ swz<KCH>(row)), tile + base * 16);
     }
 }

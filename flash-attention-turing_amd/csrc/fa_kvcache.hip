@@ -936,12 +936,12 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcach
         const f16 *kb = kc + blk * a.k_cache.batch_stride + int64_t(at) * krs;
         const f16 *vb = vc + blk * a.v_cache.batch_stride + int64_t(at) * vrs;
         const int soff = (nb & 1) * STAGE;
-        if (nb * BN + BN <= L) {
+        if (nb * BN >= t_lo && nb * BN + BN <= L) {
             kcp.template copy_to<true>(lds_addr(smem) + soff, kb, krs);
             vcp.template copy_to<true>(lds_addr(smem) + soff + TILE, vb, vrs);
-        } else {  // keys past L re-read key L - 1 (masked)
-            dma_tile<HD, BN, kKvThreads>(smem + soff, kb, krs, 0, L - 1 - nb * BN, wave, lane);
-            dma_tile<HD, BN, kKvThreads>(smem + soff + TILE, vb, vrs, 0, L - 1 - nb * BN, wave, lane);
+        } else {  // keys past L re-read key L - 1, keys that no row sees at the start re-read the first seen one (masked)
+            dma_tile<HD, BN, kKvThreads>(smem + soff, kb, krs, 0, L - 1 - nb * BN, wave, lane, t_lo - nb * BN);
+            dma_tile<HD, BN, kKvThreads>(smem + soff + TILE, vb, vrs, 0, L - 1 - nb * BN, wave, lane, t_lo - nb * BN);
         }
     };
 

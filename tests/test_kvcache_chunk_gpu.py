@@ -145,3 +145,26 @@ def test_chunk_ranked(device, hd, opt):
     assert torch.equal(got[0], again[0]) and torch.equal(got[1], again[1])
     assert_2x("out", got[0], o_ref, o_ref.to(torch.float16))
     assert_lse(got[1], l_ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pad,window", [((32, 96), (-1, -1)), ((33, 127), (-1, -1)), ((0, 0), (40, 0))])
+def test_chunk_ignores_what_unseen_keys_hold(device, pad, window):
+    """Keys before a sequence's leftpad, or before the window of every query, share a key block with the first one
+    seen; NaN in them reaches no output."""
+    b, sq, h, hk, hd, cap, lens = 2, 70, 4, 4, 128, 512, (300, 450)
+    g = torch.Generator().manual_seed(8600 + sum(pad))
+    q, kc, vc = randn16((b, sq, h, hd), g), randn16((b, cap, hk, hd), g), randn16((b, cap, hk, hd), g)
+    seqlens, leftpad = torch.tensor(lens, dtype=torch.int32), torch.tensor(pad, dtype=torch.int32)
+    print(f"case unseen keys pad={pad} window={window}", flush=True)
+    o_ref, l_ref = okv.splitkv_attention(q, *okv.materialize(kc, vc, seqlens, None, None), seqlens, hd ** -0.5, True, 1,
+                                         window=window, leftpad=leftpad)
+    for i in range(b):
+        first = pad[i] if window[0] < 0 else lens[i] - sq - window[0]
+        assert first > 0 and first % 64
+        kc[i, :first], vc[i, :first] = float("nan"), float("nan")
+    for splits in (1, 3):
+        out, lse = _call(device, q, kc, vc, None, None, seqlens, None, None, splits, True,
+                         dict(window_size=window, cache_leftpad=leftpad))[:2]
+        assert_2x("out", out, o_ref, o_ref.to(torch.float16))
+        assert_lse(lse, l_ref)
