@@ -104,12 +104,23 @@ int num_cus(int device) {
     return n;
 }
 
+// A workspace that a call is faster with but can do without: undefined where the
+// device has no memory left for it.
+at::Tensor optional_workspace(int64_t numel, const at::TensorOptions &options) {
+    try {
+        return at::empty({numel}, options);
+    } catch (const c10::OutOfMemoryError &) {
+        return at::Tensor();
+    }
+}
+
 // The workspace in which workgroups that share a query block sum their results
 // (undefined when the grid needs no sharing).
 at::Tensor fwd_workspace(fa_fwd_args &a, const at::Tensor &like) {
     const size_t bytes = fa_fwd_split_bytes(&a);
     if (bytes == 0) return at::Tensor();
-    at::Tensor ws = at::empty({int64_t(bytes)}, like.options().dtype(at::kByte));
+    at::Tensor ws = optional_workspace(int64_t(bytes), like.options().dtype(at::kByte));
+    if (!ws.defined()) return ws;
     a.split_ws = ws.data_ptr();
     a.split_ws_bytes = int64_t(bytes);
     return ws;
@@ -120,12 +131,15 @@ at::Tensor fwd_workspace(fa_fwd_args &a, const at::Tensor &like) {
 // their results (when there are such).  Calls of a few tens of microseconds of
 // GPU time wait for the host, and a second allocation was part of that (forward
 // and backward, b1 s700 16/16 d64: 85.6 -> 81.3 us; b2 s200 16/4: 95.4 -> 90.8).
+// The second part (up to 256 MiB) is left out where there is no memory for it.
 at::Tensor bwd_workspace(fa_bwd_args &a, const at::Tensor &l) {
     const int64_t split = int64_t(fa_bwd_split_bytes(&a));
     const int64_t dsum = 2 * l.numel(), at_split = split > 0 ? (dsum + 63) / 64 * 64 : dsum;  // in floats
-    at::Tensor ws = at::empty({at_split + (split + 3) / 4}, l.options());
+    at::Tensor ws = split > 0 ? optional_workspace(at_split + (split + 3) / 4, l.options()) : at::Tensor();
+    const bool shared = ws.defined();
+    if (!shared) ws = at::empty({dsum}, l.options());
     a.dsum = ws.data_ptr<float>();
-    if (split > 0) {
+    if (shared) {
         a.split_ws = a.dsum + at_split;
         a.split_ws_bytes = split;
     }

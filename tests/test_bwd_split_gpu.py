@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import fa_capi
+import flash_attention_interface as fai
 from helpers import assert_2x, check_fwd_bwd, check_varlen, cu_from_lengths, randn16
 from oracle.attention import attention_bwd, attention_fwd, bwd_fp32_noise
 from oracle.twin import bwd_twin, fwd_twin
@@ -184,3 +185,29 @@ def test_dkdv_clears_its_own_counters(device, before):
     torch.cuda.synchronize()
     for x, y, z in zip(*got, grads[1:]):
         assert torch.equal(x, z) and torch.equal(y, z)
+
+
+@pytest.mark.gpu
+def test_split_workspace_is_optional_memory(device):
+    """A training step that fits in memory without the shares' workspace still runs: the extension does without it."""
+    b, sq, h, hk, hd = 1, 8192, 32, 8, 128
+    g = torch.Generator().manual_seed(8500)
+    q, do = randn16((b, sq, h, hd), g).to(device), randn16((b, sq, h, hd), g).to(device)
+    k, v = randn16((b, sq, hk, hd), g).to(device), randn16((b, sq, hk, hd), g).to(device)
+    s = hd ** -0.5
+    print("case optional workspace", flush=True)
+    ba, o, lse, grads = _args(q, k, v, do, s, True)
+    need = fa_capi.load().fa_bwd_split_bytes(ctypes.byref(ba))
+    fa_capi.call("fa_bwd", ba)  # unshared
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    room = sum(t.numel() * t.element_size() for t in grads) + (32 << 20)
+    assert need > room
+    total = torch.cuda.get_device_properties(device).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + room) / total)
+    try:
+        got = fai._flash_attn_backward(do, q, k, v, o, lse, s, True)
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert all(torch.equal(x, y) for x, y in zip(got, grads))
