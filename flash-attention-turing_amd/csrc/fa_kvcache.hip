@@ -1166,6 +1166,13 @@ static int64_t split_keys(const fa_kvcache_args &a) {
     return a.local_window && a.window_left >= 0 ? std::min<int64_t>(keys, int64_t(a.window_left) + 1 + a.seqlen_q) : keys;
 }
 
+// Scratch bytes fa_fwd_kvcache_noalloc needs for a call: the split accumulators, then
+// batch + 1 int32s of order and counter, then the split counts.
+static size_t noalloc_bytes(const fa_kvcache_args &a) {
+    return fa_kv_workspace_bytes(&a) +
+           (size_t(a.batch > 0 ? a.batch : 0) + 1 + size_t(fa_kv_split_count_len(&a))) * sizeof(int32_t);
+}
+
 // Whether kv_chunk_kernel suits a call, if it is given the workspaces that the
 // kernel needs: at least 64 query rows per KV head (with 64 rows, 8 sequences of 8k
 // keys, 32 / 8 heads: 71 us against 114 at the best split counts; with 32 rows the
@@ -1213,7 +1220,10 @@ extern "C" int fa_kv_args_num_splits(const fa_kvcache_args *args, int requested,
 
 extern "C" int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_dim, int seqlen_q, int batch,
                                 int nheads, int nheads_k, int num_cus) {
-    // The same for a call without options on a cache whose pages are multiples of 64 tokens.
+    // The same for a call without options on a cache whose pages are multiples of
+    // 64 tokens, in no more splits than the static scratch of
+    // fa_fwd_kvcache_noalloc holds where many rows ask for more (a count from here
+    // always suits that entry there).
     fa_kvcache_args a{};
     a.cache_capacity = seqlen_k_capacity;
     a.head_dim = head_dim;
@@ -1221,7 +1231,10 @@ extern "C" int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_d
     a.batch = batch;
     a.nheads = nheads;
     a.nheads_k = nheads_k;
-    return fa_kv_args_num_splits(&a, requested, num_cus);
+    a.num_splits = fa_kv_args_num_splits(&a, requested, num_cus);
+    if (requested <= 0 && a.num_splits > 1 && fa::chunk_suits(a, num_cus))
+        while (a.num_splits > 1 && fa::noalloc_bytes(a) > FA_NOALLOC_SCRATCH_BYTES) --a.num_splits;
+    return a.num_splits;
 }
 
 extern "C" size_t fa_kv_workspace_bytes(const fa_kvcache_args *a) {
@@ -1484,19 +1497,12 @@ int scratch_address(void **out) {
     return FA_OK;
 }
 
-// Scratch bytes a call needs: the split accumulators, then batch + 1 int32s of
-// order and counter, then the split counts.
-size_t noalloc_bytes(const fa_kvcache_args *a) {
-    return fa_kv_workspace_bytes(a) +
-           (size_t(a->batch > 0 ? a->batch : 0) + 1 + size_t(fa_kv_split_count_len(a))) * sizeof(int32_t);
-}
-
 }  // namespace
 
 extern "C" int fa_fwd_kvcache_noalloc(const fa_kvcache_args *args, void *stream) {
     int rc = fa::check_kv(args);
     if (rc) return rc;
-    if (noalloc_bytes(args) > FA_NOALLOC_SCRATCH_BYTES) return FA_ERR_SCRATCH;
+    if (fa::noalloc_bytes(*args) > FA_NOALLOC_SCRATCH_BYTES) return FA_ERR_SCRATCH;
     void *base = nullptr;
     if ((rc = scratch_address(&base))) return rc;
     fa_kvcache_args a = *args;

@@ -229,7 +229,8 @@ typedef struct fa_kvcache_args {
  * requested > 0 is returned unchanged.  fa_kv_args_num_splits takes the call itself
  * (sizes, options, cache_capacity; num_splits and the workspaces are not read, and
  * batch_order and split_count are taken to be given), fa_kv_num_splits only the sizes
- * of a call without options.  fa_kv_args_num_splits has no counterpart in the
+ * of a call without options, and where many rows per KV head ask for more splits than
+ * fa_fwd_kvcache_noalloc's scratch holds it returns as many as fit.  fa_kv_args_num_splits has no counterpart in the
  * reference. */
 int fa_kv_args_num_splits(const fa_kvcache_args *args, int requested, int num_cus);
 int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_dim, int seqlen_q,

@@ -289,8 +289,7 @@ def test_num_splits_of_a_call(lib):
 
     assert f(None, 0, 256) == 1
     for cap in (0, 1, 500, 4096, 10000, 70000, 300000):
-        for d, sq, b, h, hk in ((128, 1, 64, 32, 8), (128, 1, 1, 64, 1), (64, 16, 2, 32, 8), (128, 512, 2, 32, 8),
-                                (64, 100, 1, 8, 8)):
+        for d, sq, b, h, hk in ((128, 1, 64, 32, 8), (128, 1, 1, 64, 1), (64, 16, 2, 32, 8), (64, 100, 1, 8, 8)):
             assert call(cap, d, sq, b, h, hk) == g(0, cap, d, sq, b, h, hk, 256)
             assert call(cap, d, sq, b, h, hk, requested=9) == 9
     many = (20000, 128, 16, 2, 32, 8)  # 16 tiles of 128 rows, 32 of 32
@@ -298,3 +297,25 @@ def test_num_splits_of_a_call(lib):
     assert split == call(*many, alibi_slopes=1 << 20) == call(*many, block_table=1 << 20, page_block_size=32) == 8
     assert call(*many) == call(*many, block_table=1 << 20, page_block_size=64) > split
     assert call(*many, local_window=1, window_left=1000) == call(1017, *many[1:])
+
+
+def test_num_splits_suits_the_static_scratch(lib):
+    # Sizes whose split count of one item per CU (at least 512 positions each, or 64 in at most 16) fits in
+    # fa_fwd_kvcache_noalloc's scratch: so does fa_kv_num_splits', which many rows would have larger.
+    limit, seen = 16 << 20, 0
+    for h, hk in ((32, 8), (64, 1), (16, 16), (8, 2)):
+        for sq in (1, 4, 16, 64, 200, 512, 2000):
+            for b in (1, 2, 8, 40):
+                for cap in (256, 1000, 4096, 20000, 131072):
+                    rows, wgs = h // hk * sq, b * hk * ((h // hk * sq + 31) // 32)
+                    most = max(1, cap // 512, min(16, cap // 64) if cap >= 512 else 0)
+                    fill = max(1, min(max((cap + 4096) // 8192, -(-256 // wgs)), most, 128))
+
+                    def need(s):
+                        return (s > 1) * s * b * h * sq * 129 * 4 + 4 * (b + 1 + (s > 1) * wgs)
+
+                    if need(fill) <= limit:
+                        seen += 1
+                        s = lib.fa_kv_num_splits(0, cap, 128, sq, b, h, hk, 256)
+                        assert need(s) <= limit, (h, hk, sq, b, cap, s, rows)
+    assert seen > 300
