@@ -34,7 +34,7 @@ HIP_FLAGS = [
     "-std=c++17",
     "-fPIC",
     "-ffp-contract=fast",
-    # Packed fp32 VALU ops stay off (they have given wrong results on this pool).
+    # Packed fp32 VALU ops stay off (some of their forms have given wrong results on this part).
     "-Xclang",
     "-target-feature",
     "-Xclang",

@@ -17,8 +17,11 @@
 // with ds_read_b64_tr_b16.  P^T feeds the O^T += V^T P^T MFMAs directly from
 // the accumulators (see fa_common.h).
 //
-// Two kernels share that per-wave arithmetic (so their results are the same
-// bit for bit) and differ in how the waves of a SIMD take turns:
+// Two kernels share that per-wave arithmetic and differ in how the waves of a
+// SIMD take turns.  With one wave group, which walks a row's key blocks in order,
+// their results are the same bit for bit; two groups and splits round and sum in
+// another order, so on small grids a row's bits depend on the plan, that is on
+// batch, head count and lengths (fwd_plan), but not on how GQA heads are packed:
 //   * fwd_pp_kernel (head_dim 128, grids of at least two workgroups per CU):
 //     8 waves, two per SIMD, in two groups that alternate a matrix phase (the
 //     PV product of block j - 1 and the S product of block j: all the LDS

@@ -29,13 +29,14 @@
 // caches with the same head stride take the same tile order and the same
 // arithmetic, so their results are bit-identical for the same logical cache.
 // Work items are ordered with the sequence rank slowest: when the caller
-// passes a batch_order workspace, one
+// passes a batch_order workspace and there are more items than CUs, one
 // workgroup of the append launch first ranks the sequences by key count
 // (longest first) and a resident grid of two workgroups per CU deals the items
 // out from a device counter in that order, so the longest sequences start
 // first, the short ones fill the end, and no workgroup is relaunched between
 // items.  With split counts as well, the last split item of each row tile to
 // finish combines the tile's partials, so a decode call is two launches.
+// Calls of many query rows take kv_chunk_kernel instead (below).
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -1355,9 +1356,10 @@ int launch_chunk(const fa_kvcache_args &a, hipStream_t s) {
     return int(hipGetLastError());
 }
 
-// The split kernel.  With batch_order (ranked and its counter reset by
-// launch_prep on the same stream): a resident grid of two workgroups per CU
-// that deals the items out in that order.  Without it: one workgroup per item.
+// The split kernel.  With batch_order: a resident grid of two workgroups per CU
+// that deals the items out, in its order where launch_prep on the same stream has
+// ranked the sequences and reset the counter (kv_ranked: more items than CUs; else
+// each workgroup has one item).  Without it: one workgroup per item.
 int launch_split(const fa_kvcache_args &a, hipStream_t s) {
     if (use_chunk(a)) return launch_chunk(a, s);
     const int hpi = kv_heads_per_item(a);

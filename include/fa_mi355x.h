@@ -81,17 +81,17 @@ typedef struct fa_fwd_args {
     void *split_ws;
     int64_t split_ws_bytes;
     /* Rows of the packed o tensor (varlen calls), or 0.  When set, o's rows that no
-     * sequence covers (before cu_seqlens_q[0], from cu_seqlens_q[batch] on) are
-     * zeroed on the device; 0 leaves them as they are. */
+     * sequence covers (before cu_seqlens_q[0], from cu_seqlens_q[batch] on, and past
+     * lse_seqlen within a sequence) are zeroed on the device; 0 leaves them as they are. */
     int32_t o_rows;
 } fa_fwd_args;
 
 /* Length in int32s of fa_fwd's work_order workspace: batch * ceil(lse_seqlen / 32).
  * No counterpart in the reference (its grid is in natural order). */
 size_t fa_fwd_order_len(const fa_fwd_args *args);
-/* Bytes of fa_fwd's split_ws workspace, 0 when the grid fills the chip by itself.
- * It depends on the sizes, head counts, head_dim and causal alone.  No counterpart
- * in the reference. */
+/* Bytes of fa_fwd's split_ws workspace, 0 when the grid fills the chip by itself and
+ * for varlen calls.  It depends on the sizes, head counts, head_dim, causal and the
+ * current device's CU count alone.  No counterpart in the reference. */
 size_t fa_fwd_split_bytes(const fa_fwd_args *args);
 int fa_fwd(const fa_fwd_args *args, void *stream);
 
@@ -131,7 +131,8 @@ typedef struct fa_bwd_args {
     void *split_ws;
     int64_t split_ws_bytes;
     /* Rows of the packed dq and of the packed dk / dv, or 0, as fa_fwd_args.o_rows:
-     * fa_bwd_dq zeroes dq's rows of no sequence, fa_bwd_dkdv those of dk and dv. */
+     * fa_bwd_dq zeroes dq's rows of no sequence (and past lse_seqlen within one),
+     * fa_bwd_dkdv those of dk and dv (past seqlen_k). */
     int32_t dq_rows, dkv_rows;
 } fa_bwd_args;
 
@@ -140,8 +141,8 @@ typedef struct fa_bwd_args {
  * natural order). */
 size_t fa_bwd_order_len(const fa_bwd_args *args);
 /* Bytes of the split_ws workspace, 0 when the dK/dV grid fills the chip by
- * itself.  It depends on the sizes, head counts, head_dim and causal alone.  No
- * counterpart in the reference. */
+ * itself.  It depends on the sizes, head counts, head_dim, causal and the current
+ * device's CU count alone.  No counterpart in the reference. */
 size_t fa_bwd_split_bytes(const fa_bwd_args *args);
 /* D = rowsum(dO * O) (flash_bwd_preprocess_kernel.h:23-96), stored negated in dsum plane 0. */
 int fa_bwd_preprocess(const fa_bwd_args *args, void *stream);
@@ -179,8 +180,9 @@ typedef struct fa_kvcache_args {
     float *out_accum;               /* workspace [num_splits][batch*nheads*seqlen_q][d] fp32, 8-byte aligned */
     float *lse_accum;               /* workspace [num_splits][batch*nheads*seqlen_q] fp32    */
     int32_t *batch_order;           /* workspace [batch + 1]: sequences longest first and a work
-                                       counter (both filled by fa_kv_splitkv or fa_fwd_kvcache),
-                                       or NULL for the natural order                           */
+                                       counter (filled by fa_kv_splitkv or fa_fwd_kvcache where
+                                       the call has more items than the device has CUs, else
+                                       left as they are), or NULL for the natural order        */
     /* Device-side input checks (replace the host reads of flash_api.cpp:627,
      * 634-641 and interface.py:855, so a decode step needs no host sync): a
      * sequence with cache_seqlens[b] < 0, cache_seqlens[b] + seqlen_new >
@@ -221,7 +223,7 @@ typedef struct fa_kvcache_args {
      * the num_splits items of each (batch, kv head, row tile) to finish reads them
      * and writes o and lse, so fa_kv_combine has nothing left to do (it returns at
      * once) and fa_fwd_kvcache runs two kernels (append with ordering, split) instead
-     * of four.  The ordering kernel zeroes these counts on every call. */
+     * of four.  Every call zeroes these counts itself. */
     int32_t *split_count;
 } fa_kvcache_args;
 
@@ -230,8 +232,8 @@ typedef struct fa_kvcache_args {
  * (sizes, options, cache_capacity; num_splits and the workspaces are not read, and
  * batch_order and split_count are taken to be given), fa_kv_num_splits only the sizes
  * of a call without options, and where many rows per KV head ask for more splits than
- * fa_fwd_kvcache_noalloc's scratch holds it returns as many as fit.  fa_kv_args_num_splits has no counterpart in the
- * reference. */
+ * fa_fwd_kvcache_noalloc's scratch holds it returns as many as fit.
+ * fa_kv_args_num_splits has no counterpart in the reference. */
 int fa_kv_args_num_splits(const fa_kvcache_args *args, int requested, int num_cus);
 int fa_kv_num_splits(int requested, int seqlen_k_capacity, int head_dim, int seqlen_q,
                      int batch, int nheads, int nheads_k, int num_cus);
