@@ -834,10 +834,10 @@ static int launch_dq(const fa_bwd_args &a, hipStream_t s) {
 // 32 queries, about 1 us at head_dim 128 and 0.54 at 64 with two workgroups on
 // a CU) is the busiest CU's steps (equal items: whole rounds over the CUs;
 // causal ones are dealt longest first, about half an item of imbalance; a CU
-// with one workgroup is about 10 % slower per step), plus the stores and the
-// count, the partials' traffic and the last workgroup's reads (without the first
-// of these, calls of 8 - 12 steps an item were split at a loss: b1 s44 16/4 22.8 ->
-// 24.5).  Measured on MI355X, causal
+// with one workgroup is about 10 % slower per step), plus the partials' traffic and the last
+// workgroup's reads, and the stores and the count where nothing else runs beside
+// them (without this, calls of 8 - 12 steps an item were split at a loss: b1 s44 16/4
+// 22.8 -> 24.5; with it on fuller grids, b16 64/8 d64 s77 was not: 52.7 -> 57.6).  Measured on MI355X, causal
 // unless noted, us of the dK/dV kernel at S = 1 -> the S taken (best of 1..16):
 //   b1 s8192 32/8 d128: 1285 -> 1027 (S 4, 1027)   b1 s4096 32/8: 484 -> 288 (4, 280)
 //   b1 s2048 32/8: 248 -> 102 (4, 102)             b1 s512 32/8: 70 -> 36 (4, 36)
@@ -868,7 +868,7 @@ static int dkdv_splits(const fa_bwd_args &a) {
         double t = a.causal ? std::max(longest / S, total * (1 + 0.5 * cus / wgs))
                             : double((wgs + cus - 1) / cus) * longest / S;
         if (wgs <= cus) t *= 1.1;
-        if (S > 1) t += 2 + (S - 1) * (0.025 * items + 3);
+        if (S > 1) t += (2 * wgs <= cus ? 2 : 0) + (S - 1) * (0.025 * items + 3);
         if (S == 1 || t < best_t) {
             best = S;
             best_t = t;

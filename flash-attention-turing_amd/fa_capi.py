@@ -113,6 +113,8 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
         fn.restype = ctypes.c_int
     lib.fa_kv_num_splits.argtypes = [ctypes.c_int] * 8
     lib.fa_kv_num_splits.restype = ctypes.c_int
+    lib.fa_kv_args_num_splits.argtypes = [ctypes.POINTER(FaKvcacheArgs), ctypes.c_int, ctypes.c_int]
+    lib.fa_kv_args_num_splits.restype = ctypes.c_int
     lib.fa_kv_workspace_bytes.argtypes = [ctypes.POINTER(FaKvcacheArgs)]
     lib.fa_kv_workspace_bytes.restype = ctypes.c_size_t
     lib.fa_kv_split_count_len.argtypes = [ctypes.POINTER(FaKvcacheArgs)]
