@@ -23,8 +23,8 @@ def _fa(b, sq, sk, h, hk, hd, causal):
     return fa_capi.load().fa_fwd_split_bytes(ctypes.byref(a))
 
 
-# batch, sq, sk, h, hk, hd, causal, whether workgroups share (2 to 16 of them).  Without: two groups of 2 row waves
-# (64-row blocks; from fewer rows and keys than one block to the most of that plan), then of 4.
+# batch, sq, sk, h, hk, hd, causal, whether workgroups share (2 to 16 of them).  Without: one group on one key block,
+# two groups of 2 row waves (64-row blocks, from two key blocks to the most of that plan), then of 4.
 CASES = [
     (1, 130, 2500, 8, 2, 128, True, True),
     (1, 40, 5000, 6, 2, 64, False, True),
@@ -34,6 +34,8 @@ CASES = [
     (1, 17, 9000, 2, 2, 128, True, True),
     (1, 20, 30, 2, 1, 128, False, False),
     (1, 65, 64, 6, 2, 64, True, False),
+    (1, 20, 65, 2, 1, 128, False, False),
+    (2, 70, 100, 6, 2, 64, True, False),
     (1, 509, 509, 32, 8, 128, True, False),
     (2, 512, 777, 6, 2, 64, False, False),
     (3, 257, 520, 4, 4, 128, True, False),

@@ -14,7 +14,8 @@ from test_kvcache_gpu import _paged_from_contiguous
 
 # batch, queries, heads, kv heads, head_dim, capacity, appended, lengths before the append, splits, causal, options.
 # 64 rows (the least), 65, 127 - 129, a group of 3; keys at block and page edges, an empty cache, fewer keys than
-# splits; windows smaller than a tile's positions, keys before a leftpad, every option at once.
+# splits; windows smaller than a tile's positions, keys before a leftpad, every option at once.  (Softcap and ALiBi on
+# so few tiles are the split kernel's; test_chunk_ranked has them on this one.)
 CASES = [
     (2, 16, 8, 2, 128, 512, 16, (0, 496), 1, True, {}),
     (2, 13, 10, 2, 64, 768, 5, (64, 700), 3, True, {}),
@@ -121,7 +122,8 @@ def test_chunk_over_1024_pages(device, splits):
 # Batches of chunks in more items than CUs (12 sequences x 8 KV heads x 2 tiles x 3 splits): sequences in the order of
 # their lengths, an empty one among them, later items starting while earlier ones merge.
 @pytest.mark.gpu
-@pytest.mark.parametrize("hd,opt", [(128, ""), (64, "softcap alibi"), (128, "alibi window"), (64, "leftpad")])
+@pytest.mark.parametrize("hd,opt", [(128, ""), (64, "softcap alibi"), (128, "alibi window"), (64, "leftpad"),
+                                    (128, "rotary softcap window leftpad")])
 def test_chunk_ranked(device, hd, opt):
     b, sq, h, hk, cap, new, splits = 12, 33, 32, 8, 640, 33, 3
     assert b * hk * 2 * splits > torch.cuda.get_device_properties(0).multi_processor_count, "items must be ranked"
@@ -134,9 +136,18 @@ def test_chunk_ranked(device, hd, opt):
               alibi_slopes=2.0 ** -torch.arange(1, h + 1, dtype=torch.float32) / 4 if "alibi" in opt else None,
               cache_leftpad=torch.arange(b, dtype=torch.int32) * 3 if "leftpad" in opt else None)
     print(f"case ranked hd={hd} {opt}", flush=True)
-    _, _, kc_ref, vc_ref = kv_oracle(q, kc, vc, k, v, seqlens, None, None, True, 1, None)
+    q_ref, k_ref = q, k
+    if "rotary" in opt:
+        # Quarter turns: exact, so that no element hangs on a rounding by way of fp32 or not.
+        turn = torch.randint(0, 4, (cap, 32), generator=g)
+        kw.update(rotary_cos=torch.tensor([1.0, 0.0, -1.0, 0.0])[turn].half(),
+                  rotary_sin=torch.tensor([0.0, 1.0, 0.0, -1.0])[turn].half(), rotary_interleaved=True)
+        at = seqlens.long()[:, None] + torch.arange(sq)[None, :]
+        q_ref = okv.rotary_embed(q, kw["rotary_cos"], kw["rotary_sin"], at, True)
+        k_ref = okv.rotary_embed(k, kw["rotary_cos"], kw["rotary_sin"], at, True)
+    _, _, kc_ref, vc_ref = kv_oracle(q, kc, vc, k_ref, v, seqlens, None, None, True, 1, None)
     ku, vu = okv.materialize(kc_ref, vc_ref, ends, None, None)
-    o_ref, l_ref = okv.splitkv_attention(q, ku, vu, ends, hd ** -0.5, True, 1, window=kw["window_size"],
+    o_ref, l_ref = okv.splitkv_attention(q_ref, ku, vu, ends, hd ** -0.5, True, 1, window=kw["window_size"],
                                          softcap=kw["softcap"], alibi_slopes=kw["alibi_slopes"],
                                          leftpad=kw["cache_leftpad"])
     got = _call(device, q, kc, vc, k, v, seqlens, None, None, splits, True, kw)
