@@ -764,7 +764,11 @@ __global__ __launch_bounds__(256, 2) void kv_splitkv_kernel(const fa_kvcache_arg
 // share of the keys that some row of its tile sees (with a window those are
 // few of the sequence's).  With num_splits > 1 the last split of a row tile to
 // finish adds the others' partials to its own.
-constexpr int kChunkRows = 128, kChunkKeys = 64, kChunkPages = 1024;
+constexpr int kChunkRows = 128, kChunkKeys = 64;
+// Page ids in LDS: as many as fit beside the stages of two workgroups per CU (about
+// a million tokens in pages of 256).  Staging them anew on the way, for any number,
+// cost the block loop 0.6 - 1.2 % (two sequences of 512 tokens: 215 -> 217.6 us).
+constexpr int kChunkPages = 3840;
 constexpr int kChunkMinRows = 64, kChunkMaxSplits = 32;
 
 // Merges the partial rows (O normalised, LSE) of a row tile's splits.  Every
@@ -880,7 +884,7 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcach
         if (wr >= 0) hi = min(hi, p + wr + 1);
         return hi;
     };
-    const int t_lo = key_lo(first / G + off), t_n = max(0, key_hi((first + rows_here - 1) / G + off) - t_lo);
+    const int t_lo = __builtin_amdgcn_readfirstlane(key_lo(first / G + off)), t_n = max(0, key_hi((first + rows_here - 1) / G + off) - t_lo);
     const int s0 = t_lo + int(int64_t(t_n) * split / S), s1 = t_lo + int(int64_t(t_n) * (split + 1) / S);
     const int nb0 = s0 / BN, nb1 = s1 > s0 ? (s1 - 1) / BN + 1 : nb0;
     // Of the split's keys: those the lane's row sees, [lo, hi), those some row
@@ -909,18 +913,14 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcach
             qB[g] = as_h8(v);
         }
     }
-    // Page ids of the walked keys, kChunkPages of them at a time: those from block
-    // nb's page on, which serve the blocks below nb_staged.
+    // Page ids of the walked keys (this kernel is taken only when they fit).
     const int page = a.page_block_size;
-    int pg0 = 0, nb_staged = nb1;
-    auto stage_pages = [&](int nb) {
-        pg0 = nb * BN / page;
+    const int pg0 = a.block_table ? nb0 * BN / page : 0;
+    if (a.block_table && nb1 > nb0) {
         const int32_t *bt = a.block_table + int64_t(b) * a.block_table_stride + pg0;
-        const int n_pages = min(kChunkPages, (nb1 * BN - 1) / page - pg0 + 1);
+        const int n_pages = (nb1 * BN - 1) / page - pg0 + 1;
         for (int i = tid; i < n_pages; i += kKvThreads) pages[i] = bt[i];
-        nb_staged = int(min(int64_t(nb1), int64_t(pg0 + kChunkPages) * (page / BN)));
-    };
-    if (a.block_table && nb1 > nb0) stage_pages(nb0);
+    }
     wait_vmem();  // only the tile copies are in flight in the loop
     __syncthreads();
 
@@ -937,7 +937,7 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcach
         const f16 *kb = kc + blk * a.k_cache.batch_stride + int64_t(at) * krs;
         const f16 *vb = vc + blk * a.v_cache.batch_stride + int64_t(at) * vrs;
         const int soff = (nb & 1) * STAGE;
-        if (nb * BN >= t_lo && nb * BN + BN <= L) {
+        if ((!EXT || nb * BN >= t_lo) && nb * BN + BN <= L) {
             kcp.template copy_to<true>(lds_addr(smem) + soff, kb, krs);
             vcp.template copy_to<true>(lds_addr(smem) + soff + TILE, vb, vrs);
         } else {  // keys past L re-read key L - 1, keys that no row sees at the start re-read the first seen one (masked)
@@ -954,13 +954,7 @@ __global__ __launch_bounds__(kKvThreads, 2) void kv_chunk_kernel(const fa_kvcach
     for (int nb = nb0; nb < nb1; ++nb) {
         wait_vmem();
         __syncthreads();  // block nb is in LDS; every wave is done with the other stage
-        if (nb + 1 < nb1) {
-            if (nb + 1 >= nb_staged) {
-                stage_pages(nb + 1);  // (every wave has read the ids of the blocks up to nb)
-                __syncthreads();
-            }
-            issue(nb + 1);
-        }
+        if (nb + 1 < nb1) issue(nb + 1);
         const int p0 = nb * BN;
         if (p0 >= any_hi || p0 + BN <= any_lo) continue;  // no key for this wave
         // The lane's read bases with this block's stage added (opaque, so the
@@ -1178,10 +1172,13 @@ static size_t noalloc_bytes(const fa_kvcache_args &a) {
 // kernel needs: at least 64 query rows per KV head (with 64 rows, 8 sequences of 8k
 // keys, 32 / 8 heads: 71 us against 114 at the best split counts; with 32 rows the
 // other kernel reads K and V once as well and its waves share the keys) in enough
-// tiles (chunk_pays).  Its 64-key blocks must not straddle pages.
+// tiles (chunk_pays).  Its 64-key blocks must not straddle pages, and its page ids fit
+// in LDS.
 static bool chunk_suits(const fa_kvcache_args &a, int num_cus) {
     if ((a.nheads / a.nheads_k) * a.seqlen_q < kChunkMinRows) return false;
-    if (a.block_table && a.page_block_size % kChunkKeys != 0) return false;
+    if (a.block_table && (a.page_block_size % kChunkKeys != 0 || a.cache_capacity <= 0 ||
+                          a.cache_capacity / a.page_block_size > kChunkPages))
+        return false;
     return chunk_pays(chunk_tiles(a), split_keys(a), a.softcap > 0.f || a.alibi_slopes, num_cus);
 }
 

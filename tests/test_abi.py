@@ -296,6 +296,10 @@ def test_num_splits_of_a_call(lib):
     split = call(*many, softcap=30.0)
     assert split == call(*many, alibi_slopes=1 << 20) == call(*many, block_table=1 << 20, page_block_size=32) == 8
     assert call(*many) == call(*many, block_table=1 << 20, page_block_size=64) > split
+    # Pages past those whose ids fit in LDS leave the call to the split kernel, which takes its own count.
+    wide, table = (64 * 4000, 128, 64, 2, 32, 8), dict(block_table=1 << 20)
+    assert call(*wide, **table, page_block_size=64) == call(*wide, softcap=30.0, block_table=1 << 20, page_block_size=32)
+    assert call(*wide, **table, page_block_size=256) == call(*wide)
     assert call(*many, local_window=1, window_left=1000) == call(1017, *many[1:])
 
 

@@ -95,8 +95,8 @@ def test_kvcache_chunk(device, case):
 @pytest.mark.gpu
 @pytest.mark.parametrize("splits", [1, 2])
 def test_chunk_over_1024_pages(device, splits):
-    """1100 shuffled pages of 64 tokens: with one split its page ids do not fit in LDS at once and are staged anew on
-    the way; the contiguous cache of the same tokens gives the same bits (18 KV heads of one tile: this kernel)."""
+    """1100 shuffled pages of 64 tokens: one split of this kernel holds their ids in LDS; the contiguous cache of the
+    same tokens gives the same bits (18 KV heads of one tile: this kernel)."""
     g = torch.Generator().manual_seed(8400)
     pages, page, sq, h, hd = 1100, 64, 64, 18, 64
     cap, lens = pages * page, torch.tensor([pages * page - 21], dtype=torch.int32)
