@@ -387,9 +387,10 @@ __global__ __launch_bounds__(kOrderThreads) void dq_order_kernel(const fa_bwd_ar
 }
 
 // Sums the S partial dK / dV tiles of an item.  Each of its workgroups stores
-// its own and then counts itself; the one that counts last finds all of them
-// stored and adds them in the order of their shares, so the sum does not depend
-// on who came last and no workgroup waits for another.  Returns whether this
+// its own and then counts itself; the one that counts last, or that finds all
+// others counted before it has stored anything, adds them in the order of their
+// shares, so the sum does not depend on who came last and no workgroup waits for
+// another.  Returns whether this
 // workgroup holds the sum.  Partials are stored and loaded at agent scope (past
 // the XCD's L2, as in the split KV kernel), 8 bytes a lane, 512 contiguous bytes
 // a wave.
@@ -401,19 +402,24 @@ __device__ __forceinline__ bool dkdv_reduce(const fa_bwd_args &a, int item, int 
     int32_t *count = reinterpret_cast<int32_t *>(a.split_ws) + item;
     uint64_t *slots = reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(a.split_ws) + dkdv_count_bytes(dkdv_items(a))) +
                       int64_t(item) * S * N * kDkvThreads + tid;
-    uint64_t *own = slots + int64_t(part) * N * kDkvThreads;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        f32x16 &t = i < N / 2 ? dk[i / 8] : dv[i / 8 - N / 16];
-        const f32x2 x = {t[2 * (i & 7)], t[2 * (i & 7) + 1]};
-        __hip_atomic_store(own + i * kDkvThreads, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-    }
-    wait_vmem();
-    __syncthreads();  // every wave's stores have completed
-    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0)
+        *ticket = part < 2 ? __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
     __syncthreads();
-    if (*ticket != S - 1) return false;
+    if (*ticket != S - 1) {
+        uint64_t *own = slots + int64_t(part) * N * kDkvThreads;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            f32x16 &t = i < N / 2 ? dk[i / 8] : dv[i / 8 - N / 16];
+            const f32x2 x = {t[2 * (i & 7)], t[2 * (i & 7) + 1]};
+            __hip_atomic_store(own + i * kDkvThreads, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+        wait_vmem();
+        __syncthreads();  // every wave's stores have completed
+        if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*ticket != S - 1) return false;
+    }
     // It adds to its own registers when its share is one of the first two (x0 +
     // x1 = x1 + x0), and all shares from memory otherwise.
     if (part >= 2) {

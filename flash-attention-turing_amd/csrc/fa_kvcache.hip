@@ -773,8 +773,8 @@ constexpr int kChunkMinRows = 64, kChunkMaxSplits = 32;
 
 // Merges the partial rows (O normalised, LSE) of a row tile's splits.  Every
 // item stores its own, lane by lane, and then counts itself; the one that
-// counts last finds all of them stored and sums them in split order, its own
-// from registers, so no item waits for another.  row0: the tile's first row of
+// counts last, or that finds all others counted before it has stored anything,
+// sums them in split order, its own from registers, so no item waits for another.  row0: the tile's first row of
 // a split's accumulators, rows_here x HD values from there.  Returns whether
 // this item holds the sum.
 template <int HD>
@@ -789,22 +789,26 @@ __device__ __forceinline__ bool chunk_merge(const fa_kvcache_args &a, int32_t *c
     uint64_t *pairs = reinterpret_cast<uint64_t *>(a.out_accum + row0 * HD) + hh * rows_here + row;
     const int step = 2 * rows_here;
     float *lses = a.lse_accum + row0 + row;
-    if (live) {
-        uint64_t *slot = pairs + int64_t(split) * nrow * (HD / 2);
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const f32x2 x = {o[i / 8][2 * (i & 7)], o[i / 8][2 * (i & 7) + 1]};
-            __hip_atomic_store(slot + i * step, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (hh == 0)
-            __hip_atomic_store(lses + int64_t(split) * nrow, lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    wait_vmem();
-    __syncthreads();  // every wave's stores have completed
-    if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) *ticket = __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    if (*ticket != S - 1) return false;
+    if (*ticket != S - 1) {
+        if (live) {
+            uint64_t *slot = pairs + int64_t(split) * nrow * (HD / 2);
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const f32x2 x = {o[i / 8][2 * (i & 7)], o[i / 8][2 * (i & 7) + 1]};
+                __hip_atomic_store(slot + i * step, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (hh == 0)
+                __hip_atomic_store(lses + int64_t(split) * nrow, lse, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        wait_vmem();
+        __syncthreads();  // every wave's stores have completed
+        if (tid == 0) *ticket = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*ticket != S - 1) return false;
+    }
     if (!live) return true;
     auto lse_of = [&](int s) {
         return s == split ? lse
