@@ -1118,10 +1118,11 @@ static int check_kv(const fa_kvcache_args *p) {
 //   32/8, 16 x 18k (8): 52 -> 60                       64/4, 9 x 20k (8): 67 -> 71
 //   32/8, 32 x 106k (8): 274 -> 165                    64/2, 9 x 186k (6): 318 -> 211
 //   12 - 16 tiles: 1.0 - 1.9x faster; 17 and more: 1.2 - 1.9x; up to 4k keys: 1.0 - 1.4x
-//   natural: b4 16/1, 8 x 15k (4): 54 -> 86; 16 tiles: 0.77 - 1.3x; 1 - 8 tiles x 3k: 0.84x
+//   natural: b4 16/1, 8 x 15k (4): 54 -> 86; 16 tiles: 0.77 - 1.3x; 1 - 8 tiles on 2k - 4k
+//   keys: 0.84 - 0.9x; on up to 1k: 1.07 - 1.26x
 static bool chunk_pays(int64_t tiles, int64_t keys, bool natural, int num_cus) {
     const int64_t cus = std::max(num_cus, 1);
-    if (natural) return 16 * tiles > cus;
+    if (natural) return 16 * tiles > cus || (keys > 0 && keys <= 1024);
     return 24 * tiles > cus || (keys > 0 && keys <= 4096) || (48 * tiles > cus && keys >= 65536);
 }
 
